@@ -6,7 +6,11 @@
 // is spread over the 8 lanes 8g..8g+7, 4 rows each: each lane places its 4 match bits at
 // bit 31-4*(l%8)-j, an OR over the 8 lanes (DPP, no LDS) assembles the MSB-first word,
 // and one lane per group stores it.
+#include <string.h>
+
 #include <algorithm>
+#include <type_traits>
+#include <vector>
 
 #include "common.h"
 
@@ -217,6 +221,10 @@ constexpr int kMultiLaneRows = 32;                      // rows per lane: one bi
 constexpr int kMultiTileRows = kWave * kMultiLaneRows;  // 2048 rows per wave tile
 constexpr unsigned kMultiMaxGrid = 4096;
 
+constexpr uint32_t kHistEntries = 1024;  // row counts of a workgroup: all copies
+constexpr unsigned kScanXcds = 8;
+constexpr int kRankEntries = 2 * kMultiPreds + 2;       // ranges between the bounds, and one for no row
+
 struct MultiPreds {
   uint32_t lo[kMultiPreds];
   uint32_t span[kMultiPreds];  // hi - lo
@@ -296,6 +304,237 @@ __global__ __launch_bounds__(kBlock) void k_scan_multi(const uint32_t *col, uint
     __syncthreads();
     if ((int)threadIdx.x >= pbeg && (int)threadIdx.x < pend)
       partials[(uint64_t)threadIdx.x * gridDim.x + blockIdx.x] = cnt[threadIdx.x];
+  }
+}
+
+// The same pass for many predicates (direct_preds).  The predicates' 2 * np bounds cut
+// the values into at most 2 * np + 1 ranges, and all rows of a range match the same
+// predicates: a row's range is found by a binary search in LDS and the range's predicate mask
+// (bit p: predicate p matches) read from a table, ~45 VALU instructions a row for 64
+// predicates where testing each predicate takes three a row and predicate.  A wave takes
+// 2048 rows.  Search: the wave's coalesced loads (16 bytes a lane) give lane l rows 4l..4l+3
+// of each 256; the bounds lie in breadth-first order, so that one level's nodes (at most 64)
+// are in different LDS banks.  The ranges' numbers are a byte each and go through LDS to the
+// lane that owns the row's bitmap word.  Words: lane l looks up the masks of the 32 rows of
+// word l and transposes the 32 x 32 bits in registers (two byte permutes a word, then three
+// shift-and-select steps), which leaves the word of every predicate of a half (32
+// predicates) in a register; the wave stores 64 consecutive words of each bitmap.  COUNT:
+// rows per range by LDS adds, which make each predicate's rows at the end (popcounts of the
+// words cost 180 us more at 64 predicates).  1e8 rows, 64 predicates, counted: 732 us by
+// testing each predicate, 322 this way, 176 of it when nothing is stored.
+struct RankedPreds {
+  uint32_t tree[128];             // [1, 2^levels): bounds but the smallest, breadth-first, padded with 2^32 - 1
+  uint32_t mask[2][kRankEntries];  // predicates matching range r, 32 per half; the last entry is 0
+  uint8_t r0[kMultiPreds], r1[kMultiPreds];  // predicate p matches the ranges [r0, r1)
+  uint32_t first;                 // the smallest bound
+  int levels;
+  uint32_t last;    // the last range
+  uint32_t copies;  // copies of the ranges' row counts (a power of two up to 64), stride entries apart
+  uint32_t stride;
+};
+
+// out[p] bit 31 - r = in[r] bit p, in place (word 31 - p holds predicate p afterwards).
+__device__ __forceinline__ void transpose32(uint32_t (&a)[32]) {
+#pragma unroll
+  for (int k = 0; k < 16; k++) {
+    const uint32_t x = a[k], y = a[k + 16];
+    a[k] = __builtin_amdgcn_perm(x, y, 0x07060302);       // the upper halves
+    a[k + 16] = __builtin_amdgcn_perm(x, y, 0x05040100);  // the lower halves
+  }
+#pragma unroll
+  for (int b = 0; b < 32; b += 16)
+#pragma unroll
+    for (int k = b; k < b + 8; k++) {
+      const uint32_t x = a[k], y = a[k + 8];
+      a[k] = __builtin_amdgcn_perm(x, y, 0x07030501);      // bytes 3 and 1 of each
+      a[k + 8] = __builtin_amdgcn_perm(x, y, 0x06020400);  // bytes 2 and 0 of each
+    }
+#pragma unroll
+  for (int j = 4, s = 0; s < 3; j >>= 1, s++) {
+    const uint32_t m = j == 4 ? 0x0F0F0F0Fu : j == 2 ? 0x33333333u : 0x55555555u;
+#pragma unroll
+    for (int k = 0; k < 32; k++) {
+      if (k & j) continue;
+      const uint32_t x = a[k], y = a[k + j];
+      a[k] = (x & ~m) | ((y >> j) & m);
+      a[k + j] = ((x << j) & ~m) | (y & m);
+    }
+  }
+}
+
+// The bitmap words of the wave's 64 word positions from w0 on: rank4 holds the lane's 32
+// ranges, four a word.  FULL: np = 32 * HALVES and every position is inside the bitmap.
+template <int HALVES, bool FULL>
+__device__ __forceinline__ void store_ranked(uint32_t (&rank4)[8], const uint32_t (&mask)[HALVES][kRankEntries],
+                                             int half0, int np, BITS *out, uint64_t stride, uint64_t w0, bool in,
+                                             int lane) {
+#pragma unroll 1
+  for (int h = 0; h < HALVES; h++) {
+    uint32_t a[32];
+    // the halves look their masks up separately: without this the 32 addresses stay in registers
+#pragma unroll
+    for (int r = 0; r < 8; r++) asm volatile("" : "+v"(rank4[r]));
+#pragma unroll
+    for (int r = 0; r < 32; r++) a[r] = mask[h][(rank4[r / 4] >> (8 * (r & 3))) & 0xFF];
+    transpose32(a);
+    const int p0 = 32 * (half0 + h);
+    BITS *o = out + (uint64_t)p0 * stride + w0;
+    int left = np - p0;
+#pragma unroll
+    for (int p = 0; p < 32; p++) {
+      if (FULL || (p < left && in)) o[lane] = a[31 - p];
+      o += stride;
+      // one running address and count, not 32 of each kept in scalar registers
+      asm volatile("" : "+s"(o), "+s"(left));
+    }
+  }
+}
+
+template <int HALVES, bool COUNT, bool FULL>
+__global__ __launch_bounds__(kBlock) void k_scan_ranked(const uint32_t *col, uint64_t n, uint64_t whole,
+                                                        RankedPreds rp, int np, BITS *out, uint64_t stride,
+                                                        uint32_t run, uint32_t *partials) {
+  __shared__ uint32_t tree[128];
+  __shared__ uint32_t mask[HALVES][kRankEntries];
+  __shared__ alignas(16) uint32_t xch[kBlock / kWave][kMultiTileRows / 4];
+  // rows per range (COUNT), in as many copies as fit (four for 64 predicates, one a lane for
+  // four): a wave's rows of one range would otherwise add to one address one after another
+  // (3 predicates over 2^25 rows, counted: 48 us with four copies)
+  __shared__ uint32_t hist[COUNT ? kHistEntries : 1];
+  __shared__ uint32_t below[COUNT ? kRankEntries : 1];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int half0 = HALVES == 1 ? blockIdx.y : 0;  // one half a workgroup: which one
+  if (threadIdx.x < 128) tree[threadIdx.x] = rp.tree[threadIdx.x];
+  for (int i = threadIdx.x; i < HALVES * kRankEntries; i += kBlock)
+    mask[i / kRankEntries][i % kRankEntries] = rp.mask[half0 + i / kRankEntries][i % kRankEntries];
+  if (COUNT)
+    for (uint32_t i = threadIdx.x; i < kHistEntries; i += kBlock) hist[i] = 0;
+  __syncthreads();
+  const uint64_t words = words_for_rows(n), ntiles = (n + kMultiTileRows - 1) / kMultiTileRows;
+  const uint32_t first = rp.first, root = rp.tree[1];
+  const int levels = rp.levels;
+  const uint32_t leaf0 = 1u << levels;
+  const uint32_t top = rp.last;
+  uint32_t *const hw = hist + (COUNT ? (lane & (rp.copies - 1)) * rp.stride : 0);
+  uint32_t *const xw = xch[wv];
+  // the ranks of the wave's tile, written to xw in row order, back as lane l's 32 rows of word l
+  auto exchange = [&](uint32_t(&rank4)[8]) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wave's own exchange: LDS keeps its order
+    __builtin_amdgcn_wave_barrier();
+    const uint4 ra = *reinterpret_cast<const uint4 *>(xw + 8 * lane), rb = *reinterpret_cast<const uint4 *>(xw + 8 * lane + 4);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    rank4[0] = ra.x, rank4[1] = ra.y, rank4[2] = ra.z, rank4[3] = ra.w;
+    rank4[4] = rb.x, rank4[5] = rb.y, rank4[6] = rb.z, rank4[7] = rb.w;
+  };
+  // workgroup step i of XCD x -> tile of wave 0: runs of `run` steps to an XCD, so that lines
+  // that neighbouring tiles share (bitmaps that do not start on a 128-byte line) mostly meet
+  // in one L2
+  const uint64_t xcd = blockIdx.x % kScanXcds, step0 = blockIdx.x / kScanXcds, steps = gridDim.x / kScanXcds;
+  auto tile_of = [&](uint64_t i) {
+    return (i / run * run * kScanXcds + xcd * run + i % run) * (kBlock / kWave) + wv;
+  };
+  uint4 v[8];
+  auto load = [&](uint64_t t) {
+    const uint4 *src = reinterpret_cast<const uint4 *>(col + t * (uint64_t)kMultiTileRows) + lane;
+#pragma unroll
+    for (int k = 0; k < 8; k++) v[k] = load_stream(src + 64 * k);
+  };
+  uint64_t step = step0, t = tile_of(step0);
+  // whole: every row of the tile exists, and the next tile's loads go out before this one's
+  // stores
+  auto tile = [&](auto whole_tile) __attribute__((always_inline)) {
+    constexpr bool kWhole = decltype(whole_tile)::value;
+    uint32_t i[32];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      i[4 * k] = v[k].x >= root ? 3 : 2;
+      i[4 * k + 1] = v[k].y >= root ? 3 : 2;
+      i[4 * k + 2] = v[k].z >= root ? 3 : 2;
+      i[4 * k + 3] = v[k].w >= root ? 3 : 2;
+    }
+    for (int l = 1; l < levels; l++) {
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const uint32_t t0 = tree[i[4 * k]], t1 = tree[i[4 * k + 1]], t2 = tree[i[4 * k + 2]], t3 = tree[i[4 * k + 3]];
+        i[4 * k] = 2 * i[4 * k] + (v[k].x >= t0);
+        i[4 * k + 1] = 2 * i[4 * k + 1] + (v[k].y >= t1);
+        i[4 * k + 2] = 2 * i[4 * k + 2] + (v[k].z >= t2);
+        i[4 * k + 3] = 2 * i[4 * k + 3] + (v[k].w >= t3);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      uint32_t r[4] = {i[4 * k] - leaf0 + (v[k].x >= first), i[4 * k + 1] - leaf0 + (v[k].y >= first),
+                       i[4 * k + 2] - leaf0 + (v[k].z >= first), i[4 * k + 3] - leaf0 + (v[k].w >= first)};
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const bool row = kWhole || t * (uint64_t)kMultiTileRows + 256 * k + 4 * lane + j < n;
+        // 2^32 - 1 is not below the padding bounds: its range is the last
+        if (COUNT && row) atomicAdd(&hw[min(r[j], top)], 1u);
+        if (!row) r[j] = kRankEntries - 1;  // the range that no predicate matches
+      }
+      xw[64 * k + lane] = r[0] | r[1] << 8 | r[2] << 16 | r[3] << 24;
+    }
+    const uint64_t w0 = t * (kMultiTileRows / 32);
+    // loads and stores complete in one order: issued before the stores, the next tile's
+    // loads do not wait for them
+    step += steps;
+    t = tile_of(step);
+    if (kWhole && t < whole) load(t);
+    uint32_t rank4[8];
+    exchange(rank4);
+    store_ranked<HALVES, kWhole && FULL>(rank4, mask, half0, np, out, stride, w0, kWhole || w0 + lane < words, lane);
+  };
+  // the first tile apart, so that every tile of the loop finds its loads issued before the
+  // stores of the one before
+  if (t < whole) {
+    load(t);
+    tile(std::true_type{});
+    while (t < whole) tile(std::true_type{});
+  }
+  // a column that is not 16-byte aligned, and the rows past the whole tiles: the same rows,
+  // loaded one by one where they exist
+  while (t < ntiles) {
+    const uint64_t row = t * (uint64_t)kMultiTileRows + 4 * lane;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const uint64_t r = row + 256 * k;
+      v[k] = make_uint4(r < n ? col[r] : 0, r + 1 < n ? col[r + 1] : 0, r + 2 < n ? col[r + 2] : 0, r + 3 < n ? col[r + 3] : 0);
+    }
+    tile(std::false_type{});
+  }
+  if (COUNT) {
+    __syncthreads();
+    // rows of each range over the copies, then rows below each range, then each predicate's
+    for (uint32_t r = threadIdx.x; r < kRankEntries; r += kBlock) {
+      uint32_t a = 0;
+      if (r <= top)
+        for (uint32_t c = 0; c < rp.copies; c++) a += hist[c * rp.stride + r];
+      below[r] = a;
+    }
+    __syncthreads();
+    if (threadIdx.x < kWave) {
+      const int r = 2 * lane;  // 2 * kWave + 2 entries: the last two follow the scan
+      const uint32_t a = below[r], b = below[r + 1], last = below[2 * kWave];
+      uint32_t sum = a + b;
+#pragma unroll
+      for (int o = 1; o < kWave; o <<= 1) {
+        const uint32_t u = __shfl_up(sum, o, kWave);
+        if (lane >= o) sum += u;
+      }
+      below[r] = sum - a - b;
+      below[r + 1] = sum - b;
+      if (lane == kWave - 1) {
+        below[2 * kWave] = sum;
+        below[2 * kWave + 1] = sum + last;
+      }
+    }
+    __syncthreads();
+    const int p = 32 * half0 + (int)threadIdx.x;
+    if (threadIdx.x < 32 * HALVES && p < np)
+      partials[(uint64_t)p * gridDim.x + blockIdx.x] = below[rp.r1[p]] - below[rp.r0[p]];
   }
 }
 
@@ -449,6 +688,72 @@ hipError_t scan_conjunction(const CODE *const *cols, const CODE *lo, const CODE 
   return hipSuccess;
 }
 
+// Range table of up to kMultiPreds predicates: the distinct bounds lo and hi + 1 in order
+// (range r = the values with r bounds at or below them), as k_scan_ranked searches them.
+static RankedPreds rank_table(const CODE *lo, const CODE *hi, int np) {
+  RankedPreds t;
+  std::vector<uint32_t> b;
+  for (int p = 0; p < np; p++) {
+    if (lo[p] > hi[p]) continue;
+    b.push_back(lo[p]);
+    if (hi[p] != 0xFFFFFFFFu) b.push_back(hi[p] + 1);
+  }
+  std::sort(b.begin(), b.end());
+  b.erase(std::unique(b.begin(), b.end()), b.end());
+  memset(t.mask, 0, sizeof(t.mask));
+  memset(t.r0, 0, sizeof(t.r0));
+  memset(t.r1, 0, sizeof(t.r1));
+  for (int p = 0; p < np; p++) {
+    if (lo[p] > hi[p]) continue;
+    const size_t r0 = std::lower_bound(b.begin(), b.end(), lo[p]) - b.begin() + 1;
+    // a value of 2^32 - 1 also passes the padding bounds: the last range's mask fills up
+    const size_t r1 = hi[p] == 0xFFFFFFFFu ? kRankEntries - 1 : std::lower_bound(b.begin(), b.end(), hi[p] + 1) - b.begin() + 1;
+    t.r0[p] = (uint8_t)r0;
+    t.r1[p] = (uint8_t)r1;
+    for (size_t r = r0; r < r1; r++) t.mask[p / 32][r] |= 1u << (p % 32);
+  }
+  t.last = (uint32_t)b.size();
+  t.stride = (t.last + 1) | 1;  // odd: the copies start in different LDS banks
+  t.copies = 64;
+  while (t.copies * t.stride > kHistEntries) t.copies /= 2;
+  t.first = b.empty() ? 0xFFFFFFFFu : b[0];
+  t.levels = 1;
+  while ((1u << t.levels) < b.size()) t.levels++;  // 2^levels - 1 nodes for the bounds but the first
+  for (uint32_t &v : t.tree) v = 0xFFFFFFFFu;
+  for (int l = 0; l < t.levels; l++)  // node i of level l: the bound in the middle of its span
+    for (uint32_t i = 0; i < 1u << l; i++) {
+      const size_t at = ((2 * (size_t)i + 1) << (t.levels - 1 - l));  // 1 .. 2^levels - 1
+      if (at < b.size()) t.tree[(1u << l) + i] = b[at];
+    }
+  return t;
+}
+
+template <int HALVES>
+static void launch_ranked(const uint32_t *col, uint64_t n, const RankedPreds &t, int np, BITS *out, uint64_t stride,
+                          uint32_t run, uint32_t *partials, dim3 grid, hipStream_t s) {
+  const uint64_t whole = aligned16(col) ? n / kMultiTileRows : 0;
+  const bool full = np == 32 * HALVES * (int)grid.y;
+  if (partials)
+    full ? k_scan_ranked<HALVES, true, true><<<grid, kBlock, 0, s>>>(col, n, whole, t, np, out, stride, run, partials)
+         : k_scan_ranked<HALVES, true, false><<<grid, kBlock, 0, s>>>(col, n, whole, t, np, out, stride, run, partials);
+  else
+    full ? k_scan_ranked<HALVES, false, true><<<grid, kBlock, 0, s>>>(col, n, whole, t, np, out, stride, run, partials)
+         : k_scan_ranked<HALVES, false, false><<<grid, kBlock, 0, s>>>(col, n, whole, t, np, out, stride, run, partials);
+}
+
+// Predicates up to which a pass tests each one (k_scan_multi) instead of searching
+// (k_scan_ranked).  The search costs a row the same for any number of predicates up to 32 and
+// half as much again up to 64, a test three instructions a row and predicate; on a short
+// column the search's chain of dependent steps (one tile a wave) is what shows.  Measured,
+// counted, tests against search: 1e5 rows, 64 predicates 10.7 / 11.3 us; 2^19 rows, 33: 9.3 /
+// 10.3, 64: 11.1 / 10.2; 2^20 rows, 16: 8.7 / 9.3, 24: 10.8 / 10.0, 64: 15.5 / 11.0; 4.2e6
+// rows, 8: 11.3 / 11.6, 10: 12.2 / 12.4, 16: 15.9 / 12.7; 1e8 rows, 5: 100 / 103, 8: 116 /
+// 105, 16: 199 / 119, 32: 379 / 196, 64: 732 / 322 (260 when every bitmap starts on a
+// 128-byte line: what is left is the writes' rate).
+static int direct_preds(uint64_t n) {
+  return n < (1u << 18) ? kMultiPreds : n < (1u << 20) ? 40 : n < (1u << 22) ? 16 : 8;
+}
+
 hipError_t scan_ranges(const CODE *col, uint64_t n, const CODE *lo, const CODE *hi, int np, BITS *out,
                        uint64_t stride, unsigned long long *counts, hipStream_t s) {
   if (!col || !lo || !hi || np < 1 || (n && !out)) return hipErrorInvalidValue;
@@ -458,11 +763,7 @@ hipError_t scan_ranges(const CODE *col, uint64_t n, const CODE *lo, const CODE *
     if (counts) return hipMemsetAsync(counts, 0, (size_t)np * sizeof(unsigned long long), s);
     return hipSuccess;
   }
-  const uint64_t ntiles = aligned16(col) ? n / kMultiTileRows : 0;
-  const uint64_t waves = std::max<uint64_t>(ntiles, (n - ntiles * kMultiTileRows + 63) / 64);
-  const unsigned grid = grid_for(waves, kBlock / kWave, std::min<unsigned>(kMultiMaxGrid, stream_grid_cap() * 2));
-  // predicate groups: enough workgroups for 4 per compute unit, at least 8 predicates each
-  const unsigned want = (unsigned)std::max(1, device_cu_count()) * 4;
+  const unsigned cus = (unsigned)std::max(1, device_cu_count());
   uint32_t *partials = nullptr;
   if (counts) {
     void *pp = nullptr;
@@ -473,30 +774,55 @@ hipError_t scan_ranges(const CODE *col, uint64_t n, const CODE *lo, const CODE *
   }
   for (int p0 = 0; p0 < np; p0 += kMultiPreds) {  // one pass over the column per 64 predicates
     const int k = std::min(kMultiPreds, np - p0);
-    MultiPreds mp{};
-    for (int p = 0; p < k; p++) {
-      if (lo[p0 + p] > hi[p0 + p]) {
-        mp.empty |= 1ull << p;
-      } else {
-        mp.lo[p] = lo[p0 + p];
-        mp.span[p] = hi[p0 + p] - lo[p0 + p];
-      }
-    }
     BITS *o = out + (uint64_t)p0 * stride;
-    const int groups = (int)std::max<unsigned>(1, std::min<unsigned>((k + 7) / 8, (want + grid - 1) / grid));
-    const int pper = (k + groups - 1) / groups;
-    const dim3 g2(grid, (unsigned)((k + pper - 1) / pper));
-    if (counts) {
-      hipLaunchKernelGGL(k_scan_multi<true>, g2, dim3(kBlock), 0, s, col, n, ntiles, mp, k, pper, o, stride,
-                         partials);
-      hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return e;
-      hipLaunchKernelGGL(k_multi_counts, dim3(k), dim3(kBlock), 0, s, partials, grid, counts + p0);
+    unsigned grid;
+    if (k > direct_preds(n)) {
+      const RankedPreds t = rank_table(lo + p0, hi + p0, k);
+      const uint64_t wgtiles = (n + kMultiTileRows * (kBlock / kWave) - 1) / (kMultiTileRows * (kBlock / kWave));
+      // a tile a wave while the workgroups all fit at once (4 per compute unit); a long
+      // column takes more, shorter workgroups, which even out (1e8 rows, 64 predicates: 338
+      // us with 4 per compute unit, 322 with 16; 1e7 rows: 32 against 38), and gives an XCD
+      // runs of 16 steps (337 against 366 us)
+      const bool large = wgtiles >= cus * 16;
+      grid = grid_for(wgtiles, 1, std::min<unsigned>(kMultiMaxGrid, cus * (large ? 16 : 4)));
+      grid = (grid + kScanXcds - 1) / kScanXcds * kScanXcds;
+      const uint32_t run = large ? 16 : 1;
+      if (k <= 32)
+        launch_ranked<1>(col, n, t, k, o, stride, run, partials, dim3(grid), s);
+      else if (grid < cus * 2)  // the halves in workgroups of their own, so that a short column fills the device
+        launch_ranked<1>(col, n, t, k, o, stride, run, partials, dim3(grid, 2), s);
+      else
+        launch_ranked<2>(col, n, t, k, o, stride, run, partials, dim3(grid), s);
     } else {
-      hipLaunchKernelGGL(k_scan_multi<false>, g2, dim3(kBlock), 0, s, col, n, ntiles, mp, k, pper, o, stride,
-                         nullptr);
+      const uint64_t ntiles = aligned16(col) ? n / kMultiTileRows : 0;
+      const uint64_t waves = std::max<uint64_t>(ntiles, (n - ntiles * kMultiTileRows + 63) / 64);
+      grid = grid_for(waves, kBlock / kWave, std::min<unsigned>(kMultiMaxGrid, stream_grid_cap() * 2));
+      MultiPreds mp{};
+      for (int p = 0; p < k; p++) {
+        if (lo[p0 + p] > hi[p0 + p]) {
+          mp.empty |= 1ull << p;
+        } else {
+          mp.lo[p] = lo[p0 + p];
+          mp.span[p] = hi[p0 + p] - lo[p0 + p];
+        }
+      }
+      // predicate groups: enough workgroups for 4 per compute unit, at least 8 predicates each
+      const unsigned want = cus * 4;
+      const int groups = (int)std::max<unsigned>(1, std::min<unsigned>((k + 7) / 8, (want + grid - 1) / grid));
+      const int pper = (k + groups - 1) / groups;
+      const dim3 g2(grid, (unsigned)((k + pper - 1) / pper));
+      if (counts)
+        hipLaunchKernelGGL(k_scan_multi<true>, g2, dim3(kBlock), 0, s, col, n, ntiles, mp, k, pper, o, stride,
+                           partials);
+      else
+        hipLaunchKernelGGL(k_scan_multi<false>, g2, dim3(kBlock), 0, s, col, n, ntiles, mp, k, pper, o, stride,
+                           nullptr);
     }
-    const hipError_t e = hipGetLastError();
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && counts) {
+      hipLaunchKernelGGL(k_multi_counts, dim3(k), dim3(kBlock), 0, s, partials, grid, counts + p0);
+      e = hipGetLastError();
+    }
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

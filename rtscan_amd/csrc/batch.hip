@@ -762,7 +762,7 @@ static hipError_t build_dirs(rts_batch_plan *p, hipStream_t s) {
   const int64_t ntiles = (p->n + tile_rows - 1) / tile_rows;
   p->dir_base.assign(p->ncols, nullptr);
   p->dir_tiles.assign(p->ncols, ntiles);
-  hipError_t ze = hipMalloc((void **)&p->d_zero_dir, (ntiles + 1) * sizeof(uint32_t));
+  hipError_t ze = device_malloc((void **)&p->d_zero_dir, (ntiles + 1) * sizeof(uint32_t));
   if (ze == hipSuccess) ze = hipMemsetAsync(p->d_zero_dir, 0, (ntiles + 1) * sizeof(uint32_t), s);
   if (ze != hipSuccess) return ze;
   for (int c = 0; c < p->ncols; c++) {
@@ -770,7 +770,7 @@ static hipError_t build_dirs(rts_batch_plan *p, hipStream_t s) {
     if (!b || !b->dev) continue;
     const rts_bindex_dev *d = b->dev;
     const int64_t items = (int64_t)d->bins * (ntiles + 1);
-    hipError_t e = hipMalloc((void **)&p->dir_base[c], items * sizeof(uint32_t));
+    hipError_t e = device_malloc((void **)&p->dir_base[c], items * sizeof(uint32_t));
     if (e != hipSuccess) return e;
     e = launch_tile_directory(d, ntiles, tile_rows, p->dir_base[c], s);
     if (e != hipSuccess) return e;
@@ -868,13 +868,13 @@ hipError_t rts_batch_plan_create(rts_batch_plan **out, const CODE *const *column
   }
   p->active_set = set_for(p, p->cfg);
   p->index = p->index_sets[p->active_set].data();
-  hipError_t e = hipMalloc((void **)&p->d_groups, (size_t)max_queries * sizeof(BatchGroup));
-  if (e == hipSuccess) e = hipMalloc((void **)&p->d_ngroups, sizeof(int));
-  if (e == hipSuccess) e = hipMalloc((void **)&p->d_sched, kSchedWords * sizeof(unsigned long long));
+  hipError_t e = device_malloc((void **)&p->d_groups, (size_t)max_queries * sizeof(BatchGroup));
+  if (e == hipSuccess) e = device_malloc((void **)&p->d_ngroups, sizeof(int));
+  if (e == hipSuccess) e = device_malloc((void **)&p->d_sched, kSchedWords * sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMemsetAsync(p->d_sched, 0, kSchedWords * sizeof(unsigned long long), stream);
   if (e == hipSuccess) e = build_dirs(p, stream);
   if (e == hipSuccess)
-    e = hipMalloc((void **)&p->d_partials, (size_t)max_queries * p->ntiles * sizeof(uint32_t));
+    e = device_malloc((void **)&p->d_partials, (size_t)max_queries * p->ntiles * sizeof(uint32_t));
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
   if (e != hipSuccess) {
     rts_batch_plan_free(p);
@@ -912,7 +912,7 @@ hipError_t rts_batch_plan_set_config(rts_batch_plan *p, const rts_batch_config *
   if (e == hipSuccess && retile) {
     (void)hipFree(p->d_partials);
     p->d_partials = nullptr;
-    e = hipMalloc((void **)&p->d_partials, (size_t)p->max_queries * p->ntiles * sizeof(uint32_t));
+    e = device_malloc((void **)&p->d_partials, (size_t)p->max_queries * p->ntiles * sizeof(uint32_t));
   }
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
   if (e != hipSuccess) return set_error(e, "rts_batch_plan_set_config");

@@ -270,8 +270,8 @@ hipError_t start_ranks(const rts_bindex_dev *d, std::vector<int64_t> &rk, hipStr
   CODE *est = nullptr;
   int64_t *rk_d = nullptr;
   rk.assign(2 * (size_t)bins, 0);
-  hipError_t e = hipMalloc((void **)&est, bins * sizeof(CODE));
-  if (e == hipSuccess) e = hipMalloc((void **)&rk_d, 2 * (size_t)bins * sizeof(int64_t));
+  hipError_t e = pool_alloc(&est, bins * sizeof(CODE));
+  if (e == hipSuccess) e = pool_alloc(&rk_d, 2 * (size_t)bins * sizeof(int64_t));
   if (e == hipSuccess) e = hipMemcpyAsync(est, d->estarts.data(), bins * sizeof(CODE), hipMemcpyHostToDevice, s);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_start_ranks, dim3((bins + kBlock - 1) / kBlock), dim3(kBlock), 0, s, d->sorted_val, d->n,
@@ -280,8 +280,8 @@ hipError_t start_ranks(const rts_bindex_dev *d, std::vector<int64_t> &rk, hipStr
   }
   if (e == hipSuccess) e = hipMemcpyAsync(rk.data(), rk_d, 2 * (size_t)bins * sizeof(int64_t), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  (void)hipFree(est);
-  (void)hipFree(rk_d);
+  pool_free(est, e == hipSuccess);
+  pool_free(rk_d, e == hipSuccess);
   return e;
 }
 
@@ -297,7 +297,7 @@ hipError_t rank_samples(rts_bindex_dev *d, hipStream_t s) {
   const int64_t m = (d->n + kRankSample - 1) / kRankSample;
   CODE *smp = nullptr;
   d->rank_samples.assign(m, 0);
-  hipError_t e = hipMalloc((void **)&smp, m * sizeof(CODE));
+  hipError_t e = pool_alloc(&smp, m * sizeof(CODE));
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_rank_samples, dim3((unsigned)((m + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
                        d->sorted_val, m, smp);
@@ -305,18 +305,21 @@ hipError_t rank_samples(rts_bindex_dev *d, hipStream_t s) {
   }
   if (e == hipSuccess) e = hipMemcpyAsync(d->rank_samples.data(), smp, m * sizeof(CODE), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  (void)hipFree(smp);
+  pool_free(smp, e == hipSuccess);
   return e;
 }
 
 static void free_dev(rts_bindex_dev *d) {
   if (!d) return;
-  (void)hipFree(d->sorted_val);
-  (void)hipFree(d->sorted_pos);
-  (void)hipFree(d->fvs);
-  (void)hipFree(d->bent);
-  (void)hipFree(d->boff);
-  (void)hipFree(d->bdir);
+  // queries of any stream may still read the arrays: wait for them, as hipFree does
+  int dev = 0;
+  const bool here = hipGetDevice(&dev) == hipSuccess;
+  const bool away = here && d->device != dev && hipSetDevice(d->device) == hipSuccess;
+  const bool idle = here && (away || d->device == dev) && hipDeviceSynchronize() == hipSuccess;
+  for (void *p : {(void *)d->sorted_val, (void *)d->sorted_pos, (void *)d->fvs, (void *)d->bent, (void *)d->boff,
+                  (void *)d->bdir})
+    pool_free(p, idle);
+  if (away) (void)hipSetDevice(dev);
   (void)hipFree(d->owned_column);
   delete d;
 }
@@ -424,6 +427,7 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
     return hipErrorInvalidValue;
   memset(bx, 0, sizeof(*bx));
   d = new rts_bindex_dev();
+  RTS_TRY(hipGetDevice(&d->device));
   d->n = n;
   d->words = (n + 31) / 32;
   d->fv_stride = (d->words + kFvStrideAlign - 1) / kFvStrideAlign * kFvStrideAlign;
@@ -434,22 +438,22 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   while ((1 << key_bits) <= bins) key_bits++;  // keys 0..bins
 
   // 1. stable sort of (value, row)
-  RTS_TRY(hipMalloc((void **)&d->sorted_val, n * sizeof(CODE)));
-  RTS_TRY(hipMalloc((void **)&d->sorted_pos, n * sizeof(int32_t)));
-  RTS_TRY(hipMalloc((void **)&iota, n * sizeof(uint32_t)));
+  RTS_TRY(pool_alloc(&d->sorted_val, n * sizeof(CODE)));
+  RTS_TRY(pool_alloc(&d->sorted_pos, n * sizeof(int32_t)));
+  RTS_TRY(pool_alloc(&iota, n * sizeof(uint32_t)));
   hipLaunchKernelGGL(k_iota, dim3(blocks_for(n)), dim3(kBlock), 0, s, iota, n);
   RTS_TRY(hipGetLastError());
   RTS_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, need, col, d->sorted_val, iota,
                                              (uint32_t *)d->sorted_pos, (int)n, 0, 32, s));
   tmp_bytes = need;
-  RTS_TRY(hipMalloc(&tmp, tmp_bytes));
+  RTS_TRY(pool_alloc(&tmp, tmp_bytes));
   RTS_TRY(hipcub::DeviceRadixSort::SortPairs(tmp, need, col, d->sorted_val, iota,
                                              (uint32_t *)d->sorted_pos, (int)n, 0, 32, s));
 
   // 2. area starts, then bin starts
-  RTS_TRY(hipMalloc((void **)&starts_d, kAreas * sizeof(CODE)));
-  RTS_TRY(hipMalloc((void **)&idx_d, kAreas * sizeof(int64_t)));
-  RTS_TRY(hipMalloc((void **)&estarts_d, bins * sizeof(CODE)));
+  RTS_TRY(pool_alloc(&starts_d, kAreas * sizeof(CODE)));
+  RTS_TRY(pool_alloc(&idx_d, kAreas * sizeof(int64_t)));
+  RTS_TRY(pool_alloc(&estarts_d, bins * sizeof(CODE)));
   hipLaunchKernelGGL(k_area_starts, dim3(1), dim3(kAreas), 0, s, d->sorted_val, n, starts_d, idx_d);
   RTS_TRY(hipGetLastError());
   hipLaunchKernelGGL(k_bin_starts, dim3((bins + kBlock - 1) / kBlock), dim3(kBlock), 0, s, d->sorted_val, n,
@@ -466,10 +470,10 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   RTS_TRY(hipStreamSynchronize(s));  // d->estarts
   RTS_TRY(start_ranks(d, rk, s));
   for (int k = 0; k < bins; k++) light_h[k] = rk[2 * k + 1] - rk[2 * k] <= kLightStartRows;
-  RTS_TRY(hipMalloc((void **)&light_d, bins));
+  RTS_TRY(pool_alloc(&light_d, bins));
   RTS_TRY(hipMemcpyAsync(light_d, light_h, bins, hipMemcpyHostToDevice, s));
-  RTS_TRY(hipMalloc((void **)&d->fvs, (size_t)(bins - 1) * d->fv_stride * sizeof(BITS)));
-  RTS_TRY(hipMalloc((void **)&keys, n * sizeof(uint16_t)));
+  RTS_TRY(pool_alloc(&d->fvs, (size_t)(bins - 1) * d->fv_stride * sizeof(BITS)));
+  RTS_TRY(pool_alloc(&keys, n * sizeof(uint16_t)));
   {
     const dim3 grid(blocks_for((n + kFvTileRows - 1) / kFvTileRows, kBlock / kWave));
     if (bins <= 128)
@@ -488,18 +492,19 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   RTS_TRY(hipGetLastError());
 
   // 4. B lists: stable sort of (key, row) -> rows grouped by bin in row order
-  RTS_TRY(hipMalloc((void **)&skeys, n * sizeof(uint16_t)));
-  RTS_TRY(hipMalloc((void **)&bpos_in, n * sizeof(uint32_t)));
+  RTS_TRY(pool_alloc(&skeys, n * sizeof(uint16_t)));
+  RTS_TRY(pool_alloc(&bpos_in, n * sizeof(uint32_t)));
   RTS_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, need, keys, skeys, iota, bpos_in, (int)n, 0,
                                              key_bits, s));
   if (need > tmp_bytes) {
-    (void)hipFree(tmp);
+    RTS_TRY(hipStreamSynchronize(s));
+    pool_free(tmp, true);
     tmp = nullptr;
     tmp_bytes = need;
-    RTS_TRY(hipMalloc(&tmp, tmp_bytes));
+    RTS_TRY(pool_alloc(&tmp, tmp_bytes));
   }
   RTS_TRY(hipcub::DeviceRadixSort::SortPairs(tmp, need, keys, skeys, iota, bpos_in, (int)n, 0, key_bits, s));
-  RTS_TRY(hipMalloc((void **)&d->boff, (bins + 1) * sizeof(uint32_t)));
+  RTS_TRY(pool_alloc(&d->boff, (bins + 1) * sizeof(uint32_t)));
   hipLaunchKernelGGL(k_bin_offsets, dim3((bins + 1 + kBlock - 1) / kBlock), dim3(kBlock), 0, s, skeys, n, bins,
                      d->boff);
   RTS_TRY(hipGetLastError());
@@ -510,13 +515,13 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   nb = d->boff_host[bins];
   d->nb = nb;
   mark_complete_bins(d, rk);
-  RTS_TRY(hipMalloc((void **)&d->bent, std::max<uint32_t>(nb, 1) * sizeof(uint2)));
+  RTS_TRY(pool_alloc(&d->bent, std::max<uint32_t>(nb, 1) * sizeof(uint2)));
   if (nb) {
     hipLaunchKernelGGL(k_gather_entries, dim3(blocks_for(nb)), dim3(kBlock), 0, s, col, bpos_in,
                        d->bent, (int64_t)nb);
     RTS_TRY(hipGetLastError());
   }
-  RTS_TRY(hipMalloc((void **)&d->bdir, (size_t)bins * (d->ntiles + 1) * sizeof(uint32_t)));
+  RTS_TRY(pool_alloc(&d->bdir, (size_t)bins * (d->ntiles + 1) * sizeof(uint32_t)));
   RTS_TRY(launch_tile_directory(d, d->ntiles, kTileRows, d->bdir, s));
 
   // 5. host descriptor: areas (bindex.cpp:633-652) and their blocks
@@ -538,10 +543,10 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   nblocks = (int64_t)bf_slot.size();
   d->block_first.resize(nblocks);
   d->block_last.resize(nblocks);
-  RTS_TRY(hipMalloc((void **)&bf_slot_d, nblocks * sizeof(int64_t)));
-  RTS_TRY(hipMalloc((void **)&bl_slot_d, nblocks * sizeof(int64_t)));
-  RTS_TRY(hipMalloc((void **)&bfirst_d, nblocks * sizeof(CODE)));
-  RTS_TRY(hipMalloc((void **)&blast_d, nblocks * sizeof(CODE)));
+  RTS_TRY(pool_alloc(&bf_slot_d, nblocks * sizeof(int64_t)));
+  RTS_TRY(pool_alloc(&bl_slot_d, nblocks * sizeof(int64_t)));
+  RTS_TRY(pool_alloc(&bfirst_d, nblocks * sizeof(CODE)));
+  RTS_TRY(pool_alloc(&blast_d, nblocks * sizeof(CODE)));
   RTS_TRY(hipMemcpyAsync(bf_slot_d, bf_slot.data(), nblocks * sizeof(int64_t), hipMemcpyHostToDevice, s));
   RTS_TRY(hipMemcpyAsync(bl_slot_d, bl_slot.data(), nblocks * sizeof(int64_t), hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL(k_block_bounds, dim3((unsigned)((nblocks + kBlock - 1) / kBlock)), dim3(kBlock), 0,
@@ -556,19 +561,13 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   d = nullptr;
 
 fail:
-  (void)hipFree(iota);
-  (void)hipFree(bpos_in);
-  (void)hipFree(keys);
-  (void)hipFree(skeys);
-  (void)hipFree(tmp);
-  (void)hipFree(starts_d);
-  (void)hipFree(estarts_d);
-  (void)hipFree(light_d);
-  (void)hipFree(idx_d);
-  (void)hipFree(bf_slot_d);
-  (void)hipFree(bl_slot_d);
-  (void)hipFree(bfirst_d);
-  (void)hipFree(blast_d);
+  {
+    const bool idle = hipStreamSynchronize(s) == hipSuccess;  // before other calls get the workspaces
+    for (void *p : {(void *)iota, (void *)bpos_in, (void *)keys, (void *)skeys, tmp, (void *)starts_d,
+                    (void *)estarts_d, (void *)light_d, (void *)idx_d, (void *)bf_slot_d, (void *)bl_slot_d,
+                    (void *)bfirst_d, (void *)blast_d})
+      pool_free(p, idle);
+  }
   if (d) {
     d->owned_column = nullptr;  // the caller frees what it passed in on failure
     free_dev(d);
@@ -782,6 +781,9 @@ hipError_t bindex_load(BinDex *bx, const char *path, const CODE *col) {
       h.nblocks > h.n)
     goto done;
   d = new rts_bindex_dev();
+  e = hipGetDevice(&d->device);
+  if (e != hipSuccess) goto done;
+  e = hipErrorInvalidValue;
   d->n = h.n;
   d->words = h.words;
   d->fv_stride = h.fv_stride;
@@ -802,12 +804,12 @@ hipError_t bindex_load(BinDex *bx, const char *path, const CODE *col) {
   if (host_digest(d) != h.dg_host || !host_arrays_valid(d, h.nblocks)) goto done;
   fv_words = (size_t)(d->bins - 1) * h.fv_stride;
   e = hipHostMalloc(&stage, kStage, hipHostMallocDefault);
-  if (e == hipSuccess) e = hipMalloc((void **)&d->sorted_val, h.n * sizeof(CODE));
-  if (e == hipSuccess) e = hipMalloc((void **)&d->sorted_pos, h.n * sizeof(int32_t));
-  if (e == hipSuccess) e = hipMalloc((void **)&d->fvs, fv_words * sizeof(BITS));
-  if (e == hipSuccess) e = hipMalloc((void **)&d->bent, std::max<int64_t>(h.nb, 1) * sizeof(uint2));
-  if (e == hipSuccess) e = hipMalloc((void **)&d->boff, (d->bins + 1) * sizeof(uint32_t));
-  if (e == hipSuccess) e = hipMalloc((void **)&d->bdir, (size_t)d->bins * (h.ntiles + 1) * sizeof(uint32_t));
+  if (e == hipSuccess) e = pool_alloc(&d->sorted_val, h.n * sizeof(CODE));
+  if (e == hipSuccess) e = pool_alloc(&d->sorted_pos, h.n * sizeof(int32_t));
+  if (e == hipSuccess) e = pool_alloc(&d->fvs, fv_words * sizeof(BITS));
+  if (e == hipSuccess) e = pool_alloc(&d->bent, std::max<int64_t>(h.nb, 1) * sizeof(uint2));
+  if (e == hipSuccess) e = pool_alloc(&d->boff, (d->bins + 1) * sizeof(uint32_t));
+  if (e == hipSuccess) e = pool_alloc(&d->bdir, (size_t)d->bins * (h.ntiles + 1) * sizeof(uint32_t));
   if (e == hipSuccess) e = get_device(f, d->sorted_val, h.n * sizeof(CODE), stage, kNoCheck);
   if (e == hipSuccess) e = get_device(f, d->sorted_pos, h.n * sizeof(int32_t), stage, kNoCheck);
   if (e == hipSuccess) e = get_device(f, d->fvs, fv_words * sizeof(BITS), stage, kNoCheck);

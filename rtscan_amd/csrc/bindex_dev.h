@@ -53,6 +53,7 @@ constexpr int64_t kLightStartRows = 64;       // a bin start of at most this man
 }  // namespace rts
 
 struct rts_bindex_dev {
+  int device = 0;  // that holds the arrays
   int64_t n = 0;
   int64_t words = 0;
   int64_t fv_stride = 0;

@@ -601,7 +601,7 @@ hipError_t rts_bindex_load(BinDex *bindex, const char *path, const CODE *dev_col
 hipError_t rts_bindex_build_host(BinDex *bindex, const CODE *host_column, POSTYPE n) {
   if (!bindex || !host_column || n <= 0) return set_error(hipErrorInvalidValue, "rts_bindex_build_host");
   CODE *d = nullptr;
-  hipError_t e = hipMalloc((void **)&d, (size_t)n * sizeof(CODE));
+  hipError_t e = device_malloc((void **)&d, (size_t)n * sizeof(CODE));
   if (e == hipSuccess) e = hipMemcpy(d, host_column, (size_t)n * sizeof(CODE), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = bindex_build(bindex, d, n, d, 1, ref_stream());
   if (e == hipSuccess) e = hipStreamSynchronize(ref_stream());

@@ -112,7 +112,7 @@ hipError_t thread_scratch(int kind, hipStream_t stream, size_t dev_bytes, size_t
   }
   if (created) *created = true;
   ScratchEntry x{kind, dev, (uintptr_t)stream, nullptr, nullptr};
-  if (dev_bytes) e = hipMalloc(&x.dptr, dev_bytes);
+  if (dev_bytes) e = device_malloc(&x.dptr, dev_bytes);
   if (e == hipSuccess && host_bytes) e = hipHostMalloc(&x.hptr, host_bytes, 0);
   if (e != hipSuccess) {
     ThreadScratch::release(x);
@@ -221,8 +221,8 @@ hipError_t CPUbitAndWithCuda(BITS *host_a, BITS *host_b, unsigned int size) {
   const size_t words = ref_words((int)size);
   const size_t bytes = words * sizeof(BITS);
   BITS *da = nullptr, *db = nullptr;
-  hipError_t e = hipMalloc((void **)&da, bytes);
-  if (e == hipSuccess) e = hipMalloc((void **)&db, bytes);
+  hipError_t e = device_malloc((void **)&da, bytes);
+  if (e == hipSuccess) e = device_malloc((void **)&db, bytes);
   if (e == hipSuccess) e = hipMemcpy(da, host_a, bytes, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(db, host_b, bytes, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = bitop(kAnd, da, db, nullptr, words, 0, ref_stream());
@@ -237,7 +237,7 @@ hipError_t refineWithCuda(CODE *bitmap, unsigned int size) {
   const size_t bytes = (size_t)size * sizeof(BITS);
   if (size == 0) return hipSuccess;
   BITS *d = nullptr;
-  hipError_t e = hipMalloc((void **)&d, bytes);
+  hipError_t e = device_malloc((void **)&d, bytes);
   if (e == hipSuccess) e = hipMemcpy(d, bitmap, bytes, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = flip_rows(d, size, ref_stream());
   if (e == hipSuccess) e = hipStreamSynchronize(ref_stream());
@@ -389,8 +389,8 @@ void raw_scan(struct BinDex *bindex, BITS *bitmap, CODE t1, CODE t2, enum OPERAT
   const size_t words = words_for_rows((uint64_t)n);
   CODE *dcol = nullptr;
   BITS *dbm = nullptr;
-  hipError_t e = hipMalloc((void **)&dcol, (size_t)n * sizeof(CODE));
-  if (e == hipSuccess) e = hipMalloc((void **)&dbm, words * sizeof(BITS));
+  hipError_t e = device_malloc((void **)&dcol, (size_t)n * sizeof(CODE));
+  if (e == hipSuccess) e = device_malloc((void **)&dbm, words * sizeof(BITS));
   if (e == hipSuccess) e = hipMemcpy(dcol, raw_data, (size_t)n * sizeof(CODE), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(dbm, bitmap, words * sizeof(BITS), hipMemcpyHostToDevice);
   const CODE *cols[1] = {dcol};
@@ -404,7 +404,7 @@ void raw_scan(struct BinDex *bindex, BITS *bitmap, CODE t1, CODE t2, enum OPERAT
 
 // ------------------------------------------------------------------- helpers
 
-hipError_t rts_malloc(void **ptr, size_t bytes) { return set_error(hipMalloc(ptr, bytes), "rts_malloc"); }
+hipError_t rts_malloc(void **ptr, size_t bytes) { return set_error(device_malloc(ptr, bytes), "rts_malloc"); }
 hipError_t rts_free(void *ptr) { return set_error(hipFree(ptr), "rts_free"); }
 hipError_t rts_memcpy_htod(void *dst, const void *src, size_t bytes) {
   return set_error(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice), "rts_memcpy_htod");
@@ -486,6 +486,8 @@ int rts_thread_scratch_buffers(void) { return (int)thread_scratch_entries(); }
 
 hipError_t rts_device_mem_info(size_t *free_bytes, size_t *total_bytes) {
   size_t f = 0, t = 0;
+  int dev = 0;
+  if (hipGetDevice(&dev) == hipSuccess) pool_trim(dev);  // what the library keeps counts as free
   hipError_t e = hipMemGetInfo(&f, &t);
   if (e != hipSuccess) return set_error(e, "rts_device_mem_info");
   if (free_bytes) *free_bytes = f;

@@ -276,8 +276,8 @@ extern "C" void compare_bitmap(BITS *bitmap_a, BITS *bitmap_b, int len, CODE **r
   const size_t bytes = rts::words_for_rows((uint64_t)len) * sizeof(BITS);
   BITS *da = nullptr, *db = nullptr;
   rts_compare_result r{};
-  hipError_t e = hipMalloc((void **)&da, bytes);
-  if (e == hipSuccess) e = hipMalloc((void **)&db, bytes);
+  hipError_t e = rts::device_malloc((void **)&da, bytes);
+  if (e == hipSuccess) e = rts::device_malloc((void **)&db, bytes);
   if (e == hipSuccess) e = hipMemcpy(da, bitmap_a, bytes, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(db, bitmap_b, bytes, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = rts::bitmap_compare(da, db, len, &r, rts::ref_stream());

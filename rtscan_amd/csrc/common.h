@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "device_mem.h"
 #include "rtscan_hip.h"
 
 namespace rts {

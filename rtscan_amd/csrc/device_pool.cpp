@@ -1,0 +1,142 @@
+// device_pool.cpp -- device memory that outlives one call: an index's arrays and the
+// workspaces of index builds and column encodings.
+//
+// hipMalloc and hipFree of such blocks cost as much as the work in them: 0.1 and 0.3 ms a
+// block in a fresh process, and about 25 us a megabyte to free once a process has used most
+// of the device's memory (a 1e8-row build takes 5.6 GB in 13 blocks and runs 8 ms of
+// kernels; encoding a 1e8-row column 2.9 GB in 6 blocks).  Freed blocks are therefore kept
+// for the next call of any thread or stream:
+//   - a block is given to pool_free only when no queued work can touch it any more, so it
+//     can be handed out at once;
+//   - at most kPoolBytes are kept on each device, the oldest going back first;
+//   - all of a device's kept blocks go back when an allocation of the library fails there
+//     (which is then tried again) and when a caller asks how much memory is free.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <iterator>
+#include <list>
+#include <mutex>
+#include <unordered_map>
+
+#include "device_mem.h"
+
+namespace rts {
+namespace {
+
+constexpr size_t kPoolBytes = (size_t)8 << 30;  // kept on each device, at most
+
+// Sizes are rounded up, so that a freed block fits the next call's.
+size_t rounded(size_t bytes) {
+  const size_t granule = bytes < ((size_t)1 << 20) ? (size_t)64 << 10 : (size_t)2 << 20;
+  return (std::max<size_t>(bytes, 1) + granule - 1) / granule * granule;
+}
+
+struct Block {
+  void *ptr;
+  size_t bytes;
+  int dev;
+};
+
+struct Pool {
+  std::mutex mu;
+  std::list<Block> kept;                         // oldest first
+  std::unordered_map<void *, Block> in_use;
+};
+
+// Never destroyed: blocks may be freed while the process ends, in any order.
+Pool &pool() {
+  static Pool *p = new Pool;
+  return *p;
+}
+
+// hipFree of blocks taken off the pool's lists, outside its lock (hipFree waits for the device).
+void give_back(const std::list<Block> &blocks) {
+  for (const Block &b : blocks) (void)hipFree(b.ptr);
+}
+
+}  // namespace
+
+void pool_trim(int dev) {
+  std::list<Block> out;
+  {
+    Pool &p = pool();
+    std::lock_guard<std::mutex> lock(p.mu);
+    for (auto it = p.kept.begin(); it != p.kept.end();) {
+      auto next = std::next(it);
+      if (it->dev == dev) out.splice(out.end(), p.kept, it);
+      it = next;
+    }
+  }
+  give_back(out);
+}
+
+hipError_t device_malloc(void **ptr, size_t bytes) {
+  hipError_t e = hipMalloc(ptr, bytes);
+  int dev = 0;
+  if (e != hipErrorOutOfMemory || hipGetDevice(&dev) != hipSuccess) return e;
+  (void)hipGetLastError();  // the first try's error is not the caller's
+  pool_trim(dev);
+  return hipMalloc(ptr, bytes);
+}
+
+hipError_t pool_alloc(void **ptr, size_t bytes) {
+  *ptr = nullptr;
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  bytes = rounded(bytes);
+  Pool &p = pool();
+  {
+    std::lock_guard<std::mutex> lock(p.mu);
+    auto best = p.kept.end();  // the smallest block that holds it and wastes at most a quarter
+    for (auto it = p.kept.begin(); it != p.kept.end(); ++it)
+      if (it->dev == dev && it->bytes >= bytes && it->bytes <= bytes + bytes / 4 &&
+          (best == p.kept.end() || it->bytes < best->bytes))
+        best = it;
+    if (best != p.kept.end()) {
+      p.in_use.emplace(best->ptr, *best);
+      *ptr = best->ptr;
+      p.kept.erase(best);
+      return hipSuccess;
+    }
+  }
+  void *q = nullptr;
+  e = device_malloc(&q, bytes);
+  if (e != hipSuccess) return e;
+  std::lock_guard<std::mutex> lock(p.mu);
+  p.in_use.emplace(q, Block{q, bytes, dev});
+  *ptr = q;
+  return hipSuccess;
+}
+
+void pool_free(void *ptr, bool idle) {
+  if (!ptr) return;
+  std::list<Block> out;
+  {
+    Pool &p = pool();
+    std::lock_guard<std::mutex> lock(p.mu);
+    auto it = p.in_use.find(ptr);
+    if (it == p.in_use.end()) return;
+    const Block b = it->second;
+    p.in_use.erase(it);
+    if (!idle) {  // the device may still use it: hipFree waits
+      out.push_back(b);
+    } else {
+      p.kept.push_back(b);
+      size_t total = 0;
+      for (const Block &k : p.kept) total += k.dev == b.dev ? k.bytes : 0;
+      for (auto k = p.kept.begin(); k != p.kept.end() && total > kPoolBytes;) {
+        auto next = std::next(k);
+        if (k->dev == b.dev) {
+          total -= k->bytes;
+          out.splice(out.end(), p.kept, k);
+        }
+        k = next;
+      }
+    }
+  }
+  give_back(out);
+}
+
+}  // namespace rts

@@ -122,11 +122,12 @@ struct Runs {
   uint32_t *run = nullptr;
   bool own_spos = false;
   int64_t m = 0;
-  void release() {
-    (void)hipFree(sval);
-    if (own_spos) (void)hipFree(spos);
-    (void)hipFree(head);
-    (void)hipFree(run);
+  // idle: no queued work uses them any more
+  void release(bool idle) {
+    pool_free(sval, idle);
+    if (own_spos) pool_free(spos, idle);
+    pool_free(head, idle);
+    pool_free(run, idle);
   }
 };
 
@@ -137,23 +138,23 @@ hipError_t sorted_runs(const CODE *data, int64_t n, POSTYPE *caller_spos, Runs &
   size_t need = 0, have = 0;
   uint32_t last = 0;
 
-  RTS_TRY(hipMalloc((void **)&R.sval, n * sizeof(CODE)));
+  RTS_TRY(pool_alloc(&R.sval, n * sizeof(CODE)));
   if (caller_spos) {
     R.spos = (uint32_t *)caller_spos;
   } else {
-    RTS_TRY(hipMalloc((void **)&R.spos, n * sizeof(uint32_t)));
+    RTS_TRY(pool_alloc(&R.spos, n * sizeof(uint32_t)));
     R.own_spos = true;
   }
-  RTS_TRY(hipMalloc((void **)&R.head, n * sizeof(uint32_t)));
-  RTS_TRY(hipMalloc((void **)&R.run, n * sizeof(uint32_t)));
-  RTS_TRY(hipMalloc((void **)&iota, n * sizeof(uint32_t)));
+  RTS_TRY(pool_alloc(&R.head, n * sizeof(uint32_t)));
+  RTS_TRY(pool_alloc(&R.run, n * sizeof(uint32_t)));
+  RTS_TRY(pool_alloc(&iota, n * sizeof(uint32_t)));
   hipLaunchKernelGGL(k_remap_iota, dim3(grid_for(n)), dim3(kRemapBlock), 0, s, iota, n);
   RTS_TRY(hipGetLastError());
   RTS_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, need, data, R.sval, iota, R.spos, (int)n, 0, 32, s));
   have = need;
   RTS_TRY(hipcub::DeviceScan::InclusiveSum(nullptr, need, R.head, R.run, (int)n, s));
   have = need > have ? need : have;
-  RTS_TRY(hipMalloc(&tmp, have));
+  RTS_TRY(pool_alloc(&tmp, have));
   need = have;
   RTS_TRY(hipcub::DeviceRadixSort::SortPairs(tmp, need, data, R.sval, iota, R.spos, (int)n, 0, 32, s));
   hipLaunchKernelGGL(k_run_heads, dim3(grid_for(n)), dim3(kRemapBlock), 0, s, R.sval, n, R.head);
@@ -165,8 +166,8 @@ hipError_t sorted_runs(const CODE *data, int64_t n, POSTYPE *caller_spos, Runs &
   R.m = last;
 
 fail:
-  (void)hipFree(iota);
-  (void)hipFree(tmp);
+  pool_free(iota, err == hipSuccess);
+  pool_free(tmp, err == hipSuccess);
   return err;
 }
 
@@ -189,9 +190,10 @@ hipError_t encode_rank(const CODE *data, int64_t n, CODE encode_min, CODE encode
   hipLaunchKernelGGL(k_rank_codes, dim3(grid_for(n)), dim3(kRemapBlock), 0, s, R.sval, R.spos, R.head,
                      R.run, n, encode_min, interval, codes, sorted_codes, map_values, map_starts);
   RTS_TRY(hipGetLastError());
+  RTS_TRY(hipStreamSynchronize(s));
   *map_size = R.m;
 fail:
-  R.release();
+  R.release(err == hipSuccess);
   return err;
 }
 
@@ -207,16 +209,16 @@ hipError_t encode_dispersed(const CODE *data, int64_t n, CODE encode_min, CODE e
   // remap.cpp:222: double intervalPerObject = (double(max) - double(min)) / double(n)
   const double per_row = ((double)encode_max - (double)encode_min) / (double)n;
   RTS_TRY(sorted_runs(data, n, nullptr, R, s));
-  RTS_TRY(hipMalloc((void **)&first, R.m * sizeof(uint32_t)));
-  RTS_TRY(hipMalloc((void **)&step, R.m * sizeof(uint32_t)));
-  RTS_TRY(hipMalloc((void **)&excl, R.m * sizeof(uint32_t)));
+  RTS_TRY(pool_alloc(&first, R.m * sizeof(uint32_t)));
+  RTS_TRY(pool_alloc(&step, R.m * sizeof(uint32_t)));
+  RTS_TRY(pool_alloc(&excl, R.m * sizeof(uint32_t)));
   hipLaunchKernelGGL(k_run_firsts, dim3(grid_for(n)), dim3(kRemapBlock), 0, s, R.sval, R.head, R.run, n,
                      map_values, first);
   RTS_TRY(hipGetLastError());
   hipLaunchKernelGGL(k_run_steps, dim3(grid_for(R.m)), dim3(kRemapBlock), 0, s, first, R.m, n, per_row, step);
   RTS_TRY(hipGetLastError());
   RTS_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, need, step, excl, (int)R.m, s));
-  RTS_TRY(hipMalloc(&tmp, need));
+  RTS_TRY(pool_alloc(&tmp, need));
   RTS_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, need, step, excl, (int)R.m, s));
   hipLaunchKernelGGL(k_run_starts, dim3(grid_for(R.m)), dim3(kRemapBlock), 0, s, excl, R.m, encode_min,
                      map_starts);
@@ -227,11 +229,8 @@ hipError_t encode_dispersed(const CODE *data, int64_t n, CODE encode_min, CODE e
   RTS_TRY(hipStreamSynchronize(s));
   *map_size = R.m;
 fail:
-  (void)hipFree(first);
-  (void)hipFree(step);
-  (void)hipFree(excl);
-  (void)hipFree(tmp);
-  R.release();
+  for (void *p : {(void *)first, (void *)step, (void *)excl, tmp}) pool_free(p, err == hipSuccess);
+  R.release(err == hipSuccess);
   return err;
 }
 

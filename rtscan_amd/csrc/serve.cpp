@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "admission.h"
+#include "device_mem.h"
 #include "rts_serve.h"
 
 namespace {
@@ -30,7 +31,7 @@ inline uint64_t now_ns() {
 // business (host only).
 struct DeviceRegion {
   char *base = nullptr;
-  bool init(size_t bytes) { return hipMalloc((void **)&base, bytes) == hipSuccess; }
+  bool init(size_t bytes) { return rts::device_malloc((void **)&base, bytes) == hipSuccess; }
   void destroy() {
     if (base) (void)hipFree(base);
     base = nullptr;
@@ -250,7 +251,7 @@ hipError_t rts_server_create(rts_server **out, const rts_server_config *cfg) {
   for (Worker &w : s->workers) {
     hipError_t e = hipStreamCreateWithFlags(&w.stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&w.done, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipMalloc((void **)&w.dcounts, s->cfg.max_batch * sizeof(unsigned long long));
+    if (e == hipSuccess) e = rts::device_malloc((void **)&w.dcounts, s->cfg.max_batch * sizeof(unsigned long long));
     if (e == hipSuccess) e = hipHostMalloc((void **)&w.hcounts, s->cfg.max_batch * sizeof(unsigned long long), 0);
     if (e != hipSuccess) {
       rts_server_destroy(s);

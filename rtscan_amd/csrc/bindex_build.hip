@@ -781,9 +781,6 @@ hipError_t bindex_load(BinDex *bx, const char *path, const CODE *col) {
       h.nblocks > h.n)
     goto done;
   d = new rts_bindex_dev();
-  e = hipGetDevice(&d->device);
-  if (e != hipSuccess) goto done;
-  e = hipErrorInvalidValue;
   d->n = h.n;
   d->words = h.words;
   d->fv_stride = h.fv_stride;
@@ -803,7 +800,8 @@ hipError_t bindex_load(BinDex *bx, const char *path, const CODE *col) {
     goto done;
   if (host_digest(d) != h.dg_host || !host_arrays_valid(d, h.nblocks)) goto done;
   fv_words = (size_t)(d->bins - 1) * h.fv_stride;
-  e = hipHostMalloc(&stage, kStage, hipHostMallocDefault);
+  e = hipGetDevice(&d->device);
+  if (e == hipSuccess) e = hipHostMalloc(&stage, kStage, hipHostMallocDefault);
   if (e == hipSuccess) e = pool_alloc(&d->sorted_val, h.n * sizeof(CODE));
   if (e == hipSuccess) e = pool_alloc(&d->sorted_pos, h.n * sizeof(int32_t));
   if (e == hipSuccess) e = pool_alloc(&d->fvs, fv_words * sizeof(BITS));

@@ -6,8 +6,8 @@
 // (~30k per column at 1e8 rows).  Here everything stays on the device: one stable radix
 // sort of (value, row), a K-thread kernel for the area starts and one for the bin starts
 // (each area cut into `sub` equal-count bins), one pass over the column for all bins-1
-// filter vectors and the bin keys, one stable radix sort of the bin keys for the
-// row-ordered B lists, and a directory kernel.
+// filter vectors and the bin keys, and one stable partition of the rows by bin key for the
+// row-ordered B lists and their tile directory.
 #include <hipcub/hipcub.hpp>
 
 #include <stdio.h>
@@ -162,28 +162,156 @@ __global__ __launch_bounds__(kBlock) void k_build_fvs(const CODE *col, int64_t n
   }
 }
 
-// B-list entries: (row, value of the row).
-__global__ void k_gather_entries(const CODE *col, const uint32_t *pos, uint2 *ent, int64_t m) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t p = pos[i];
-    ent[i] = make_uint2(p, col[p]);
+// B lists by one stable partition of the rows by list key, with no sort and no gather: rows
+// per (bin, directory tile) -> one exclusive scan over bins and tiles, which is the tile
+// directory -> every tile's entries written where the directory says.  (Sorting 16-bit keys
+// with their rows and gathering the values afterwards, a random 4-byte read a row, took 2.7
+// ms at 1e8 rows and 128 bins; this takes 0.5.)
+
+// counts[k * (ntiles + 1) + t] = rows of tile t with key k (k < bins), and 0 for t = ntiles.
+// One workgroup per tile, and one for the zeros; LDS adds, a count copy per wave.
+__global__ __launch_bounds__(kBlock) void k_list_counts(const uint16_t *keys, int64_t n, int bins, int64_t ntiles,
+                                                        uint32_t *counts) {
+  extern __shared__ uint32_t cnt[];  // kBlock / kWave copies of bins + 1
+  const int64_t t = blockIdx.x;
+  const int copies = kBlock / kWave, per = bins + 1;
+  for (int i = threadIdx.x; i < copies * per; i += kBlock) cnt[i] = 0;
+  __syncthreads();
+  uint32_t *mine = cnt + threadIdx.x / kWave * per;
+  const int64_t r0 = t * kTileRows, r1 = std::min<int64_t>(n, r0 + kTileRows);
+  if (r0 + kTileRows <= n) {
+    const uint4 *src = reinterpret_cast<const uint4 *>(keys + r0);  // 8 keys each
+#pragma unroll 4
+    for (int i = threadIdx.x; i < kTileRows / 8; i += kBlock) {
+      const uint4 v = src[i];
+      for (const uint32_t w : {v.x, v.y, v.z, v.w}) {
+        if ((int)(w & 0xFFFF) < bins) atomicAdd(&mine[w & 0xFFFF], 1u);
+        if ((int)(w >> 16) < bins) atomicAdd(&mine[w >> 16], 1u);
+      }
+    }
+  } else {
+    for (int64_t r = r0 + threadIdx.x; r < r1; r += kBlock)
+      if (keys[r] < bins) atomicAdd(&mine[keys[r]], 1u);
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < bins; k += kBlock) {
+    uint32_t c = 0;
+    for (int w = 0; w < copies; w++) c += cnt[w * per + k];
+    counts[k * (ntiles + 1) + t] = c;
   }
 }
 
-// boff[k] = first sorted key >= k, for k in [0, bins]
-__global__ void k_bin_offsets(const uint16_t *skeys, int64_t n, int bins, uint32_t *boff) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k > bins) return;
-  int64_t lo = 0, hi = n;
-  while (lo < hi) {
-    const int64_t mid = lo + (hi - lo) / 2;
-    if ((int)skeys[mid] < k)
-      lo = mid + 1;
-    else
-      hi = mid;
+// The entries (row, value) of `parts`-th parts of the directory tiles: workgroup -> part j of
+// tile t, in chunks of kPartRows rows.  In a chunk each wave takes kPartRows / waves rows, 64
+// a step: a row's place among its wave's rows of the same key is the count so far (LDS, one
+// counter per key and wave) plus the lanes before it with the same key (NB ballots, one per
+// key bit).  The chunk is then laid out by key in LDS and written out in that order, so that
+// a bin's entries go to memory as one run (kPartRows / bins entries of 8 bytes) and in row
+// order.  parts > 1 (short columns, to fill the device) count the keys of the tile's rows
+// before theirs first.
+constexpr int kPartRows = 4096;
+constexpr int kPartRowBits = 12;
+template <int NB>
+__global__ __launch_bounds__(kBlock) void k_list_entries(const CODE *col, const uint16_t *keys, int64_t n, int bins,
+                                                         int64_t ntiles, const uint32_t *bdir, int parts, uint2 *bent) {
+  constexpr int kWaves = kBlock / kWave, kSteps = kPartRows / kBlock, kPer = (1 << (NB - 1)) / kBlock + 1;
+  extern __shared__ uint2 part_lds[];
+  uint2 *const stage = part_lds;                                           // kPartRows entries
+  uint32_t *const wcnt = reinterpret_cast<uint32_t *>(stage + kPartRows);  // per wave: bins + 1
+  uint32_t *const next = wcnt + kWaves * (bins + 1);                       // bins: the bin's next entry
+  uint32_t *const delta = next + bins;                                     // bins: entry - slot of the chunk
+  __shared__ uint32_t wsum[kWaves];
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  const int64_t t = blockIdx.x / parts;
+  const int j = blockIdx.x % parts;
+  for (int k = threadIdx.x; k < bins; k += kBlock) next[k] = bdir[k * (ntiles + 1) + t];
+  const int64_t tile0 = t * kTileRows, part = kTileRows / parts;
+  const int64_t p0 = tile0 + j * part, p1 = std::min<int64_t>(n, p0 + part);
+  __syncthreads();
+  for (int64_t r = tile0 + threadIdx.x; r < std::min<int64_t>(p0, n); r += kBlock) {
+    const uint32_t k = keys[r];
+    if ((int)k < bins) atomicAdd(&next[k], 1u);
   }
-  boff[k] = (uint32_t)lo;
+  for (int64_t c0 = p0; c0 < p1; c0 += kPartRows) {
+    uint32_t key[kSteps], place[kSteps];
+    CODE x[kSteps];
+    const uint32_t left = (uint32_t)std::min<int64_t>(kPartRows, p1 - c0);
+    const uint32_t w0 = wv * (kPartRows / kWaves) + lane;
+#pragma unroll
+    for (int i = 0; i < kSteps; i++) {
+      const uint32_t r = w0 + i * kWave;
+      key[i] = r < left ? keys[c0 + r] : (uint32_t)bins;
+      x[i] = r < left ? col[c0 + r] : 0;
+    }
+    for (int i = threadIdx.x; i < kWaves * (bins + 1); i += kBlock) wcnt[i] = 0;
+    __syncthreads();  // also: the chunk before has been written out, the counts above are done
+    uint32_t *const mine = wcnt + wv * (bins + 1);
+#pragma unroll
+    for (int i = 0; i < kSteps; i++) {
+      uint64_t same = ~0ull;
+#pragma unroll
+      for (int b = 0; b < NB; b++) {
+        const bool bit = (key[i] >> b) & 1;
+        const uint64_t with = __ballot(bit);
+        same &= bit ? with : ~with;
+      }
+      const uint32_t before = __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0));
+      place[i] = mine[key[i]] + before;
+      // the wave's LDS accesses run in order: this step's reads, then the first lane's add
+      if (before == 0) atomicAdd(&mine[key[i]], (uint32_t)__popcll(same));
+    }
+    __syncthreads();
+    // slots of the chunk: bins in order, a bin's waves in order (kPer bins a thread)
+    uint32_t total[kPer], sum = 0;
+    const int k0 = threadIdx.x * kPer;
+#pragma unroll
+    for (int q = 0; q < kPer; q++) {
+      total[q] = 0;
+      if (k0 + q < bins)
+        for (int w = 0; w < kWaves; w++) total[q] += wcnt[w * (bins + 1) + k0 + q];
+      sum += total[q];
+    }
+    uint32_t upto = sum;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const uint32_t u = __shfl_up(upto, o, kWave);
+      if (lane >= o) upto += u;
+    }
+    if (lane == kWave - 1) wsum[wv] = upto;
+    __syncthreads();
+    uint32_t slot = upto - sum, entries = 0;
+    for (int w = 0; w < kWaves; w++) {
+      if (w < wv) slot += wsum[w];
+      entries += wsum[w];
+    }
+#pragma unroll
+    for (int q = 0; q < kPer; q++) {
+      if (k0 + q < bins) {
+        delta[k0 + q] = next[k0 + q] - slot;
+        next[k0 + q] += total[q];
+        for (int w = 0; w < kWaves; w++) {
+          const uint32_t c = wcnt[w * (bins + 1) + k0 + q];
+          wcnt[w * (bins + 1) + k0 + q] = slot;
+          slot += c;
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kSteps; i++)
+      if ((int)key[i] < bins) stage[mine[key[i]] + place[i]] = make_uint2(key[i] << kPartRowBits | (w0 + i * kWave), x[i]);
+    __syncthreads();
+    for (uint32_t e = threadIdx.x; e < entries; e += kBlock) {
+      const uint2 v = stage[e];
+      bent[delta[v.x >> kPartRowBits] + e] = make_uint2((uint32_t)c0 + (v.x & (kPartRows - 1)), v.y);
+    }
+  }
+}
+
+// boff[k] = the directory's first entry of bin k, for k in [0, bins] (its rows end at the next bin's).
+__global__ void k_bin_offsets(const uint32_t *bdir, int64_t ntiles, int bins, uint32_t *boff) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k <= bins) boff[k] = k < bins ? bdir[k * (ntiles + 1)] : bdir[bins * (ntiles + 1) - 1];
 }
 
 // bdir[k * (ntiles + 1) + t] = first entry of bin k with row >= t * tile_rows
@@ -407,8 +535,8 @@ hipError_t bindex_host_blocks(BinDex *bx) {
 hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int sub, hipStream_t s) {
   hipError_t err = hipSuccess;
   rts_bindex_dev *d = nullptr;
-  uint32_t *iota = nullptr, *bpos_in = nullptr;
-  uint16_t *keys = nullptr, *skeys = nullptr;
+  uint32_t *iota = nullptr, *counts = nullptr;
+  uint16_t *keys = nullptr;
   void *tmp = nullptr;
   size_t tmp_bytes = 0, need = 0;
   CODE *starts_d = nullptr, *estarts_d = nullptr;
@@ -418,7 +546,7 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   int64_t nblocks = 0;
   int64_t idx_h[kAreas];
   uint32_t nb = 0;
-  int bins = 0, key_bits = 0;
+  int bins = 0;
   std::vector<int64_t> rk;
   uint8_t light_h[kMaxBins];
   uint8_t *light_d = nullptr;
@@ -435,7 +563,6 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   d->owned_column = owned;
   d->sub = sub;
   d->bins = bins = kAreas * sub;
-  while ((1 << key_bits) <= bins) key_bits++;  // keys 0..bins
 
   // 1. stable sort of (value, row)
   RTS_TRY(pool_alloc(&d->sorted_val, n * sizeof(CODE)));
@@ -491,23 +618,28 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   }
   RTS_TRY(hipGetLastError());
 
-  // 4. B lists: stable sort of (key, row) -> rows grouped by bin in row order
-  RTS_TRY(pool_alloc(&skeys, n * sizeof(uint16_t)));
-  RTS_TRY(pool_alloc(&bpos_in, n * sizeof(uint32_t)));
-  RTS_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, need, keys, skeys, iota, bpos_in, (int)n, 0,
-                                             key_bits, s));
-  if (need > tmp_bytes) {
-    RTS_TRY(hipStreamSynchronize(s));
-    pool_free(tmp, true);
-    tmp = nullptr;
-    tmp_bytes = need;
-    RTS_TRY(pool_alloc(&tmp, tmp_bytes));
+  // 4. tile directory and B lists
+  {
+    const int64_t items = (int64_t)bins * (d->ntiles + 1);
+    RTS_TRY(pool_alloc(&d->bdir, items * sizeof(uint32_t)));
+    RTS_TRY(pool_alloc(&counts, items * sizeof(uint32_t)));
+    RTS_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, need, counts, d->bdir, items, s));
+    if (need > tmp_bytes) {
+      RTS_TRY(hipStreamSynchronize(s));
+      pool_free(tmp, true);
+      tmp = nullptr;
+      tmp_bytes = need;
+      RTS_TRY(pool_alloc(&tmp, tmp_bytes));
+    }
+    hipLaunchKernelGGL(k_list_counts, dim3((unsigned)(d->ntiles + 1)), dim3(kBlock),
+                       kBlock / kWave * (bins + 1) * sizeof(uint32_t), s, keys, n, bins, d->ntiles, counts);
+    RTS_TRY(hipGetLastError());
+    RTS_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, need, counts, d->bdir, items, s));
+    RTS_TRY(pool_alloc(&d->boff, (bins + 1) * sizeof(uint32_t)));
+    hipLaunchKernelGGL(k_bin_offsets, dim3((bins + 1 + kBlock - 1) / kBlock), dim3(kBlock), 0, s, d->bdir, d->ntiles,
+                       bins, d->boff);
+    RTS_TRY(hipGetLastError());
   }
-  RTS_TRY(hipcub::DeviceRadixSort::SortPairs(tmp, need, keys, skeys, iota, bpos_in, (int)n, 0, key_bits, s));
-  RTS_TRY(pool_alloc(&d->boff, (bins + 1) * sizeof(uint32_t)));
-  hipLaunchKernelGGL(k_bin_offsets, dim3((bins + 1 + kBlock - 1) / kBlock), dim3(kBlock), 0, s, skeys, n, bins,
-                     d->boff);
-  RTS_TRY(hipGetLastError());
   d->boff_host.resize(bins + 1);
   RTS_TRY(hipMemcpyAsync(d->boff_host.data(), d->boff, (bins + 1) * sizeof(uint32_t),
                          hipMemcpyDeviceToHost, s));
@@ -517,12 +649,21 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   mark_complete_bins(d, rk);
   RTS_TRY(pool_alloc(&d->bent, std::max<uint32_t>(nb, 1) * sizeof(uint2)));
   if (nb) {
-    hipLaunchKernelGGL(k_gather_entries, dim3(blocks_for(nb)), dim3(kBlock), 0, s, col, bpos_in,
-                       d->bent, (int64_t)nb);
+    // a workgroup a tile when that fills the device, else the tiles in up to 8 parts
+    int parts = 1;
+    while (parts < kTileRows / kPartRows && d->ntiles * parts < 4 * (int64_t)device_cu_count()) parts *= 2;
+    const dim3 grid((unsigned)(d->ntiles * parts));
+    const size_t lds = kPartRows * sizeof(uint2) + (kBlock / kWave * (bins + 1) + 2 * bins) * sizeof(uint32_t);
+#define RTS_LIST_ENTRIES(NB)                                                                             \
+  hipLaunchKernelGGL(k_list_entries<NB>, grid, dim3(kBlock), lds, s, col, keys, n, bins, d->ntiles, d->bdir, \
+                     parts, d->bent)
+    if (bins <= 128) RTS_LIST_ENTRIES(8);
+    else if (bins <= 256) RTS_LIST_ENTRIES(9);
+    else if (bins <= 512) RTS_LIST_ENTRIES(10);
+    else RTS_LIST_ENTRIES(11);
+#undef RTS_LIST_ENTRIES
     RTS_TRY(hipGetLastError());
   }
-  RTS_TRY(pool_alloc(&d->bdir, (size_t)bins * (d->ntiles + 1) * sizeof(uint32_t)));
-  RTS_TRY(launch_tile_directory(d, d->ntiles, kTileRows, d->bdir, s));
 
   // 5. host descriptor: areas (bindex.cpp:633-652) and their blocks
   for (int k = 0; k < kAreas; k++) {
@@ -563,7 +704,7 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
 fail:
   {
     const bool idle = hipStreamSynchronize(s) == hipSuccess;  // before other calls get the workspaces
-    for (void *p : {(void *)iota, (void *)bpos_in, (void *)keys, (void *)skeys, tmp, (void *)starts_d,
+    for (void *p : {(void *)iota, (void *)counts, (void *)keys, tmp, (void *)starts_d,
                     (void *)estarts_d, (void *)light_d, (void *)idx_d, (void *)bf_slot_d, (void *)bl_slot_d,
                     (void *)bfirst_d, (void *)blast_d})
       pool_free(p, idle);

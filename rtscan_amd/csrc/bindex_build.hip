@@ -17,14 +17,9 @@
 #include <mutex>
 
 #include "bindex_dev.h"
+#include "sort_rows.h"
 
 namespace rts {
-
-__global__ void k_iota(uint32_t *p, int64_t n) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = (uint32_t)i;
-}
 
 // Area starts (bindex.cpp:613-631): start[i] = sorted[i * avg]; if it equals the previous
 // start the area begins mid-run at i * avg, otherwise at the first occurrence of the value.
@@ -535,10 +530,10 @@ hipError_t bindex_host_blocks(BinDex *bx) {
 hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int sub, hipStream_t s) {
   hipError_t err = hipSuccess;
   rts_bindex_dev *d = nullptr;
-  uint32_t *iota = nullptr, *counts = nullptr;
+  uint32_t *counts = nullptr;
   uint16_t *keys = nullptr;
-  void *tmp = nullptr;
-  size_t tmp_bytes = 0, need = 0;
+  void *sort_tmp = nullptr, *tmp = nullptr;
+  size_t need = 0;
   CODE *starts_d = nullptr, *estarts_d = nullptr;
   int64_t *idx_d = nullptr, *bf_slot_d = nullptr, *bl_slot_d = nullptr;
   CODE *bfirst_d = nullptr, *blast_d = nullptr;
@@ -567,15 +562,8 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   // 1. stable sort of (value, row)
   RTS_TRY(pool_alloc(&d->sorted_val, n * sizeof(CODE)));
   RTS_TRY(pool_alloc(&d->sorted_pos, n * sizeof(int32_t)));
-  RTS_TRY(pool_alloc(&iota, n * sizeof(uint32_t)));
-  hipLaunchKernelGGL(k_iota, dim3(blocks_for(n)), dim3(kBlock), 0, s, iota, n);
-  RTS_TRY(hipGetLastError());
-  RTS_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, need, col, d->sorted_val, iota,
-                                             (uint32_t *)d->sorted_pos, (int)n, 0, 32, s));
-  tmp_bytes = need;
-  RTS_TRY(pool_alloc(&tmp, tmp_bytes));
-  RTS_TRY(hipcub::DeviceRadixSort::SortPairs(tmp, need, col, d->sorted_val, iota,
-                                             (uint32_t *)d->sorted_pos, (int)n, 0, 32, s));
+  RTS_TRY(pool_alloc(&sort_tmp, sort_rows_workspace(n)));
+  RTS_TRY(sort_rows(col, n, d->sorted_val, (uint32_t *)d->sorted_pos, sort_tmp, s));
 
   // 2. area starts, then bin starts
   RTS_TRY(pool_alloc(&starts_d, kAreas * sizeof(CODE)));
@@ -624,13 +612,7 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
     RTS_TRY(pool_alloc(&d->bdir, items * sizeof(uint32_t)));
     RTS_TRY(pool_alloc(&counts, items * sizeof(uint32_t)));
     RTS_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, need, counts, d->bdir, items, s));
-    if (need > tmp_bytes) {
-      RTS_TRY(hipStreamSynchronize(s));
-      pool_free(tmp, true);
-      tmp = nullptr;
-      tmp_bytes = need;
-      RTS_TRY(pool_alloc(&tmp, tmp_bytes));
-    }
+    RTS_TRY(pool_alloc(&tmp, need));
     hipLaunchKernelGGL(k_list_counts, dim3((unsigned)(d->ntiles + 1)), dim3(kBlock),
                        kBlock / kWave * (bins + 1) * sizeof(uint32_t), s, keys, n, bins, d->ntiles, counts);
     RTS_TRY(hipGetLastError());
@@ -704,7 +686,7 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
 fail:
   {
     const bool idle = hipStreamSynchronize(s) == hipSuccess;  // before other calls get the workspaces
-    for (void *p : {(void *)iota, (void *)counts, (void *)keys, tmp, (void *)starts_d,
+    for (void *p : {sort_tmp, (void *)counts, (void *)keys, tmp, (void *)starts_d,
                     (void *)estarts_d, (void *)light_d, (void *)idx_d, (void *)bf_slot_d, (void *)bl_slot_d,
                     (void *)bfirst_d, (void *)blast_d})
       pool_free(p, idle);

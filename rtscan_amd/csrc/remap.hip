@@ -24,6 +24,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "sort_rows.h"
 #define RTS_REMAP_NO_CXX
 #include "rts_remap.h"
 
@@ -33,11 +34,6 @@ namespace {
 constexpr int kRemapBlock = 256;
 
 unsigned grid_for(int64_t items) { return (unsigned)((items + kRemapBlock - 1) / kRemapBlock); }
-
-__global__ void k_remap_iota(uint32_t *p, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = (uint32_t)i;
-}
 
 __device__ __forceinline__ uint32_t row_hash(uint64_t seed, uint32_t row) {
   uint64_t z = seed + 0x9E3779B97F4A7C15ull * ((uint64_t)row + 1);
@@ -347,9 +343,9 @@ struct Runs {
 
 hipError_t sorted_runs(const CODE *data, int64_t n, POSTYPE *caller_spos, Runs &R, hipStream_t s) {
   hipError_t err = hipSuccess;
-  uint32_t *iota = nullptr, *heads = nullptr;
-  void *tmp = nullptr;
-  size_t need = 0, have = 0;
+  uint32_t *heads = nullptr;
+  void *sort_tmp = nullptr, *tmp = nullptr;
+  size_t need = 0;
   uint32_t last = 0;
 
   R.tiles = (n + kRunTile - 1) / kRunTile;
@@ -362,26 +358,19 @@ hipError_t sorted_runs(const CODE *data, int64_t n, POSTYPE *caller_spos, Runs &
   }
   RTS_TRY(pool_alloc(&heads, (R.tiles + 1) * sizeof(uint32_t)));
   RTS_TRY(pool_alloc(&R.base, (R.tiles + 1) * sizeof(uint32_t)));
-  RTS_TRY(pool_alloc(&iota, n * sizeof(uint32_t)));
-  hipLaunchKernelGGL(k_remap_iota, dim3(grid_for(n)), dim3(kRemapBlock), 0, s, iota, n);
-  RTS_TRY(hipGetLastError());
-  RTS_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, need, data, R.sval, iota, R.spos, (int)n, 0, 32, s));
-  have = need;
+  RTS_TRY(pool_alloc(&sort_tmp, sort_rows_workspace(n)));
   RTS_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, need, heads, R.base, (int)R.tiles + 1, s));
-  have = need > have ? need : have;
-  RTS_TRY(pool_alloc(&tmp, have));
-  need = have;
-  RTS_TRY(hipcub::DeviceRadixSort::SortPairs(tmp, need, data, R.sval, iota, R.spos, (int)n, 0, 32, s));
+  RTS_TRY(pool_alloc(&tmp, need));
+  RTS_TRY(sort_rows(data, n, R.sval, R.spos, sort_tmp, s));
   hipLaunchKernelGGL(k_run_heads, dim3((unsigned)R.tiles), dim3(kRunThreads), 0, s, R.sval, n, R.tiles, heads);
   RTS_TRY(hipGetLastError());
-  need = have;
   RTS_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, need, heads, R.base, (int)R.tiles + 1, s));
   RTS_TRY(hipMemcpyAsync(&last, R.base + R.tiles, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   RTS_TRY(hipStreamSynchronize(s));
   R.m = last;
 
 fail:
-  pool_free(iota, err == hipSuccess);
+  pool_free(sort_tmp, err == hipSuccess);
   pool_free(heads, err == hipSuccess);
   pool_free(tmp, err == hipSuccess);
   return err;

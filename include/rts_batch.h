@@ -6,15 +6,26 @@
  * columns all have n rows.  Each query-column is evaluated from the column's BinDex (filter
  * vectors + boundary-bin refine lists) or directly from its values; for RTS_EVAL_AUTO the
  * planner's cost model chooses (the bytes per row each form reads, the direct form weighted
- * by the config's direct_weight; a column without an index is evaluated directly).  Query q's bitmap is written at out + q * out_stride_words
- * (MSB-first words, bits past row n cleared) and its popcount at counts[q] (device).
+ * by the config's direct_weight; a column without an index is evaluated directly).  Query q's
+ * bitmap is written at out + q * out_stride_words (MSB-first words, bits past row n cleared)
+ * and its popcount at counts[q] (device).
+ *
+ * Eight queries or more, none of whose columns is RTS_EVAL_BINDEX, may be evaluated together
+ * instead where the planner expects that to take less time: each row's values are looked up
+ * among the queries' bounds once for up to 256 queries.  The results are the same.  Columns
+ * are then read from the plan's column pointers (RTS_EVAL_DIRECT, or no index) and, for an
+ * indexed column, from the column that its index refers to (BinDex::rawDataInGPU, which
+ * outlives the index); a column that is not 16-byte aligned, or an index loaded without its
+ * column, keeps its queries out.  Of the launch shape below it depends on nothing, and the
+ * planner statistics count a query's columns as their own forms.
  *
  * The launch is one persistent kernel over (row tile, query group) work items, handed out by
- * per-XCD counters so that one tile's work items run on one XCD back to back, plus one small
- * kernel summing the per-(query, tile) popcounts.  Launches of one plan must not overlap
- * (use one stream per plan, or order them): they share the plan's counters and partials.  rts_batch_plan_graph_launch captures both in a hipGraph and
- * replays it; queries set with rts_batch_plan_set_queries live in device memory at a fixed
- * address, so a replay evaluates the current set.
+ * per-XCD counters so that one tile's work items run on one XCD back to back (and another for
+ * the queries that are evaluated together), plus one small kernel summing the popcounts.
+ * Launches of one plan must not overlap (use one stream per plan, or order them): they share
+ * the plan's counters and partials.  rts_batch_plan_graph_launch captures them in a hipGraph
+ * and replays it; queries set with rts_batch_plan_set_queries live in device memory at a fixed
+ * address, so a replay, of a graph of the caller's own too, evaluates the current set.
  */
 #ifndef RTS_BATCH_H_
 #define RTS_BATCH_H_
@@ -54,7 +65,8 @@ typedef struct rts_batch_config {
                    created with; see rts_batch_plan_add_indexes) */
   int direct_weight; /* cost of evaluating an RTS_EVAL_AUTO query-column directly, per mille
                         of its column's 4 bytes per row, against the BinDex form's filter-
-                        vector and list bytes per row; 0: never direct when indexed */
+                        vector and list bytes per row; 0: an indexed column is never
+                        evaluated directly by itself */
 } rts_batch_config;
 
 typedef struct rts_batch_plan rts_batch_plan;
@@ -90,7 +102,8 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *plan, const rts_query_
 hipError_t rts_batch_plan_launch(rts_batch_plan *plan, BITS *out, int64_t out_stride_words,
                                  unsigned long long *counts, hipStream_t stream);
 /* As rts_batch_plan_launch through a captured hipGraph (captured on first use and again
- * when out / counts / stride / query count change).  stream must not be the null stream. */
+ * when out / counts / stride / query count or the kernels that the queries need change).
+ * stream must not be the null stream. */
 hipError_t rts_batch_plan_graph_launch(rts_batch_plan *plan, BITS *out, int64_t out_stride_words,
                                        unsigned long long *counts, hipStream_t stream);
 /* Planner statistics of the current queries: query-columns on the BinDex path, on the direct

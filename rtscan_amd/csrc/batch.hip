@@ -5,7 +5,8 @@
 // (two filter vectors and the tile slices of up to two bins' refine lists, as in
 // k_bindex_query; or, for a range over one or two bins whose lists hold all their rows,
 // those lists alone) or directly from the column's values (the wave64 DPP word assembly
-// of k_scan_tiles).
+// of k_scan_tiles).  Queries that are cheaper evaluated together from the columns' values go
+// to k_batch_ranked instead (batch_rank.hip).
 //
 // Work item = (row tile t, query group g): the workgroup writes the tile's output words of
 // every query of the group.  The items of one tile run on the same XCD one after another
@@ -36,7 +37,9 @@
 #include <vector>
 
 #include "batch.h"
+#include "batch_rank.h"
 #include "bindex_dev.h"
+#include "device_ptr.h"
 
 namespace rts {
 
@@ -114,29 +117,7 @@ struct BatchLds {
 
 constexpr int ilog2(int v) { return v <= 1 ? 0 : 1 + ilog2(v / 2); }
 
-// Device memory reached through pointers read from the group records (columns, filter
-// vectors, list entries and directories, result bitmaps) is global memory.  Saying so turns
-// the generic (flat) accesses the compiler would emit for such pointers into global ones:
-// flat accesses also count against the LDS wait counter, so every LDS wait in the kernel
-// would wait for outstanding loads and result stores as well.
-#define RTS_GLOBAL __attribute__((address_space(1)))
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-template <class T>
-__device__ __forceinline__ const RTS_GLOBAL T *gmem(const T *p) {
-  return (const RTS_GLOBAL T *)p;
-}
-template <class T>
-__device__ __forceinline__ RTS_GLOBAL T *gmem(T *p) {
-  return (RTS_GLOBAL T *)p;
-}
-// Memory that no kernel writes while a batch runs (the lists' tile directories), read
-// through the constant address space: a wave-uniform address then becomes a scalar load,
-// whose wait does not also wait for the wave's outstanding result stores.
-#define RTS_CONST __attribute__((address_space(4)))
-template <class T>
-__device__ __forceinline__ const RTS_CONST T *cmem(const T *p) {
-  return (const RTS_CONST T *)p;
-}
 
 // Toggle layout: thread t owns tile words t * kPer .. t * kPer + kPer - 1 (kPer = TW / NT)
 // as kPer / U units of U words (U = 2 when kPer >= 2: 64-bit LDS accesses), stored
@@ -269,21 +250,6 @@ __device__ __forceinline__ Words<KP> base_words(const BITS *fv_any, uint32_t bas
     for (int k = 0; k < KP; k++) r.v[k] = w + k < words ? fv[w + k] : 0u;
   }
   return r;
-}
-
-
-// A value that is the same in every lane, moved to a scalar register (the builtin takes and
-// returns 32-bit values: a pointer goes one half at a time).
-__device__ __forceinline__ uint32_t uniform_u32(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
-}
-__device__ __forceinline__ uint64_t uniform_u64(uint64_t v) {
-  return ((uint64_t)uniform_u32((uint32_t)(v >> 32)) << 32) | uniform_u32((uint32_t)v);
-}
-template <class T>
-__device__ __forceinline__ T *uniform_ptr(T *p) {
-  const uint64_t a = (uint64_t)p;
-  return (T *)(((uint64_t)uniform_u32((uint32_t)(a >> 32)) << 32) | uniform_u32((uint32_t)a));
 }
 
 // Result words are written once and not read again by the launch: non-temporal stores keep
@@ -621,6 +587,34 @@ __global__ __launch_bounds__(kBlock) void k_batch_counts(const uint32_t *partial
   }
 }
 
+// The same where queries may be evaluated together (`ranked`, per query): those have their sum
+// in rank_counts, which is left at zero for the next launch.
+__global__ __launch_bounds__(kBlock) void k_batch_counts_mixed(const uint32_t *partials, int64_t ntiles,
+                                                               const uint8_t *ranked,
+                                                               unsigned long long *rank_counts,
+                                                               unsigned long long *counts) {
+  __shared__ unsigned long long part[kBlock / kWave];
+  unsigned long long s = 0;
+  if (ranked[blockIdx.x]) {
+    if (threadIdx.x == 0) {
+      s = rank_counts[blockIdx.x];
+      rank_counts[blockIdx.x] = 0;
+    }
+  } else {
+    const uint32_t *p = partials + (int64_t)blockIdx.x * ntiles;
+    for (int64_t i = threadIdx.x; i < ntiles; i += kBlock) s += p[i];
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, kWave);
+  if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x / kWave] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long t = 0;
+    for (int i = 0; i < kBlock / kWave; i++) t += part[i];
+    counts[blockIdx.x] = t;
+  }
+}
+
 // Planned form of one query-column before grouping.
 struct PlannedBound {
   uint32_t base = kBaseZero;
@@ -695,9 +689,16 @@ struct rts_batch_plan {
   rts_batch_config cfg{};
   int64_t ntiles = 0;
   BatchGroup *d_groups = nullptr;  // max_queries records
-  int *d_ngroups = nullptr;        // device copy of ngroups
+  // One block of device memory, uploaded in one copy as far as a set of queries fills it:
+  // the header, per query a byte that says whether it is evaluated together with others
+  // (k_batch_ranked), the groups of those; then their counts (zero between launches).
+  uint8_t *d_plan = nullptr;
+  std::vector<uint8_t> h_plan;
+  size_t rank_groups_at = 0, rank_counts_at = 0;
+  int max_rank_groups = 0;
+  bool has_ranked = false, has_bindex = false;  // the forms that the current queries need
   uint32_t *d_zero_dir = nullptr;  // ntiles + 1 zeros: the directory of an unused list
-  int ngroups = 0;
+  int ngroups = 0;  // of k_batch
   uint32_t *d_partials = nullptr;
   unsigned long long *d_sched = nullptr;  // per-XCD work-item counters + finished workgroups
   std::vector<BatchGroup> h_groups;
@@ -709,6 +710,7 @@ struct rts_batch_plan {
   unsigned long long *graph_counts = nullptr;
   int graph_nq = -1;
   int64_t graph_stride = 0;
+  int graph_forms = 0;
   int stats_bindex_cols = 0, stats_direct_cols = 0, stats_narrow_cols = 0, stats_auto_direct = 0;
   int stats_list_cols = 0;
   std::vector<rts_query_spec> specs;  // the current queries, re-planned on a new tiling
@@ -803,28 +805,125 @@ static void launch_k_batch(rts_batch_plan *p, BITS *out, int64_t out_stride, hip
   // work items to a second round: clamp to the occupancy limit
   unsigned grid = (unsigned)(cus * std::min(p->cfg.blocks_per_cu, batch_resident_per_cu<TW, NT>()));
   grid = std::max<unsigned>(kXcds, grid / kXcds * kXcds);
-  hipLaunchKernelGGL((k_batch<TW, NT>), dim3(grid), dim3(NT), 0, s, p->d_groups, p->d_ngroups, p->n,
+  hipLaunchKernelGGL((k_batch<TW, NT>), dim3(grid), dim3(NT), 0, s, p->d_groups,
+                     &reinterpret_cast<const RankHeader *>(p->d_plan)->bindex_groups, p->n,
                      p->words, p->ntiles, out, out_stride, p->d_partials, p->d_sched);
 }
 
-static hipError_t launch_batch(rts_batch_plan *p, BITS *out, int64_t out_stride,
-                               unsigned long long *counts, hipStream_t s) {
-  const bool small = p->cfg.threads == 256;
-  switch (p->cfg.tile_words) {
-    case 2048:
-      small ? launch_k_batch<2048, 256>(p, out, out_stride, s) : launch_k_batch<2048, 512>(p, out, out_stride, s);
-      break;
-    case 1024:
-      small ? launch_k_batch<1024, 256>(p, out, out_stride, s) : launch_k_batch<1024, 512>(p, out, out_stride, s);
-      break;
-    default:
-      small ? launch_k_batch<512, 256>(p, out, out_stride, s) : launch_k_batch<512, 512>(p, out, out_stride, s);
+// The forms of evaluation a launch runs.
+enum : int { kFormBindex = 1, kFormRanked = 2 };
+
+static int forms_needed(const rts_batch_plan *p) {
+  return (p->has_bindex ? kFormBindex : 0) | (p->has_ranked ? kFormRanked : 0);
+}
+
+static hipError_t launch_batch(rts_batch_plan *p, BITS *out, int64_t out_stride, unsigned long long *counts, int forms,
+                               hipStream_t s) {
+  auto *const rank_counts = reinterpret_cast<unsigned long long *>(p->d_plan + p->rank_counts_at);
+  hipError_t e = hipSuccess;
+  if (forms & kFormRanked)
+    e = launch_rank_groups(reinterpret_cast<const RankGroup *>(p->d_plan + p->rank_groups_at),
+                           reinterpret_cast<const RankHeader *>(p->d_plan), p->n, out, out_stride,
+                           counts ? rank_counts : nullptr, s);
+  if (e == hipSuccess && (forms & kFormBindex)) {
+    const bool small = p->cfg.threads == 256;
+    switch (p->cfg.tile_words) {
+      case 2048:
+        small ? launch_k_batch<2048, 256>(p, out, out_stride, s) : launch_k_batch<2048, 512>(p, out, out_stride, s);
+        break;
+      case 1024:
+        small ? launch_k_batch<1024, 256>(p, out, out_stride, s) : launch_k_batch<1024, 512>(p, out, out_stride, s);
+        break;
+      default:
+        small ? launch_k_batch<512, 256>(p, out, out_stride, s) : launch_k_batch<512, 512>(p, out, out_stride, s);
+    }
+    e = hipGetLastError();
   }
-  hipError_t e = hipGetLastError();
   if (e != hipSuccess || !counts) return e;
-  hipLaunchKernelGGL(k_batch_counts, dim3((unsigned)p->nq), dim3(kBlock), 0, s, p->d_partials, p->ntiles,
-                     counts);
+  if (forms & kFormRanked)
+    hipLaunchKernelGGL(k_batch_counts_mixed, dim3((unsigned)p->nq), dim3(kBlock), 0, s, p->d_partials, p->ntiles,
+                       p->d_plan + sizeof(RankHeader), rank_counts, counts);
+  else
+    hipLaunchKernelGGL(k_batch_counts, dim3((unsigned)p->nq), dim3(kBlock), 0, s, p->d_partials, p->ntiles,
+                       counts);
   return hipGetLastError();
+}
+
+// Query-columns a work item has toggle arrays for.
+static int batch_slots(const rts_batch_config &c) { return kBatchLdsWords / 512 * c.threads / c.tile_words; }
+
+// First fit of queries with decreasing slot counts `need`: the group of each, and how many.
+static int pack_groups(const std::vector<int> &need, int slot_cap, int per_group, std::vector<int> *group_of) {
+  group_of->resize(need.size());
+  std::vector<int> free_slots, queries;
+  std::vector<std::set<int>> open(slot_cap + 1);  // groups with room, by free slots
+  for (size_t i = 0; i < need.size(); i++) {
+    int k = -1, kf = 0;
+    for (int f = std::max(need[i], 1); f <= slot_cap; f++)  // first fit: the earliest group with room
+      if (!open[f].empty() && (k < 0 || *open[f].begin() < k)) k = *open[f].begin(), kf = f;
+    if (k < 0) {
+      k = (int)free_slots.size();
+      free_slots.push_back(slot_cap);
+      queries.push_back(0);
+    } else {
+      open[kf].erase(k);
+    }
+    (*group_of)[i] = k;
+    free_slots[k] -= need[i];
+    if (++queries[k] < per_group && free_slots[k] > 0) open[free_slots[k]].insert(k);
+  }
+  return (int)free_slots.size();
+}
+
+// Time of k_batch in microseconds for nq queries whose columns take the forms pc: latency that
+// grows with the items up to a chain of them, the bitmaps, and of each query-column its share
+// of reads, where filter vectors that other queries have read cost less.  Measured (mixed
+// queries unless noted): 1e8 rows, 4 columns, 256 bins: 8 queries 145, 32 370, 64 650, 256
+// 2110, 1024 7170; one column and bin each: 64 373, 256 1175; 2e7 rows, 2 columns: 8 73, 32
+// 107, 64 144; 4.2e6 rows, 4 columns: 8 40, 32 78, 256 140; 1e6 rows: 8 30, 64 44.
+static double batch_us(const rts_batch_plan *p, const std::vector<RankQuery> &queries, const std::vector<int> &ncols,
+                       const std::vector<PlannedCol> &pc) {
+  std::vector<int> wide((size_t)p->ncols, 0);  // query-columns that read filter vectors
+  auto reads = [&](const PlannedCol &P) { return !P.direct && !P.narrow && P.list_b0 < 0; };
+  auto each = [&](auto f) {
+    for (const RankQuery &q : queries)
+      for (int c = 0; !q.empty && c < ncols[q.id]; c++) f(pc[(size_t)q.id * kBatchMaxCols + c]);
+  };
+  each([&](const PlannedCol &P) { wide[P.col] += reads(P); });
+  const double n = (double)p->n, nq = (double)queries.size();
+  double us = 2.7 * nq;
+  each([&](const PlannedCol &P) {
+    us += P.direct ? 20.0
+          : reads(P) ? 1.9 + 1.6 * std::min(1.0, p->index[P.col]->dev->bins / 2.0 / wide[P.col])
+                     : 1.1;
+  });
+  const double chain = std::max(std::min(40.0, n / 1e5), n / 1e6);
+  return 28 + chain * std::min(1.0, nq / 64 * std::max(1.0, n / 4e6)) + 0.08 * nq + us * n / 1e8;
+}
+
+// The query as plan_rank_groups takes it, its columns read where its forms would read or have
+// indexed them (an index's column must outlive the index).  False: it can't be evaluated
+// together with others.
+static bool rank_query(const rts_batch_plan *p, const rts_query_spec &in, RankQuery *R) {
+  for (int c = 0; c < in.ncols; c++) {
+    if (in.mode[c] == RTS_EVAL_BINDEX) return false;
+    const BinDex *b = p->index[in.column[c]];
+    const CODE *col = in.mode[c] == RTS_EVAL_DIRECT || !b ? p->columns[in.column[c]] : b->rawDataInGPU;
+    if (!col || ((uintptr_t)col & 15)) return false;
+    if (in.lo[c] > in.hi[c]) R->empty = true;
+    int k = 0;
+    while (k < R->ncols && R->col[k] != col) k++;
+    if (k == R->ncols) {
+      R->col[R->ncols++] = col;
+      R->lo[k] = in.lo[c];
+      R->hi[k] = in.hi[c];
+    } else {  // two ranges of one column
+      R->lo[k] = std::max(R->lo[k], in.lo[c]);
+      R->hi[k] = std::min(R->hi[k], in.hi[c]);
+      if (R->lo[k] > R->hi[k]) R->empty = true;
+    }
+  }
+  return true;
 }
 
 }  // namespace rts
@@ -869,7 +968,12 @@ hipError_t rts_batch_plan_create(rts_batch_plan **out, const CODE *const *column
   p->active_set = set_for(p, p->cfg);
   p->index = p->index_sets[p->active_set].data();
   hipError_t e = device_malloc((void **)&p->d_groups, (size_t)max_queries * sizeof(BatchGroup));
-  if (e == hipSuccess) e = device_malloc((void **)&p->d_ngroups, sizeof(int));
+  p->max_rank_groups = max_rank_groups(max_queries);
+  p->rank_groups_at = (sizeof(RankHeader) + (size_t)max_queries + 15) / 16 * 16;
+  p->rank_counts_at = p->rank_groups_at + (size_t)p->max_rank_groups * sizeof(RankGroup);
+  const size_t rank_counts = p->max_rank_groups ? (size_t)max_queries * sizeof(unsigned long long) : 0;
+  if (e == hipSuccess) e = device_malloc((void **)&p->d_plan, p->rank_counts_at + rank_counts);
+  if (e == hipSuccess && rank_counts) e = hipMemsetAsync(p->d_plan + p->rank_counts_at, 0, rank_counts, stream);
   if (e == hipSuccess) e = device_malloc((void **)&p->d_sched, kSchedWords * sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMemsetAsync(p->d_sched, 0, kSchedWords * sizeof(unsigned long long), stream);
   if (e == hipSuccess) e = build_dirs(p, stream);
@@ -955,7 +1059,7 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
     if (!outs[q] || ((uintptr_t)outs[q] & 15))
       return set_error(hipErrorInvalidValue, "rts_batch_plan_set_queries: outputs must be 16-byte aligned");
   // 1. every query-column in BinDex or direct form
-  p->stats_auto_direct = 0;
+  int st_auto = 0;
   std::vector<PlannedCol> pc((size_t)nq * kBatchMaxCols);
   std::vector<int> qcols(nq, 0), qempty(nq, 0);
   int st_bindex = 0, st_direct = 0, st_narrow = 0, st_list = 0;
@@ -984,7 +1088,7 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
         if (in.mode[c] == RTS_EVAL_AUTO && aligned && !list_form(b->dev, sl, sh, &b0, &b1) &&
             direct_cheaper(b->dev, sl, sh, p->cfg.direct_weight)) {
           direct = true;
-          p->stats_auto_direct++;
+          st_auto++;
         }
       }
       if (direct) {
@@ -1021,14 +1125,33 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
       st_bindex++;
     }
   }
-  // 2. the order queries are grouped in: the caller's, or sorted by the (column, lower and
+  // 2. the queries that are evaluated together, the rest each by its columns' forms
+  RankHeader header{};
+  header.own_outs = outs != nullptr;
+  std::vector<RankGroup> rank_groups;
+  std::vector<uint8_t> ranked((size_t)nq, 0);
+  if (p->max_rank_groups) {
+    std::vector<RankQuery> together;
+    together.reserve((size_t)nq);
+    for (int q = 0; q < nq; q++) {
+      RankQuery R;
+      if (!rank_query(p, queries[q], &R)) continue;
+      R.id = q;
+      R.own = outs ? outs[q] : nullptr;
+      together.push_back(R);
+    }
+    if (plan_rank_groups(together, p->n, p->max_rank_groups, batch_us(p, together, qcols, pc), rank_groups, &header))
+      for (const RankQuery &R : together) ranked[R.id] = 1;
+  }
+  // 3. the order the others are grouped in: the caller's, or sorted by the (column, lower and
   //    upper filter vector) of their BinDex columns taken in column order, so that the
   //    groups a tile's workgroups run together read few distinct filter vectors
-  std::vector<int> order(nq);
-  for (int q = 0; q < nq; q++) order[q] = q;
+  std::vector<int> order;
+  for (int q = 0; q < nq; q++)
+    if (!ranked[q]) order.push_back(q);
   if (p->cfg.order == 1) {
     std::vector<std::vector<int>> key(nq);
-    for (int q = 0; q < nq; q++) {
+    for (const int q : order) {
       std::vector<std::array<int, 3>> cols;
       for (int c = 0; c < qcols[q]; c++) {
         const PlannedCol &P = pc[(size_t)q * kBatchMaxCols + c];
@@ -1040,14 +1163,14 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
     }
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return key[a] < key[b]; });
   }
-  // 3. groups, each one self-contained record of queries whose slots fit the LDS of one
+  // 4. groups, each one self-contained record of queries whose slots fit the LDS of one
   //    tile, at most the configured group size.  Work items, and their fixed costs, scale
   //    with the group count, so groups are packed full: first fit by decreasing slot count
   //    (4 | 3 + 1 | 2 + 2 for four slots), each size class taken in that order, and the
   //    groups run in the order of their first query.  Partners are then paired in order
   //    too (the i-th 3-column query with the i-th 1-column one), so neighbouring groups
   //    still share filter vectors in the locality order.
-  const int slot_cap = kBatchLdsWords / 512 * p->cfg.threads / p->cfg.tile_words;
+  const int slot_cap = batch_slots(p->cfg);
   const int64_t per = p->ntiles + 1;
   auto add_query = [&](BatchGroup &g, int q) {
     const int need = qempty[q] ? 0 : qcols[q];
@@ -1102,32 +1225,23 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
     g.nq++;
     g.qslot[g.nq] = (uint8_t)g.nslots;
   };
-  std::vector<int> byneed(nq);  // positions in the order, by decreasing slot count
-  for (int i = 0; i < nq; i++) byneed[i] = i;
+  std::vector<int> byneed(order.size());  // positions in the order, by decreasing slot count
+  for (size_t i = 0; i < order.size(); i++) byneed[i] = (int)i;
   auto need_at = [&](int oi) { return qempty[order[oi]] ? 0 : qcols[order[oi]]; };
   std::stable_sort(byneed.begin(), byneed.end(), [&](int a, int b) { return need_at(a) > need_at(b); });
-  std::vector<BatchGroup> cg;
-  cg.reserve(nq);
-  std::vector<int> lead;                         // order position of each group's first query
-  std::vector<std::set<int>> open(slot_cap + 1);  // groups with room, by free slots
-  for (int oi : byneed) {
-    const int need = need_at(oi);
-    int k = -1, kf = 0;
-    for (int f = std::max(need, 1); f <= slot_cap; f++)  // first fit: the earliest group with room
-      if (!open[f].empty() && (k < 0 || *open[f].begin() < k)) k = *open[f].begin(), kf = f;
-    if (k < 0) {
-      k = (int)cg.size();
-      cg.emplace_back();
-      BatchGroup &g = cg.back();
-      memset(&g, 0, sizeof(g));
-      for (BatchList &L : g.list) L.dir = p->d_zero_dir;
-      lead.push_back(oi);
-    } else {
-      open[kf].erase(k);
+  std::vector<int> need(order.size());
+  for (size_t i = 0; i < order.size(); i++) need[i] = need_at(byneed[i]);
+  std::vector<int> group_of;
+  std::vector<BatchGroup> cg(pack_groups(need, slot_cap, p->cfg.queries_per_group, &group_of));
+  std::vector<int> lead(cg.size(), -1);  // order position of each group's first query
+  for (size_t i = 0; i < order.size(); i++) {
+    const int k = group_of[i];
+    if (lead[k] < 0) {
+      memset(&cg[k], 0, sizeof(BatchGroup));
+      for (BatchList &L : cg[k].list) L.dir = p->d_zero_dir;
+      lead[k] = byneed[i];
     }
-    add_query(cg[k], order[oi]);
-    const int free_slots = slot_cap - cg[k].nslots;
-    if (free_slots > 0 && cg[k].nq < p->cfg.queries_per_group) open[free_slots].insert(k);
+    add_query(cg[k], order[byneed[i]]);
   }
   std::vector<int> gi(cg.size());
   for (size_t k = 0; k < cg.size(); k++) gi[k] = (int)k;
@@ -1144,15 +1258,23 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
   p->stats_direct_cols = st_direct;
   p->stats_narrow_cols = st_narrow;
   p->stats_list_cols = st_list;
+  p->stats_auto_direct = st_auto;
   p->nq = nq;
   p->specs.assign(queries, queries + nq);
   p->h_groups.swap(groups);
   p->ngroups = (int)p->h_groups.size();
+  p->has_bindex = p->ngroups > 0;
+  p->has_ranked = !rank_groups.empty();
   if (nq == 0) return hipSuccess;
-  hipError_t e = hipMemcpyAsync(p->d_groups, p->h_groups.data(), (size_t)p->ngroups * sizeof(BatchGroup),
-                                hipMemcpyHostToDevice, stream);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(p->d_ngroups, &p->ngroups, sizeof(int), hipMemcpyHostToDevice, stream);
+  header.bindex_groups = p->ngroups;
+  p->h_plan.resize(p->rank_groups_at + rank_groups.size() * sizeof(RankGroup));
+  memcpy(p->h_plan.data(), &header, sizeof(header));
+  memcpy(p->h_plan.data() + sizeof(header), ranked.data(), ranked.size());
+  memcpy(p->h_plan.data() + p->rank_groups_at, rank_groups.data(), rank_groups.size() * sizeof(RankGroup));
+  hipError_t e = hipMemcpyAsync(p->d_plan, p->h_plan.data(), p->h_plan.size(), hipMemcpyHostToDevice, stream);
+  if (e == hipSuccess && p->has_bindex)
+    e = hipMemcpyAsync(p->d_groups, p->h_groups.data(), (size_t)p->ngroups * sizeof(BatchGroup),
+                       hipMemcpyHostToDevice, stream);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);  // the host vectors change on the next call
   return set_error(e, "rts_batch_plan_set_queries");
 }
@@ -1167,7 +1289,15 @@ hipError_t rts_batch_plan_launch(rts_batch_plan *p, BITS *out, int64_t out_strid
   if (!valid_output(p, out, out_stride_words))
     return set_error(hipErrorInvalidValue, "rts_batch_plan_launch: output must be 16-byte aligned, stride a multiple of 4 words");
   if (p->nq == 0) return hipSuccess;
-  return set_error(launch_batch(p, out, out_stride_words, counts, stream), "rts_batch_plan_launch");
+  int forms = forms_needed(p);
+  if (p->max_rank_groups && stream) {
+    // a launch captured by the caller runs both forms: either may have the queries set later
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const hipError_t e = hipStreamIsCapturing(stream, &capture);
+    if (e != hipSuccess) return set_error(e, "rts_batch_plan_launch");
+    if (capture != hipStreamCaptureStatusNone) forms = kFormBindex | kFormRanked;
+  }
+  return set_error(launch_batch(p, out, out_stride_words, counts, forms, stream), "rts_batch_plan_launch");
 }
 
 hipError_t rts_batch_plan_graph_launch(rts_batch_plan *p, BITS *out, int64_t out_stride_words,
@@ -1177,14 +1307,14 @@ hipError_t rts_batch_plan_graph_launch(rts_batch_plan *p, BITS *out, int64_t out
   if (p->nq == 0) return hipSuccess;
   hipError_t e = hipSuccess;
   if (!p->exec || p->graph_out != out || p->graph_counts != counts || p->graph_nq != p->nq ||
-      p->graph_stride != out_stride_words) {
+      p->graph_stride != out_stride_words || p->graph_forms != forms_needed(p)) {
     if (p->exec) (void)hipGraphExecDestroy(p->exec);
     if (p->graph) (void)hipGraphDestroy(p->graph);
     p->exec = nullptr;
     p->graph = nullptr;
     e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return set_error(e, "rts_batch_plan_graph_launch: capture");
-    hipError_t le = launch_batch(p, out, out_stride_words, counts, stream);
+    hipError_t le = launch_batch(p, out, out_stride_words, counts, forms_needed(p), stream);
     e = hipStreamEndCapture(stream, &p->graph);
     if (le != hipSuccess) e = le;
     if (e == hipSuccess) e = hipGraphInstantiate(&p->exec, p->graph, nullptr, nullptr, 0);
@@ -1193,6 +1323,7 @@ hipError_t rts_batch_plan_graph_launch(rts_batch_plan *p, BITS *out, int64_t out
     p->graph_counts = counts;
     p->graph_nq = p->nq;
     p->graph_stride = out_stride_words;
+    p->graph_forms = forms_needed(p);
   }
   return set_error(hipGraphLaunch(p->exec, stream), "rts_batch_plan_graph_launch");
 }
@@ -1252,7 +1383,16 @@ unsigned long long rts_batch_plan_mix_digest(const rts_batch_plan *p) {
 int rts_batch_plan_groups(const rts_batch_plan *p, rts_batch_config *cfg) {
   if (!p) return -1;
   if (cfg) *cfg = p->cfg;
-  return p->ngroups;
+  // as if each query were evaluated by its columns' forms
+  std::vector<int> need(p->specs.size());
+  for (size_t q = 0; q < need.size(); q++) {
+    need[q] = p->specs[q].ncols;
+    for (int c = 0; c < p->specs[q].ncols; c++)
+      if (p->specs[q].lo[c] > p->specs[q].hi[c]) need[q] = 0;
+  }
+  std::sort(need.begin(), need.end(), [](int a, int b) { return a > b; });
+  std::vector<int> group_of;
+  return pack_groups(need, batch_slots(p->cfg), p->cfg.queries_per_group, &group_of);
 }
 
 void rts_batch_plan_info(const rts_batch_plan *p, long long *n, int *ncols, int *nq) {
@@ -1268,7 +1408,7 @@ void rts_batch_plan_free(rts_batch_plan *p) {
   if (p->graph) (void)hipGraphDestroy(p->graph);
   free_dirs(p);
   (void)hipFree(p->d_groups);
-  (void)hipFree(p->d_ngroups);
+  (void)hipFree(p->d_plan);
   (void)hipFree(p->d_partials);
   (void)hipFree(p->d_sched);
   delete p;

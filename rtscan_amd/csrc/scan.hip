@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "common.h"
+#include "transpose.h"
 
 namespace rts {
 
@@ -332,35 +333,6 @@ struct RankedPreds {
   uint32_t copies;  // copies of the ranges' row counts (a power of two up to 64), stride entries apart
   uint32_t stride;
 };
-
-// out[p] bit 31 - r = in[r] bit p, in place (word 31 - p holds predicate p afterwards).
-__device__ __forceinline__ void transpose32(uint32_t (&a)[32]) {
-#pragma unroll
-  for (int k = 0; k < 16; k++) {
-    const uint32_t x = a[k], y = a[k + 16];
-    a[k] = __builtin_amdgcn_perm(x, y, 0x07060302);       // the upper halves
-    a[k + 16] = __builtin_amdgcn_perm(x, y, 0x05040100);  // the lower halves
-  }
-#pragma unroll
-  for (int b = 0; b < 32; b += 16)
-#pragma unroll
-    for (int k = b; k < b + 8; k++) {
-      const uint32_t x = a[k], y = a[k + 8];
-      a[k] = __builtin_amdgcn_perm(x, y, 0x07030501);      // bytes 3 and 1 of each
-      a[k + 8] = __builtin_amdgcn_perm(x, y, 0x06020400);  // bytes 2 and 0 of each
-    }
-#pragma unroll
-  for (int j = 4, s = 0; s < 3; j >>= 1, s++) {
-    const uint32_t m = j == 4 ? 0x0F0F0F0Fu : j == 2 ? 0x33333333u : 0x55555555u;
-#pragma unroll
-    for (int k = 0; k < 32; k++) {
-      if (k & j) continue;
-      const uint32_t x = a[k], y = a[k + j];
-      a[k] = (x & ~m) | ((y >> j) & m);
-      a[k + j] = ((x << j) & ~m) | (y & m);
-    }
-  }
-}
 
 // The bitmap words of the wave's 64 word positions from w0 on: rank4 holds the lane's 32
 // ranges, four a word.  FULL: np = 32 * HALVES and every position is inside the bitmap.

@@ -222,6 +222,13 @@ constexpr int kMultiLaneRows = 32;                      // rows per lane: one bi
 constexpr int kMultiTileRows = kWave * kMultiLaneRows;  // 2048 rows per wave tile
 constexpr unsigned kMultiMaxGrid = 4096;
 
+constexpr int kStaged = 8;               // predicates whose words pass through LDS at once
+// Bitmaps that do not start on cache lines: bytes of them from which on that pays.  In less
+// the parts of a line meet in the caches before they are written, and the barriers show (33
+// bitmaps of 5e7 rows, 206 MB, counted: 93 us without, 98 with); more is bound by the rate at
+// which partial lines are written: 64 bitmaps of 1e8 rows, 800 MB, 322 -> 286 us (259 when
+// they start on lines), 32, 400 MB, 197 -> 181; 64 of 2e8 rows 607 -> 517.
+constexpr uint64_t kStagedBytes = 320u << 20;
 constexpr uint32_t kHistEntries = 1024;  // row counts of a workgroup: all copies
 constexpr unsigned kScanXcds = 8;
 constexpr int kRankEntries = 2 * kMultiPreds + 2;       // ranges between the bounds, and one for no row
@@ -322,7 +329,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_multi(const uint32_t *col, uint
 // predicates) in a register; the wave stores 64 consecutive words of each bitmap.  COUNT:
 // rows per range by LDS adds, which make each predicate's rows at the end (popcounts of the
 // words cost 180 us more at 64 predicates).  1e8 rows, 64 predicates, counted: 732 us by
-// testing each predicate, 322 this way, 176 of it when nothing is stored.
+// testing each predicate, 288 this way, 176 of it when nothing is stored.
 struct RankedPreds {
   uint32_t tree[128];             // [1, 2^levels): bounds but the smallest, breadth-first, padded with 2^32 - 1
   uint32_t mask[2][kRankEntries];  // predicates matching range r, 32 per half; the last entry is 0
@@ -362,13 +369,59 @@ __device__ __forceinline__ void store_ranked(uint32_t (&rank4)[8], const uint32_
   }
 }
 
-template <int HALVES, bool COUNT, bool FULL>
+// As store_ranked for a workgroup of whole tiles, in step: the waves' words pass through LDS,
+// so that one wave stores the workgroup's 1 KB of a predicate at once, and fewer cache lines
+// are filled by several stores (256 bytes a store: 2.7 TB/s where the bitmaps do not start on
+// lines, 1 KB: 3.9).  Bitmaps at 16-byte offsets take non-temporal 16-byte stores (64 of 1e8
+// rows: 303 -> 286 us); 4-byte ones are slower non-temporal (322 -> 336).  w0: of wave 0.
+template <int HALVES, bool FULL>
+__device__ __forceinline__ void store_ranked_staged(uint32_t (&rank4)[8], const uint32_t (&mask)[HALVES][kRankEntries],
+                                                    uint32_t (&words)[2][kStaged][kBlock], int half0, int np, BITS *out,
+                                                    uint64_t stride, uint64_t w0, int wv, int lane) {
+#pragma unroll 1
+  for (int h = 0; h < HALVES; h++) {
+    uint32_t a[32];
+#pragma unroll
+    for (int r = 0; r < 8; r++) asm volatile("" : "+v"(rank4[r]));  // as in store_ranked
+#pragma unroll
+    for (int r = 0; r < 32; r++) a[r] = mask[h][(rank4[r / 4] >> (8 * (r & 3))) & 0xFF];
+    transpose32(a);
+    const int p0 = 32 * (half0 + h) + wv;
+    BITS *o = out + (uint64_t)p0 * stride + w0;
+    const bool vec = (((uint64_t)out | stride * sizeof(BITS)) & 15) == 0;
+    int left = np - p0;
+#pragma unroll
+    for (int k = 0; k < 32; k += kStaged) {
+      uint32_t(&buf)[kStaged][kBlock] = words[k / kStaged % 2];
+#pragma unroll
+      for (int q = 0; q < kStaged; q++) buf[q][kWave * wv + lane] = a[31 - k - q];
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < kStaged; q += kBlock / kWave) {
+        if (FULL || left > 0) {
+          if (vec) {
+            __builtin_nontemporal_store(reinterpret_cast<const u32x4 *>(buf[q + wv])[lane], reinterpret_cast<u32x4 *>(o) + lane);
+          } else {
+#pragma unroll
+            for (int j = 0; j < kBlock / kWave; j++) o[kWave * j + lane] = buf[q + wv][kWave * j + lane];
+          }
+        }
+        o += stride * (kBlock / kWave);
+        left -= kBlock / kWave;
+        asm volatile("" : "+s"(left));
+      }
+    }
+  }
+}
+
+template <int HALVES, bool COUNT, bool FULL, bool STAGED>
 __global__ __launch_bounds__(kBlock) void k_scan_ranked(const uint32_t *col, uint64_t n, uint64_t whole,
                                                         RankedPreds rp, int np, BITS *out, uint64_t stride,
                                                         uint32_t run, uint32_t *partials) {
   __shared__ uint32_t tree[128];
   __shared__ uint32_t mask[HALVES][kRankEntries];
   __shared__ alignas(16) uint32_t xch[kBlock / kWave][kMultiTileRows / 4];
+  __shared__ alignas(16) uint32_t staged[2][kStaged][kBlock];
   // rows per range (COUNT), in as many copies as fit (four for 64 predicates, one a lane for
   // four): a wave's rows of one range would otherwise add to one address one after another
   // (3 predicates over 2^25 rows, counted: 48 us with four copies)
@@ -457,7 +510,10 @@ __global__ __launch_bounds__(kBlock) void k_scan_ranked(const uint32_t *col, uin
     if (kWhole && t < whole) load(t);
     uint32_t rank4[8];
     exchange(rank4);
-    store_ranked<HALVES, kWhole && FULL>(rank4, mask, half0, np, out, stride, w0, kWhole || w0 + lane < words, lane);
+    if constexpr (kWhole && STAGED)
+      store_ranked_staged<HALVES, FULL>(rank4, mask, staged, half0, np, out, stride, w0 - wv * (kMultiTileRows / 32), wv, lane);
+    else
+      store_ranked<HALVES, kWhole && FULL>(rank4, mask, half0, np, out, stride, w0, kWhole || w0 + lane < words, lane);
   };
   // the first tile apart, so that every tile of the loop finds its loads issued before the
   // stores of the one before
@@ -703,14 +759,24 @@ static RankedPreds rank_table(const CODE *lo, const CODE *hi, int np) {
 template <int HALVES>
 static void launch_ranked(const uint32_t *col, uint64_t n, const RankedPreds &t, int np, BITS *out, uint64_t stride,
                           uint32_t run, uint32_t *partials, dim3 grid, hipStream_t s) {
-  const uint64_t whole = aligned16(col) ? n / kMultiTileRows : 0;
   const bool full = np == 32 * HALVES * (int)grid.y;
-  if (partials)
-    full ? k_scan_ranked<HALVES, true, true><<<grid, kBlock, 0, s>>>(col, n, whole, t, np, out, stride, run, partials)
-         : k_scan_ranked<HALVES, true, false><<<grid, kBlock, 0, s>>>(col, n, whole, t, np, out, stride, run, partials);
-  else
-    full ? k_scan_ranked<HALVES, false, true><<<grid, kBlock, 0, s>>>(col, n, whole, t, np, out, stride, run, partials)
-         : k_scan_ranked<HALVES, false, false><<<grid, kBlock, 0, s>>>(col, n, whole, t, np, out, stride, run, partials);
+  const bool staged = ((uintptr_t)out % 128 || stride * sizeof(BITS) % 128) &&
+                      (uint64_t)np * words_for_rows(n) * sizeof(BITS) >= kStagedBytes;
+  // staged, a workgroup's waves go in step: whole tiles for all of them
+  const uint64_t tiles = aligned16(col) ? n / kMultiTileRows : 0, whole = staged ? tiles / (kBlock / kWave) * (kBlock / kWave) : tiles;
+  auto go = [&](auto count, auto full, auto staged) {
+    k_scan_ranked<HALVES, decltype(count)::value, decltype(full)::value, decltype(staged)::value>
+        <<<grid, kBlock, 0, s>>>(col, n, whole, t, np, out, stride, run, partials);
+  };
+  auto pick = [&](auto count) {
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    if (staged)
+      full ? go(count, yes, yes) : go(count, no, yes);
+    else
+      full ? go(count, yes, no) : go(count, no, no);
+  };
+  partials ? pick(std::true_type{}) : pick(std::false_type{});
 }
 
 // Predicates up to which a pass tests each one (k_scan_multi) instead of searching
@@ -720,7 +786,7 @@ static void launch_ranked(const uint32_t *col, uint64_t n, const RankedPreds &t,
 // counted, tests against search: 1e5 rows, 64 predicates 10.7 / 11.3 us; 2^19 rows, 33: 9.3 /
 // 10.3, 64: 11.1 / 10.2; 2^20 rows, 16: 8.7 / 9.3, 24: 10.8 / 10.0, 64: 15.5 / 11.0; 4.2e6
 // rows, 8: 11.3 / 11.6, 10: 12.2 / 12.4, 16: 15.9 / 12.7; 1e8 rows, 5: 100 / 103, 8: 116 /
-// 105, 16: 199 / 119, 32: 379 / 196, 64: 732 / 322 (260 when every bitmap starts on a
+// 105, 16: 199 / 119, 32: 379 / 181, 64: 732 / 288 (259 when every bitmap starts on a
 // 128-byte line: what is left is the writes' rate).
 static int direct_preds(uint64_t n) {
   return n < (1u << 18) ? kMultiPreds : n < (1u << 20) ? 40 : n < (1u << 22) ? 16 : 8;
@@ -753,7 +819,7 @@ hipError_t scan_ranges(const CODE *col, uint64_t n, const CODE *lo, const CODE *
       const uint64_t wgtiles = (n + kMultiTileRows * (kBlock / kWave) - 1) / (kMultiTileRows * (kBlock / kWave));
       // a tile a wave while the workgroups all fit at once (4 per compute unit); a long
       // column takes more, shorter workgroups, which even out (1e8 rows, 64 predicates: 338
-      // us with 4 per compute unit, 322 with 16; 1e7 rows: 32 against 38), and gives an XCD
+      // us with 4 per compute unit, 322 with 16, stored from registers; 1e7 rows: 32 against 38), and gives an XCD
       // runs of 16 steps (337 against 366 us)
       const bool large = wgtiles >= cus * 16;
       grid = grid_for(wgtiles, 1, std::min<unsigned>(kMultiMaxGrid, cus * (large ? 16 : 4)));

@@ -101,3 +101,31 @@ def test_ranges_of_a_column_of_one_value(eng):
     for value in (0, 12345, MAXU):
         x = np.full((1 << 20) + 5, value, np.uint32)
         _check(eng, x, _ranges(x, 64, 1) + [(value, value)] * 3)
+
+
+@pytest.mark.parametrize("n,npred,pad", [(45_000_003, 63, 0), (45_000_003, 64, 2), (90_000_001, 31, 1)])
+def test_bitmaps_of_many_bytes_off_cache_lines(eng, n, npred, pad):
+    """Bitmaps of more bytes than the caches hold that don't start on cache lines, at 4- and at
+    16-byte offsets: against one range a call, and numpy for some."""
+    words = (n + 31) // 32
+    stride = words + pad
+    assert 4 * words * npred >= 320 << 20 and stride % 32
+    x = _column(n, n % 1000)
+    preds = _ranges(x, npred, npred)
+    col = eng.DeviceBuffer.from_numpy(x)
+    out = eng.DeviceBuffer(4 * npred * stride).fill(0xA5)
+    counts = eng.DeviceBuffer(8 * npred)
+    eng.scan_ranges(col, n, [p[0] for p in preds], [p[1] for p in preds], out, stride, counts)
+    eng.synchronize()
+    got = out.to_numpy(np.uint32, npred * stride).reshape(npred, stride)
+    cnt = counts.to_numpy(np.uint64, npred)
+    one, c1 = eng.DeviceBuffer(4 * words), eng.DeviceBuffer(8)
+    for p, (lo, hi) in enumerate(preds):
+        eng.scan_range(col, n, lo, hi, one, c1)
+        eng.synchronize()
+        assert np.array_equal(got[p, :words], one.to_numpy(np.uint32, words)), p
+        assert cnt[p] == c1.to_numpy(np.uint64, 1)[0], p
+        if p % 29 == 2 and lo <= hi:
+            assert np.array_equal(got[p, :words], pack_rows(interval_mask(x, lo, hi))), p
+    if pad:
+        assert (got[:, words:] == 0xA5A5A5A5).all()

@@ -13,9 +13,9 @@
 // a search of every column (24 VALU instructions, 8 LDS reads at 254 bounds) and per 32
 // queries 17 VALU instructions for four columns (8 lookups and ANDs, 8 the transpose), and
 // memory moves the columns and the bitmaps alone.  Launches, k_batch against this, us: 1e8
-// rows x 4, 1024 queries 7180 / 5510; 2^26 x 2, 64 queries 374 / 232 (its memory traffic
-// alone 210); 2e7 x 3, 333 queries 530 / 358; queries that no index serves, 1e8 x 4, 256:
-// 15500 / 1420.  plan_rank_groups says where the lines lie.
+// rows x 4, 1024 queries 7180 / 5250; 2^26 x 2, 64 queries 374 / 226 (its memory traffic
+// alone 210); 2e7 x 3, 333 queries 530 / 327; queries that no index serves, 1e8 x 4, 256:
+// 15500 / 1400.  plan_rank_groups says where the lines lie.
 #include <string.h>
 
 #include <algorithm>
@@ -97,8 +97,10 @@ __device__ __forceinline__ uint32_t wave_counts32(const uint32_t (&words)[32], i
 // - Writes: lines that two stores fill in part are what a long batch waits for.  Stored
 //   straight from the transposed registers (256 bytes a wave and query) bitmaps of 12.5 MB,
 //   which start 32 bytes past a line, are written at 2.7 TB/s, aligned ones at 5.4; passed
-//   through LDS, 1 KB a workgroup and query, at 3.9 (1e8 rows x 4, 1024 queries: 7.2 ms / 5.6).
-//   Two buffers: one barrier for every 8 queries.
+//   through LDS, 1 KB a workgroup and query, at 3.9 (1e8 rows x 4, 1024 queries: 7.2 ms / 5.6),
+//   and non-temporal, which leaves the caches to the columns that the other groups read
+//   again, at 4.2 (5.49 ms / 5.25; 2e7 rows x 3, 333 queries 358 us / 327).  Two buffers: one
+//   barrier for every 8 queries.
 // - 256 registers a lane: the next column's 32 rows are loaded during the search of this
 //   one's, and the next step's before this one's stores, which later loads would wait for
 //   (5.8 -> 5.6 ms); 64 queries' masks come with one address each.  With 128 registers (twice
@@ -303,7 +305,7 @@ __global__ __launch_bounds__(kRankThreads) __attribute__((amdgpu_waves_per_eu(kR
                 const u32x4 x = *reinterpret_cast<const u32x4 *>(&lds.words[p / kRankStaged % 2][q + wv][4 * lane]);
                 RTS_GLOBAL BITS *o = (RTS_GLOBAL BITS *)(place0 + place[p + q] * place1) + w0;
                 if (kWhole || w0 + 4 <= words) {
-                  *(RTS_GLOBAL u32x4 *)o = x;
+                  __builtin_nontemporal_store(x, (RTS_GLOBAL u32x4 *)o);
                 } else {
 #pragma unroll
                   for (int j = 0; j < 3; j++)
@@ -403,7 +405,7 @@ struct GroupPlan {
     for (int c = 0; c < ncols; c++) compute += 14 * levels(c);
     for (size_t i = 0; i < query.size(); i += 64)
       compute += (52 + 7 * __builtin_popcount(cols_of(i, q))) * (i + 32 < query.size() ? 2 : 1);
-    return 3.2 * query.size() + std::max(memory ? 82.0 * ncols : 0.0, compute / 2);
+    return 2.9 * query.size() + std::max(memory ? 82.0 * ncols : 0.0, compute / 2);
   }
 };
 
@@ -488,8 +490,8 @@ Plan groups_dealt(const std::vector<Predicates> &q, const std::vector<int> &orde
 
 // Time of a plan in microseconds.  A workgroup that stays with its group waits for those of the
 // longest.  Measured (1e8 rows, 4 columns / 2 columns, mixed queries, us): 32 queries 440 / 271,
-// 64 550 / 377, 128 790 / 653, 256 1430 / 1230, 1024 5510 / -; 2e7 rows, 4 columns: 32 121, 64
-// 147, 256 324; 1e6 rows, 4 columns: 16 25, 64 31.
+// 64 550 / 377, 128 764 / 608, 256 1420 / 1230, 1024 5250 / -; 2e7 rows, 4 columns: 32 121, 64
+// 147, 128 191; 1e6 rows, 4 columns: 16 25, 64 31.
 double plan_us(const Plan &p, const std::vector<Predicates> &q, int64_t n) {
   const uint32_t steps = (uint32_t)((n + kRankStepRows - 1) / kRankStepRows), grid = rank_grid();
   const uint32_t stride = rank_stride((uint32_t)p.size(), grid / kXcds);
@@ -512,7 +514,7 @@ bool plan_rank_groups(const std::vector<RankQuery> &in, int64_t n, int max_group
   header->steps = 1;
   if (in.size() < (size_t)kRankMinQueries || in.size() > (size_t)max_groups * kRankQueries) return false;
   // at least the bitmaps are written
-  if (3.2 * in.size() * n / 1e8 >= bindex_us) return false;
+  if (2.9 * in.size() * n / 1e8 >= bindex_us) return false;
   std::vector<Column> columns;
   std::vector<std::vector<std::pair<uint32_t, int *>>> bounds;  // (bound less one, where its number goes)
   std::vector<Predicates> q(in.size());

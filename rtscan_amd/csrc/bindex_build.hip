@@ -21,42 +21,88 @@
 
 namespace rts {
 
+// What the build finds out on the device, for the host in one copy and for the kernels after.
+struct BuildHead {
+  int64_t idx[kAreas];       // first sorted slot of each area
+  int64_t rk[2 * kMaxBins];  // as start_ranks
+  CODE starts[kAreas], estarts[kMaxBins];
+  uint32_t boff[kMaxBins + 1];
+  CODE data_max;
+  uint8_t light[kMaxBins];  // a bin start of at most kLightStartRows rows goes into its bin's list
+};
+
 // Area starts (bindex.cpp:613-631): start[i] = sorted[i * avg]; if it equals the previous
 // start the area begins mid-run at i * avg, otherwise at the first occurrence of the value.
-__global__ void k_area_starts(const CODE *sorted, int64_t n, CODE *starts, int64_t *idx) {
-  const int i = threadIdx.x;
-  if (i >= kAreas) return;
-  const int64_t avg = n / kAreas;
-  const CODE v = sorted[i * avg];
-  starts[i] = v;
-  if (i == 0) {
-    idx[0] = 0;
-    return;
-  }
-  if (v == sorted[(i - 1) * avg]) {
-    idx[i] = i * avg;
-    return;
-  }
-  int64_t lo = (i - 1) * avg, hi = i * avg;  // first slot in (lo, hi] holding v
-  while (lo + 1 < hi) {
-    const int64_t mid = lo + (hi - lo) / 2;
-    if (sorted[mid] < v)
-      lo = mid;
-    else
-      hi = mid;
-  }
-  idx[i] = hi;
-}
-
 // Bin starts: area a (sorted slots [idx[a], idx[a + 1])) cut into `sub` equal-count bins;
 // bin a * sub + j starts at the value in slot idx[a] + j * len / sub, so bin a * sub is
-// the area's own start.
-__global__ void k_bin_starts(const CODE *sorted, int64_t n, const int64_t *idx, int sub, CODE *estarts) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= kAreas * sub) return;
-  const int a = b / sub, j = b % sub;
-  const int64_t s0 = idx[a], len = (a + 1 < kAreas ? idx[a + 1] : n) - s0;
-  estarts[b] = sorted[s0 + (int64_t)j * len / sub];
+// the area's own start.  Ranks of the bin starts: searched between the neighbouring bins'
+// slots, unless a run reaches over one.  Bound by latency, chains of a dozen or two loads in
+// one workgroup.  Three kernels with the host between them, and the blocks' slots from the
+// host, made a build of 1e6 rows and 256 bins take 423 us; it is 308 (1e5: 353, 245).
+constexpr int kStartThreads = 1024;
+__global__ __launch_bounds__(kStartThreads) void k_build_starts(const CODE *sorted, int64_t n, int sub, BuildHead *head) {
+  __shared__ int64_t idx[kAreas + 1];
+  const int i = threadIdx.x;
+  if (i < kAreas) {
+    const int64_t avg = n / kAreas;
+    const CODE v = sorted[i * avg];
+    int64_t hi = i * avg;
+    if (i > 0 && v != sorted[(i - 1) * avg]) {  // first slot in (lo, hi] holding v
+      int64_t lo = (i - 1) * avg;
+      while (lo + 1 < hi) {
+        const int64_t mid = lo + (hi - lo) / 2;
+        if (sorted[mid] < v)
+          lo = mid;
+        else
+          hi = mid;
+      }
+    }
+    idx[i] = hi;
+    head->idx[i] = hi;
+    head->starts[i] = v;
+  }
+  if (i == 0) {
+    idx[kAreas] = n;
+    head->data_max = sorted[n - 1];
+  }
+  __syncthreads();
+  const int bins = kAreas * sub;
+  auto slot = [&](int b) {
+    const int64_t s0 = idx[b / sub];
+    return s0 + b % sub * (idx[b / sub + 1] - s0) / sub;
+  };
+  for (int r = i; r < 2 * bins; r += kStartThreads) {
+    const int b = r / 2;
+    const bool above = r & 1;  // first slot with a value > v, else with one >= v
+    const int64_t at = slot(b);
+    const CODE v = sorted[at];
+    int64_t lo, hi;
+    if (above) {
+      const int64_t next = b + 1 < bins ? slot(b + 1) : n;
+      const bool ends = next == n || sorted[next] > v;
+      lo = ends ? at + 1 : next + 1;
+      hi = ends ? next : n;
+    } else {
+      const int64_t prev = b > 0 ? slot(b - 1) : 0;
+      const bool begins = sorted[prev] < v;
+      lo = begins ? prev + 1 : 0;
+      hi = begins ? at : prev;
+    }
+    while (lo < hi) {
+      const int64_t mid = lo + (hi - lo) / 2;
+      const CODE x = sorted[mid];
+      if (above ? x > v : x >= v)
+        hi = mid;
+      else
+        lo = mid + 1;
+    }
+    head->rk[r] = lo;
+    const int64_t other = __shfl_xor((long long)lo, 1, kWave);
+    if (above) {
+      head->estarts[b] = v;
+      head->light[b] = lo - other <= kLightStartRows;
+    }
+  }
 }
 
 // out[i] = sorted[i * kRankSample] for i < m.
@@ -303,10 +349,10 @@ __global__ __launch_bounds__(kBlock) void k_list_entries(const CODE *col, const 
   }
 }
 
-// boff[k] = the directory's first entry of bin k, for k in [0, bins] (its rows end at the next bin's).
-__global__ void k_bin_offsets(const uint32_t *bdir, int64_t ntiles, int bins, uint32_t *boff) {
+// boff[k] = boff2[k] = the directory's first entry of bin k, for k in [0, bins] (its rows end at the next bin's).
+__global__ void k_bin_offsets(const uint32_t *bdir, int64_t ntiles, int bins, uint32_t *boff, uint32_t *boff2) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k <= bins) boff[k] = k < bins ? bdir[k * (ntiles + 1)] : bdir[bins * (ntiles + 1) - 1];
+  if (k <= bins) boff[k] = boff2[k] = k < bins ? bdir[k * (ntiles + 1)] : bdir[bins * (ntiles + 1) - 1];
 }
 
 // bdir[k * (ntiles + 1) + t] = first entry of bin k with row >= t * tile_rows
@@ -336,15 +382,28 @@ hipError_t launch_tile_directory(const rts_bindex_dev *d, int64_t ntiles, int64_
   return hipGetLastError();
 }
 
-// First and last value of every 3276-row block of every area (init_area,
-// bindex.cpp:410-427), for the host-side in_which_block.
-__global__ void k_block_bounds(const CODE *sorted, const int64_t *blk_first_slot,
-                               const int64_t *blk_last_slot, int64_t nblocks, CODE *first,
-                               CODE *last) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nblocks) return;
-  first[i] = sorted[blk_first_slot[i]];
-  last[i] = sorted[blk_last_slot[i]];
+// Blocks of an area of `len` rows (init_area, bindex.cpp:410-427).
+__host__ __device__ __forceinline__ int64_t area_blocks(int64_t len) {
+  return (len + RTS_BLOCK_INIT_SIZE - 1) / RTS_BLOCK_INIT_SIZE;
+}
+
+// First and last value of every 3276-row block of every area, in order, for the host-side
+// in_which_block.  A workgroup an area.
+__global__ __launch_bounds__(kAreas) void k_block_bounds(const CODE *sorted, int64_t n, const int64_t *idx, CODE *first,
+                                                         CODE *last) {
+  __shared__ unsigned long long before;
+  const int a = blockIdx.x, t = threadIdx.x;
+  auto len = [&](int k) { return (k + 1 < kAreas ? idx[k + 1] : n) - idx[k]; };
+  if (t == 0) before = 0;
+  __syncthreads();
+  if (t < a) atomicAdd(&before, (unsigned long long)area_blocks(len(t)));
+  __syncthreads();
+  const int64_t s0 = idx[a], rows = len(a), blocks = area_blocks(rows);
+  for (int64_t b = t; b < blocks; b += kAreas) {
+    const int64_t r = b * RTS_BLOCK_INIT_SIZE;
+    first[before + b] = sorted[s0 + r];
+    last[before + b] = sorted[s0 + min(r + RTS_BLOCK_INIT_SIZE, rows) - 1];
+  }
 }
 
 static unsigned blocks_for(int64_t items, int per = kBlock) {
@@ -527,6 +586,9 @@ hipError_t bindex_host_blocks(BinDex *bx) {
   return hipSuccess;
 }
 
+// Values of the sorted column that are copied to the host with the starts, at most (64 KB).
+constexpr int64_t kStagedTail = 1 << 14;
+
 hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int sub, hipStream_t s) {
   hipError_t err = hipSuccess;
   rts_bindex_dev *d = nullptr;
@@ -534,17 +596,17 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   uint16_t *keys = nullptr;
   void *sort_tmp = nullptr, *tmp = nullptr;
   size_t need = 0;
-  CODE *starts_d = nullptr, *estarts_d = nullptr;
-  int64_t *idx_d = nullptr, *bf_slot_d = nullptr, *bl_slot_d = nullptr;
-  CODE *bfirst_d = nullptr, *blast_d = nullptr;
-  std::vector<int64_t> bf_slot, bl_slot;
+  BuildHead *head_d = nullptr;
+  std::vector<BuildHead> head(1);
+  CODE *tail_d = nullptr;  // rank samples, then the blocks' first and last values
+  const int64_t samples = (n + kRankSample - 1) / kRankSample, max_blocks = n / RTS_BLOCK_INIT_SIZE + kAreas;
+  std::vector<CODE> tail;
+  // few: copied with the head and moved on the host
+  const bool tail_host = samples + 2 * max_blocks <= kStagedTail;
   int64_t nblocks = 0;
-  int64_t idx_h[kAreas];
   uint32_t nb = 0;
   int bins = 0;
   std::vector<int64_t> rk;
-  uint8_t light_h[kMaxBins];
-  uint8_t *light_d = nullptr;
 
   if (!bx || !col || n < kAreas || n > 0x7FFFFFFFll || (sub != 1 && sub != 2 && sub != 4 && sub != 8))
     return hipErrorInvalidValue;
@@ -565,43 +627,34 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   RTS_TRY(pool_alloc(&sort_tmp, sort_rows_workspace(n)));
   RTS_TRY(sort_rows(col, n, d->sorted_val, (uint32_t *)d->sorted_pos, sort_tmp, s));
 
-  // 2. area starts, then bin starts
-  RTS_TRY(pool_alloc(&starts_d, kAreas * sizeof(CODE)));
-  RTS_TRY(pool_alloc(&idx_d, kAreas * sizeof(int64_t)));
-  RTS_TRY(pool_alloc(&estarts_d, bins * sizeof(CODE)));
-  hipLaunchKernelGGL(k_area_starts, dim3(1), dim3(kAreas), 0, s, d->sorted_val, n, starts_d, idx_d);
+  // 2. area and bin starts; the values the host keeps of the sorted column
+  RTS_TRY(pool_alloc(&head_d, sizeof(BuildHead)));
+  hipLaunchKernelGGL(k_build_starts, dim3(1), dim3(kStartThreads), 0, s, d->sorted_val, n, sub, head_d);
   RTS_TRY(hipGetLastError());
-  hipLaunchKernelGGL(k_bin_starts, dim3((bins + kBlock - 1) / kBlock), dim3(kBlock), 0, s, d->sorted_val, n,
-                     idx_d, sub, estarts_d);
+  RTS_TRY(pool_alloc(&tail_d, (samples + 2 * max_blocks) * sizeof(CODE)));
+  hipLaunchKernelGGL(k_rank_samples, dim3((unsigned)((samples + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
+                     d->sorted_val, samples, tail_d);
   RTS_TRY(hipGetLastError());
-  d->estarts.resize(bins);
-  RTS_TRY(hipMemcpyAsync(d->starts, starts_d, sizeof(d->starts), hipMemcpyDeviceToHost, s));
-  RTS_TRY(hipMemcpyAsync(d->estarts.data(), estarts_d, bins * sizeof(CODE), hipMemcpyDeviceToHost, s));
-  RTS_TRY(hipMemcpyAsync(idx_h, idx_d, sizeof(idx_h), hipMemcpyDeviceToHost, s));
-  RTS_TRY(hipMemcpyAsync(&bx->data_max, d->sorted_val + n - 1, sizeof(CODE), hipMemcpyDeviceToHost, s));
+  hipLaunchKernelGGL(k_block_bounds, dim3(kAreas), dim3(kAreas), 0, s, d->sorted_val, n, head_d->idx, tail_d + samples,
+                     tail_d + samples + max_blocks);
+  RTS_TRY(hipGetLastError());
 
-  // 3. filter vectors + list keys; a bin start of at most kLightStartRows rows goes into
-  //    its bin's list
-  RTS_TRY(hipStreamSynchronize(s));  // d->estarts
-  RTS_TRY(start_ranks(d, rk, s));
-  for (int k = 0; k < bins; k++) light_h[k] = rk[2 * k + 1] - rk[2 * k] <= kLightStartRows;
-  RTS_TRY(pool_alloc(&light_d, bins));
-  RTS_TRY(hipMemcpyAsync(light_d, light_h, bins, hipMemcpyHostToDevice, s));
+  // 3. filter vectors + list keys
   RTS_TRY(pool_alloc(&d->fvs, (size_t)(bins - 1) * d->fv_stride * sizeof(BITS)));
   RTS_TRY(pool_alloc(&keys, n * sizeof(uint16_t)));
   {
     const dim3 grid(blocks_for((n + kFvTileRows - 1) / kFvTileRows, kBlock / kWave));
     if (bins <= 128)
-      hipLaunchKernelGGL(k_build_fvs<8>, grid, dim3(kBlock), 0, s, col, n, estarts_d, light_d, bins, d->fvs,
+      hipLaunchKernelGGL(k_build_fvs<8>, grid, dim3(kBlock), 0, s, col, n, head_d->estarts, head_d->light, bins, d->fvs,
                          d->fv_stride, keys);
     else if (bins <= 256)
-      hipLaunchKernelGGL(k_build_fvs<9>, grid, dim3(kBlock), 0, s, col, n, estarts_d, light_d, bins, d->fvs,
+      hipLaunchKernelGGL(k_build_fvs<9>, grid, dim3(kBlock), 0, s, col, n, head_d->estarts, head_d->light, bins, d->fvs,
                          d->fv_stride, keys);
     else if (bins <= 512)
-      hipLaunchKernelGGL(k_build_fvs<10>, grid, dim3(kBlock), 0, s, col, n, estarts_d, light_d, bins, d->fvs,
+      hipLaunchKernelGGL(k_build_fvs<10>, grid, dim3(kBlock), 0, s, col, n, head_d->estarts, head_d->light, bins, d->fvs,
                          d->fv_stride, keys);
     else
-      hipLaunchKernelGGL(k_build_fvs<11>, grid, dim3(kBlock), 0, s, col, n, estarts_d, light_d, bins, d->fvs,
+      hipLaunchKernelGGL(k_build_fvs<11>, grid, dim3(kBlock), 0, s, col, n, head_d->estarts, head_d->light, bins, d->fvs,
                          d->fv_stride, keys);
   }
   RTS_TRY(hipGetLastError());
@@ -619,15 +672,22 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
     RTS_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, need, counts, d->bdir, items, s));
     RTS_TRY(pool_alloc(&d->boff, (bins + 1) * sizeof(uint32_t)));
     hipLaunchKernelGGL(k_bin_offsets, dim3((bins + 1 + kBlock - 1) / kBlock), dim3(kBlock), 0, s, d->bdir, d->ntiles,
-                       bins, d->boff);
+                       bins, d->boff, head_d->boff);
     RTS_TRY(hipGetLastError());
   }
-  d->boff_host.resize(bins + 1);
-  RTS_TRY(hipMemcpyAsync(d->boff_host.data(), d->boff, (bins + 1) * sizeof(uint32_t),
-                         hipMemcpyDeviceToHost, s));
+  RTS_TRY(hipMemcpyAsync(head.data(), head_d, sizeof(BuildHead), hipMemcpyDeviceToHost, s));
+  if (tail_host) {
+    tail.resize(samples + 2 * max_blocks);
+    RTS_TRY(hipMemcpyAsync(tail.data(), tail_d, tail.size() * sizeof(CODE), hipMemcpyDeviceToHost, s));
+  }
   RTS_TRY(hipStreamSynchronize(s));
+  memcpy(d->starts, head[0].starts, sizeof(d->starts));
+  d->estarts.assign(head[0].estarts, head[0].estarts + bins);
+  d->boff_host.assign(head[0].boff, head[0].boff + bins + 1);
+  bx->data_max = head[0].data_max;
   nb = d->boff_host[bins];
   d->nb = nb;
+  rk.assign(head[0].rk, head[0].rk + 2 * bins);
   mark_complete_bins(d, rk);
   RTS_TRY(pool_alloc(&d->bent, std::max<uint32_t>(nb, 1) * sizeof(uint2)));
   if (nb) {
@@ -649,36 +709,25 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
 
   // 5. host descriptor: areas (bindex.cpp:633-652) and their blocks
   for (int k = 0; k < kAreas; k++) {
-    d->area_start[k] = idx_h[k];
-    d->area_len[k] = (k < kAreas - 1 ? idx_h[k + 1] : n) - idx_h[k];
+    d->area_start[k] = head[0].idx[k];
+    d->area_len[k] = (k < kAreas - 1 ? head[0].idx[k + 1] : n) - head[0].idx[k];
+    nblocks += area_blocks(d->area_len[k]);
   }
-  for (int k = 0; k < kAreas; k++) {
-    const int64_t len = d->area_len[k];
-    int64_t i = 0;
-    while (i + RTS_BLOCK_INIT_SIZE < len) {
-      bf_slot.push_back(d->area_start[k] + i);
-      bl_slot.push_back(d->area_start[k] + i + RTS_BLOCK_INIT_SIZE - 1);
-      i += RTS_BLOCK_INIT_SIZE;
-    }
-    bf_slot.push_back(d->area_start[k] + i);
-    bl_slot.push_back(d->area_start[k] + len - 1);
+  if (tail_host) {
+    const CODE *t = tail.data();
+    d->rank_samples.assign(t, t + samples);
+    d->block_first.assign(t + samples, t + samples + nblocks);
+    d->block_last.assign(t + samples + max_blocks, t + samples + max_blocks + nblocks);
+  } else {
+    d->rank_samples.resize(samples);
+    d->block_first.resize(nblocks);
+    d->block_last.resize(nblocks);
+    RTS_TRY(hipMemcpyAsync(d->rank_samples.data(), tail_d, samples * sizeof(CODE), hipMemcpyDeviceToHost, s));
+    RTS_TRY(hipMemcpyAsync(d->block_first.data(), tail_d + samples, nblocks * sizeof(CODE), hipMemcpyDeviceToHost, s));
+    RTS_TRY(hipMemcpyAsync(d->block_last.data(), tail_d + samples + max_blocks, nblocks * sizeof(CODE),
+                           hipMemcpyDeviceToHost, s));
   }
-  nblocks = (int64_t)bf_slot.size();
-  d->block_first.resize(nblocks);
-  d->block_last.resize(nblocks);
-  RTS_TRY(pool_alloc(&bf_slot_d, nblocks * sizeof(int64_t)));
-  RTS_TRY(pool_alloc(&bl_slot_d, nblocks * sizeof(int64_t)));
-  RTS_TRY(pool_alloc(&bfirst_d, nblocks * sizeof(CODE)));
-  RTS_TRY(pool_alloc(&blast_d, nblocks * sizeof(CODE)));
-  RTS_TRY(hipMemcpyAsync(bf_slot_d, bf_slot.data(), nblocks * sizeof(int64_t), hipMemcpyHostToDevice, s));
-  RTS_TRY(hipMemcpyAsync(bl_slot_d, bl_slot.data(), nblocks * sizeof(int64_t), hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_block_bounds, dim3((unsigned)((nblocks + kBlock - 1) / kBlock)), dim3(kBlock), 0,
-                     s, d->sorted_val, bf_slot_d, bl_slot_d, nblocks, bfirst_d, blast_d);
-  RTS_TRY(hipGetLastError());
-  RTS_TRY(hipMemcpyAsync(d->block_first.data(), bfirst_d, nblocks * sizeof(CODE), hipMemcpyDeviceToHost, s));
-  RTS_TRY(hipMemcpyAsync(d->block_last.data(), blast_d, nblocks * sizeof(CODE), hipMemcpyDeviceToHost, s));
   RTS_TRY(hipStreamSynchronize(s));
-  RTS_TRY(rank_samples(d, s));
 
   describe(bx, d, col);
   d = nullptr;
@@ -686,9 +735,7 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
 fail:
   {
     const bool idle = hipStreamSynchronize(s) == hipSuccess;  // before other calls get the workspaces
-    for (void *p : {sort_tmp, (void *)counts, (void *)keys, tmp, (void *)starts_d,
-                    (void *)estarts_d, (void *)light_d, (void *)idx_d, (void *)bf_slot_d, (void *)bl_slot_d,
-                    (void *)bfirst_d, (void *)blast_d})
+    for (void *p : {sort_tmp, (void *)counts, (void *)keys, tmp, (void *)head_d, (void *)tail_d})
       pool_free(p, idle);
   }
   if (d) {

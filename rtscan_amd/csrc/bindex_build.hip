@@ -111,94 +111,166 @@ __global__ void k_rank_samples(const CODE *sorted, int64_t m, CODE *out) {
   if (i < m) out[i] = sorted[i * kRankSample];
 }
 
+// 2 i + (v >= t), in two instructions.
+__device__ __forceinline__ uint32_t descend(uint32_t i, uint32_t v, uint32_t t) {
+  asm("v_cmp_ge_u32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(i) : "v"(v), "v"(t) : "vcc");
+  return i;
+}
+
+// Eight bytes, x = rows 0 to 3 and y = 4 to 7 from the top byte down, as an 8 x 8 bit matrix
+// transposed: then byte 3 - k of x (k < 4) and byte 7 - k of y hold bit 7 - k of the rows,
+// row 0 topmost.
+__device__ __forceinline__ void transpose8(uint32_t &x, uint32_t &y) {
+  uint32_t t = (x ^ x >> 7) & 0x00AA00AAu;
+  x ^= t ^ t << 7;
+  t = (y ^ y >> 7) & 0x00AA00AAu;
+  y ^= t ^ t << 7;
+  t = (x ^ x >> 14) & 0x0000CCCCu;
+  x ^= t ^ t << 14;
+  t = (y ^ y >> 14) & 0x0000CCCCu;
+  y ^= t ^ t << 14;
+  t = (x & 0xF0F0F0F0u) | (y >> 4 & 0x0F0F0F0Fu);
+  y = (x << 4 & 0xF0F0F0F0u) | (y & 0x0F0F0F0Fu);
+  x = t;
+}
+
 // One pass over the column: all bins-1 filter vectors (fv[k] bit i = x_i < estart[k+1],
 // set_fv_val_less, bindex.cpp:553-560) and each row's list key (its bin if estart[bin] <
 // x, or x = estart[bin] with light[bin] set, else `bins` = in no list).  A wave takes 2048
-// consecutive rows, 64 words of every filter vector: lane l the 32 rows of word l.  The
-// lane finds its rows' bins t (binary search in LDS) and keeps them bit-sliced: NB words,
-// word b holding bit b of the 32 rows' t, MSB-first like the bitmaps.  Then for each k,
-// fv[k] = fv[k - 1] | {rows with t = k}, the equality taken over the NB slices (two
-// instructions a slice), and the 64 lanes store their words with one instruction.  A row
-// past n has t = bins, in no filter vector; the words past the last (up to the 64-word
-// padded stride) are written as zeros.  NB = bits of `bins` + 1 (t <= bins).
+// consecutive rows, 64 words of every filter vector.  Each lane finds the bins t of 32 rows
+// (a search of M levels in LDS, the rows' chains side by side; rows 256 j + 4 lane + i, so
+// that loads and the keys' stores are consecutive over the lanes), which go through LDS to
+// the lane that makes their word, and are transposed there into M bit slices, MSB-first like
+// the bitmaps.  With t = 16 h + l, fv[16 h + l] = (rows below h) | (rows of h) & (rows of at
+// most l): one instruction a word once the 16 words of l and those of h are made.  A row past
+// n is in no filter vector; the words past the last (up to the 64-word padded stride) are
+// written as zeros.
+//
+// Bound by the writes (1e8 rows, 128 bins: 1.6 GB of filter vectors, 0.2 of keys, 438 us).  Taking
+// each fv[k] from all M slices, a search loop a row and the slices a bit at a time cost 170
+// instructions a row, and 620 us; now 50.  1e6 rows, 256 bins: 44 -> 14 us.
 constexpr int kFvTileRows = 2048;
-template <int NB>
-__global__ __launch_bounds__(kBlock) void k_build_fvs(const CODE *col, int64_t n,
-                                                      const CODE *starts_g, const uint8_t *light_g,
-                                                      int bins, BITS *fvs, int64_t fv_stride,
+template <int M>
+__global__ __launch_bounds__(kBlock) void k_build_fvs(const CODE *col, int64_t n, const CODE *starts,
+                                                      const uint8_t *light, BITS *fvs, int64_t fv_stride,
                                                       uint16_t *keys) {
-  __shared__ CODE starts[kMaxBins];
-  __shared__ uint8_t light[kMaxBins];
-  for (int i = threadIdx.x; i < bins; i += blockDim.x) {
-    starts[i] = starts_g[i];
-    light[i] = light_g[i];
+  constexpr int kBins = 1 << M;
+  __shared__ uint32_t tree[kBins];   // [1, kBins): starts but the first, breadth-first
+  __shared__ CODE unlisted[kBins];   // the value of the bin that is in no list, or one that isn't in the bin
+  __shared__ alignas(16) uint16_t xch[kBlock / kWave][kFvTileRows];
+  for (int i = threadIdx.x; i < kBins; i += kBlock) {
+    // a light start's bin holds no value below it, nor (a start of 0) 2^32 - 1, the last bin's
+    unlisted[i] = light[i] ? starts[i] - 1 : starts[i];
+    if (i) {
+      const int level = 31 - __clz(i);
+      tree[i] = starts[(2 * (i - (1 << level)) + 1) << (M - 1 - level)];
+    }
   }
   __syncthreads();
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t wave = (int64_t)blockIdx.x * (kBlock / kWave) + threadIdx.x / kWave;
-  const int64_t nwaves = (int64_t)gridDim.x * (kBlock / kWave);
+  const int lane = threadIdx.x & (kWave - 1), wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  uint16_t *const xw = xch[wv];
+  const int64_t wave = (int64_t)blockIdx.x * (kBlock / kWave) + wv, nwaves = (int64_t)gridDim.x * (kBlock / kWave);
   const int64_t ntiles = (n + kFvTileRows - 1) / kFvTileRows;
-  const bool aligned = ((uintptr_t)col & 15) == 0;  // 16-byte loads of the column
+  const uint32_t root = tree[1], node2 = tree[2], node3 = tree[3];
   for (int64_t tile = wave; tile < ntiles; tile += nwaves) {
-    const int64_t r0 = tile * kFvTileRows + 32 * lane;  // this lane's 32 rows
-    uint32_t slice[NB];
+    const int64_t row0 = tile * kFvTileRows;
+    const bool whole = row0 + kFvTileRows <= n;
+    CODE x[32];
+    if (whole && ((uintptr_t)col & 15) == 0) {
+      const uint4 *src = reinterpret_cast<const uint4 *>(col + row0) + lane;
 #pragma unroll
-    for (int b = 0; b < NB; b++) slice[b] = 0;
-    const bool whole = r0 + 32 <= n;
-    uint32_t kw[16];  // the 32 rows' keys, two per word
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-      uint4 v = make_uint4(0, 0, 0, 0);
-      if (whole && aligned) {
-        v = *reinterpret_cast<const uint4 *>(col + r0 + 4 * q);
-      } else {
-        if (r0 + 4 * q < n) v.x = col[r0 + 4 * q];
-        if (r0 + 4 * q + 1 < n) v.y = col[r0 + 4 * q + 1];
-        if (r0 + 4 * q + 2 < n) v.z = col[r0 + 4 * q + 2];
-        if (r0 + 4 * q + 3 < n) v.w = col[r0 + 4 * q + 3];
+      for (int j = 0; j < 8; j++) {
+        const uint4 v = load_stream(src + 64 * j);
+        x[4 * j] = v.x, x[4 * j + 1] = v.y, x[4 * j + 2] = v.z, x[4 * j + 3] = v.w;
       }
-      const CODE xs[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int j = 4 * q + i;
-        const CODE x = xs[i];
-        int lo = 1, hi = bins;  // t = number of k in [1, bins-1] with start[k] <= x
-        while (lo < hi) {
-          const int mid = (lo + hi) >> 1;
-          if (starts[mid] <= x)
-            lo = mid + 1;
-          else
-            hi = mid;
-        }
-        const int t0 = lo - 1;
-        const bool valid = r0 + j < n;
-        const uint32_t t = valid ? (uint32_t)t0 : (uint32_t)bins;
-        const uint32_t key = starts[t0] < x || light[t0] ? (uint32_t)t0 : (uint32_t)bins;
-        if (j & 1)
-          kw[j / 2] |= key << 16;
-        else
-          kw[j / 2] = key;
-#pragma unroll
-        for (int b = 0; b < NB; b++) slice[b] = (slice[b] << 1) | ((t >> b) & 1u);
-      }
-    }
-    if (whole) {
-      uint4 *kd = reinterpret_cast<uint4 *>(keys + r0);
-#pragma unroll
-      for (int q = 0; q < 4; q++) kd[q] = make_uint4(kw[4 * q], kw[4 * q + 1], kw[4 * q + 2], kw[4 * q + 3]);
     } else {
 #pragma unroll
-      for (int j = 0; j < 32; j++)
-        if (r0 + j < n) keys[r0 + j] = (uint16_t)(kw[j / 2] >> (16 * (j & 1)));
+      for (int j = 0; j < 32; j++) x[j] = col[min(row0 + 256 * (j / 4) + 4 * lane + j % 4, n - 1)];
     }
-    BITS *dst = fvs + tile * (kFvTileRows / 32) + lane;
-    uint32_t acc = 0;  // fv[k] restricted to this lane's word
-    for (int k = 0; k < bins - 1; k++) {
+    uint32_t t[32];
+#pragma unroll
+    for (int j = 0; j < 32; j++) {
+      const bool up = x[j] >= root;
+      t[j] = descend(up ? 3 : 2, x[j], up ? node3 : node2);
+    }
+    for (int l = 2; l < M; l++) {
+#pragma unroll
+      for (int j = 0; j < 32; j++) t[j] = descend(t[j], x[j], tree[t[j]]);
+    }
+#pragma unroll
+    for (int j = 0; j < 32; j += 4) {
+      uint32_t key[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        t[j + i] -= kBins;
+        key[i] = x[j + i] != unlisted[t[j + i]] ? t[j + i] : (uint32_t)kBins;
+      }
+      const int at = 64 * j + 4 * lane;
+      const uint2 k4 = make_uint2(key[0] | key[1] << 16, key[2] | key[3] << 16);
+      if (whole) {
+        *reinterpret_cast<uint2 *>(keys + row0 + at) = k4;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (row0 + at + i < n) keys[row0 + at + i] = (uint16_t)key[i];
+      }
+      *reinterpret_cast<uint2 *>(xw + at) = make_uint2(t[j] | t[j + 1] << 16, t[j + 2] | t[j + 3] << 16);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wave's own exchange: LDS keeps its order
+    __builtin_amdgcn_wave_barrier();
+    // slices of the lane's 32 rows, in groups of eight
+    uint32_t part[4][2], slice[M], high[2] = {0, 0};
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      const uint4 v = reinterpret_cast<const uint4 *>(xw + 32 * lane)[g];  // rows 8 g + 1, 8 g, ...
+      part[g][0] = __builtin_amdgcn_perm(v.x, v.y, 0x04060002);
+      part[g][1] = __builtin_amdgcn_perm(v.z, v.w, 0x04060002);
+      transpose8(part[g][0], part[g][1]);
+      if (M > 8) {
+#pragma unroll
+        for (int b = 8; b < M; b++)
+          for (const uint32_t w : {v.x, v.y, v.z, v.w})
+            high[b - 8] = high[b - 8] << 2 | (w >> b & 1) << 1 | (w >> (16 + b) & 1);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int b = 0; b < M; b++) {
+      if (b < 8) {  // byte b % 4 of part[g][0] for the upper, [1] for the lower four bits; group 0 topmost
+        constexpr uint32_t kPair = 0x04000C0C;
+        const int h = b < 4;
+        const uint32_t sel = kPair + 0x01010000u * (b % 4);
+        slice[b] = __builtin_amdgcn_perm(part[0][h], part[1][h], sel) |
+                   __builtin_amdgcn_perm(part[2][h], part[3][h], 0x0C0C0400u + 0x0101u * (b % 4));
+      } else {
+        slice[b] = high[b - 8];
+      }
+    }
+    const int64_t left = n - row0 - 32 * lane;  // rows of the lane's word
+    const uint32_t valid = left >= 32 ? ~0u : left <= 0 ? 0u : ~0u << (32 - left);
+    uint32_t upto[16];  // rows with t % 16 <= l
+#pragma unroll
+    for (int l = 0; l < 16; l++) {
       uint32_t eq = ~0u;
 #pragma unroll
-      for (int b = 0; b < NB; b++) eq &= slice[b] ^ (((uint32_t)k >> b) & 1u ? 0u : ~0u);
-      acc |= eq;
-      dst[k * fv_stride] = acc;
+      for (int b = 0; b < 4; b++) eq &= l >> b & 1 ? slice[b] : ~slice[b];
+      upto[l] = l ? upto[l - 1] | eq : eq;
+    }
+    BITS *dst = fvs + tile * (kFvTileRows / 32);
+    uint32_t below = 0;  // rows with t / 16 < h
+#pragma unroll 1
+    for (int h = 0; h < kBins / 16; h++) {
+      uint32_t eq = valid;
+#pragma unroll
+      for (int b = 4; b < M; b++) eq &= slice[b] ^ (h >> (b - 4) & 1 ? 0u : ~0u);
+#pragma unroll
+      for (int l = 0; l < 16; l++) {
+        if (l < 15 || h < kBins / 16 - 1) dst[lane] = below | (eq & upto[l]);
+        dst += fv_stride;
+        asm volatile("" : "+s"(dst));  // one running address, not 16
+      }
+      below |= eq;
     }
   }
 }
@@ -644,18 +716,14 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   RTS_TRY(pool_alloc(&keys, n * sizeof(uint16_t)));
   {
     const dim3 grid(blocks_for((n + kFvTileRows - 1) / kFvTileRows, kBlock / kWave));
-    if (bins <= 128)
-      hipLaunchKernelGGL(k_build_fvs<8>, grid, dim3(kBlock), 0, s, col, n, head_d->estarts, head_d->light, bins, d->fvs,
-                         d->fv_stride, keys);
-    else if (bins <= 256)
-      hipLaunchKernelGGL(k_build_fvs<9>, grid, dim3(kBlock), 0, s, col, n, head_d->estarts, head_d->light, bins, d->fvs,
-                         d->fv_stride, keys);
-    else if (bins <= 512)
-      hipLaunchKernelGGL(k_build_fvs<10>, grid, dim3(kBlock), 0, s, col, n, head_d->estarts, head_d->light, bins, d->fvs,
-                         d->fv_stride, keys);
-    else
-      hipLaunchKernelGGL(k_build_fvs<11>, grid, dim3(kBlock), 0, s, col, n, head_d->estarts, head_d->light, bins, d->fvs,
-                         d->fv_stride, keys);
+#define RTS_BUILD_FVS(M)                                                                                        \
+  hipLaunchKernelGGL(k_build_fvs<M>, grid, dim3(kBlock), 0, s, col, n, head_d->estarts, head_d->light, d->fvs, \
+                     d->fv_stride, keys)
+    if (bins == 128) RTS_BUILD_FVS(7);
+    else if (bins == 256) RTS_BUILD_FVS(8);
+    else if (bins == 512) RTS_BUILD_FVS(9);
+    else RTS_BUILD_FVS(10);
+#undef RTS_BUILD_FVS
   }
   RTS_TRY(hipGetLastError());
 

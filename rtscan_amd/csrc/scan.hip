@@ -239,6 +239,38 @@ struct MultiPreds {
   uint64_t empty;              // bit p: predicate p matches no row
 };
 
+// Rows of the predicates of a launch.  A workgroup adds (1 << 44) | its rows to the predicate's
+// accumulator of its group (blockIdx.x % kMultiGroups); the one whose ticket completes the
+// group adds the group's rows to the predicate's last accumulator in the same way, and the
+// one that completes that writes the count; all accumulators are left at zero.  A second
+// kernel that summed the workgroups' rows took longer for every size: 64 predicates over 1e5
+// rows 10.6 -> 9.2 us, 2^20 11.1 -> 9.6, 8e6 25.7 -> 23.2, 1e8 292 -> 287.  One accumulator a
+// predicate (one group) is slower from 2^20 rows on (11.4, 8e6: 34.8), 4 to 32 groups are alike.
+constexpr int kMultiGroups = 16;
+constexpr size_t kMultiAccBytes = (size_t)(kMultiGroups + 1) * kMultiPreds * sizeof(unsigned long long);
+struct MultiSink {
+  unsigned long long *acc;  // per group, and once more, of each predicate
+  unsigned long long *counts;
+};
+__device__ __forceinline__ void multi_count(const MultiSink &sink, int p, uint32_t rows) {
+  constexpr unsigned long long kOne = 1ull << kCountTicketShift;
+  const unsigned g = blockIdx.x % kMultiGroups;
+  unsigned long long *acc = sink.acc + g * kMultiPreds + p;
+  unsigned long long old = atomicAdd(acc, kOne | rows);
+  if ((old >> kCountTicketShift) != (gridDim.x - g - 1) / kMultiGroups) return;
+  atomicExch(acc, 0ull);
+  const unsigned long long sum = (old & (kOne - 1)) + rows;
+  acc = sink.acc + kMultiGroups * kMultiPreds + p;
+  old = atomicAdd(acc, kOne | sum);
+  if ((old >> kCountTicketShift) + 1 != min(gridDim.x, (unsigned)kMultiGroups)) return;
+  sink.counts[p] = (old & (kOne - 1)) + sum;
+  atomicExch(acc, 0ull);
+}
+
+__global__ __launch_bounds__(kBlock) void k_zero_multi(unsigned long long *acc) {
+  for (size_t i = threadIdx.x; i < kMultiAccBytes / sizeof(*acc); i += kBlock) acc[i] = 0;
+}
+
 // Up to kMultiPreds closed ranges over one column in one pass.  A wave takes a tile of
 // 2048 rows, lane l the 32 rows of bitmap word l (eight 16-byte loads of its own 128 bytes;
 // the wave's loads cover the tile's 8 KB once), kept in registers; for every predicate p
@@ -249,12 +281,11 @@ struct MultiPreds {
 // wave step.  The predicates are split over gridDim.y groups of `pper` (workgroup y takes
 // [y * pper, y * pper + pper)), so that a short column still fills the device; the groups
 // read the same tiles, the later ones from L2.  COUNT: per-workgroup totals per predicate
-// (DPP wave totals added in LDS) into partials[p * gridDim.x + blockIdx.x], summed by
-// k_multi_counts.
+// (DPP wave totals added in LDS) into the sink.
 template <bool COUNT>
 __global__ __launch_bounds__(kBlock) void k_scan_multi(const uint32_t *col, uint64_t n, uint64_t ntiles,
                                                        MultiPreds mp, int np, int pper, BITS *out,
-                                                       uint64_t stride, uint32_t *partials) {
+                                                       uint64_t stride, MultiSink sink) {
   __shared__ uint32_t cnt[kMultiPreds];
   const int lane = threadIdx.x & (kWave - 1);
   const int pbeg = blockIdx.y * pper, pend = min(np, pbeg + pper);
@@ -311,7 +342,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_multi(const uint32_t *col, uint
   if (COUNT) {
     __syncthreads();
     if ((int)threadIdx.x >= pbeg && (int)threadIdx.x < pend)
-      partials[(uint64_t)threadIdx.x * gridDim.x + blockIdx.x] = cnt[threadIdx.x];
+      multi_count(sink, threadIdx.x, cnt[threadIdx.x]);
   }
 }
 
@@ -417,7 +448,7 @@ __device__ __forceinline__ void store_ranked_staged(uint32_t (&rank4)[8], const 
 template <int HALVES, bool COUNT, bool FULL, bool STAGED>
 __global__ __launch_bounds__(kBlock) void k_scan_ranked(const uint32_t *col, uint64_t n, uint64_t whole,
                                                         RankedPreds rp, int np, BITS *out, uint64_t stride,
-                                                        uint32_t run, uint32_t *partials) {
+                                                        uint32_t run, MultiSink sink) {
   __shared__ uint32_t tree[128];
   __shared__ uint32_t mask[HALVES][kRankEntries];
   __shared__ alignas(16) uint32_t xch[kBlock / kWave][kMultiTileRows / 4];
@@ -562,24 +593,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_ranked(const uint32_t *col, uin
     __syncthreads();
     const int p = 32 * half0 + (int)threadIdx.x;
     if (threadIdx.x < 32 * HALVES && p < np)
-      partials[(uint64_t)p * gridDim.x + blockIdx.x] = below[rp.r1[p]] - below[rp.r0[p]];
-  }
-}
-
-// counts[p] = sum of partials[p * nblocks .. + nblocks); one workgroup per predicate.
-__global__ __launch_bounds__(kBlock) void k_multi_counts(const uint32_t *partials, unsigned nblocks,
-                                                         unsigned long long *counts) {
-  __shared__ unsigned long long part[kBlock / kWave];
-  const uint32_t *src = partials + (uint64_t)blockIdx.x * nblocks;
-  unsigned long long s = 0;
-  for (unsigned i = threadIdx.x; i < nblocks; i += kBlock) s += src[i];
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, kWave);
-  if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x / kWave] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long t = 0;
-    for (int i = 0; i < kBlock / kWave; i++) t += part[i];
-    counts[blockIdx.x] = t;
+      multi_count(sink, p, below[rp.r1[p]] - below[rp.r0[p]]);
   }
 }
 
@@ -758,7 +772,7 @@ static RankedPreds rank_table(const CODE *lo, const CODE *hi, int np) {
 
 template <int HALVES>
 static void launch_ranked(const uint32_t *col, uint64_t n, const RankedPreds &t, int np, BITS *out, uint64_t stride,
-                          uint32_t run, uint32_t *partials, dim3 grid, hipStream_t s) {
+                          uint32_t run, const MultiSink &sink, dim3 grid, hipStream_t s) {
   const bool full = np == 32 * HALVES * (int)grid.y;
   const bool staged = ((uintptr_t)out % 128 || stride * sizeof(BITS) % 128) &&
                       (uint64_t)np * words_for_rows(n) * sizeof(BITS) >= kStagedBytes;
@@ -766,7 +780,7 @@ static void launch_ranked(const uint32_t *col, uint64_t n, const RankedPreds &t,
   const uint64_t tiles = aligned16(col) ? n / kMultiTileRows : 0, whole = staged ? tiles / (kBlock / kWave) * (kBlock / kWave) : tiles;
   auto go = [&](auto count, auto full, auto staged) {
     k_scan_ranked<HALVES, decltype(count)::value, decltype(full)::value, decltype(staged)::value>
-        <<<grid, kBlock, 0, s>>>(col, n, whole, t, np, out, stride, run, partials);
+        <<<grid, kBlock, 0, s>>>(col, n, whole, t, np, out, stride, run, sink);
   };
   auto pick = [&](auto count) {
     constexpr std::true_type yes{};
@@ -776,20 +790,20 @@ static void launch_ranked(const uint32_t *col, uint64_t n, const RankedPreds &t,
     else
       full ? go(count, yes, no) : go(count, no, no);
   };
-  partials ? pick(std::true_type{}) : pick(std::false_type{});
+  sink.counts ? pick(std::true_type{}) : pick(std::false_type{});
 }
 
 // Predicates up to which a pass tests each one (k_scan_multi) instead of searching
 // (k_scan_ranked).  The search costs a row the same for any number of predicates up to 32 and
 // half as much again up to 64, a test three instructions a row and predicate; on a short
 // column the search's chain of dependent steps (one tile a wave) is what shows.  Measured,
-// counted, tests against search: 1e5 rows, 64 predicates 10.7 / 11.3 us; 2^19 rows, 33: 9.3 /
-// 10.3, 64: 11.1 / 10.2; 2^20 rows, 16: 8.7 / 9.3, 24: 10.8 / 10.0, 64: 15.5 / 11.0; 4.2e6
-// rows, 8: 11.3 / 11.6, 10: 12.2 / 12.4, 16: 15.9 / 12.7; 1e8 rows, 5: 100 / 103, 8: 116 /
-// 105, 16: 199 / 119, 32: 379 / 181, 64: 732 / 288 (259 when every bitmap starts on a
-// 128-byte line: what is left is the writes' rate).
+// counted, tests against search: 2^18 rows, 64 predicates 7.2 / 8.6 us; 2^19 rows, 33: 7.7 /
+// 8.9, 40: 9.2 / 9.0, 64: 9.4 / 8.8; 2^20 rows, 16: 7.1 / 8.2, 24: 9.3 / 8.8, 64: 13.7 / 9.6;
+// 4.2e6 rows, 8: 10.9 / 11.3, 10: 11.4 / 12.2, 12: 12.8 / 12.3, 16: 15.8 / 12.5; 1e8 rows, 5:
+// 95 / 99, 8: 110 / 100, 16: 194 / 117, 32: 374 / 172, 64: 730 / 281 (252 when every bitmap
+// starts on a 128-byte line: what is left is the writes' rate).
 static int direct_preds(uint64_t n) {
-  return n < (1u << 18) ? kMultiPreds : n < (1u << 20) ? 40 : n < (1u << 22) ? 16 : 8;
+  return n < 3u << 17 ? kMultiPreds : n < 1u << 20 ? 40 : n < 1u << 22 ? 16 : 8;
 }
 
 hipError_t scan_ranges(const CODE *col, uint64_t n, const CODE *lo, const CODE *hi, int np, BITS *out,
@@ -802,18 +816,23 @@ hipError_t scan_ranges(const CODE *col, uint64_t n, const CODE *lo, const CODE *
     return hipSuccess;
   }
   const unsigned cus = (unsigned)std::max(1, device_cu_count());
-  uint32_t *partials = nullptr;
+  MultiSink sink{};
   if (counts) {
-    void *pp = nullptr;
-    const hipError_t e = thread_scratch(kScratchMulti, s, (size_t)kMultiPreds * kMultiMaxGrid * sizeof(uint32_t), 0,
-                                        &pp, nullptr);
+    void *acc = nullptr;
+    bool created = false;
+    hipError_t e = thread_scratch(kScratchMulti, s, kMultiAccBytes, 0, &acc, nullptr, &created);
+    if (e == hipSuccess && created) {  // the kernels leave the accumulators at zero; new ones start there too
+      hipLaunchKernelGGL(k_zero_multi, dim3(1), dim3(kBlock), 0, s, static_cast<unsigned long long *>(acc));
+      e = hipGetLastError();
+    }
     if (e != hipSuccess) return e;
-    partials = static_cast<uint32_t *>(pp);
+    sink.acc = static_cast<unsigned long long *>(acc);
   }
   for (int p0 = 0; p0 < np; p0 += kMultiPreds) {  // one pass over the column per 64 predicates
     const int k = std::min(kMultiPreds, np - p0);
     BITS *o = out + (uint64_t)p0 * stride;
     unsigned grid;
+    if (counts) sink.counts = counts + p0;
     if (k > direct_preds(n)) {
       const RankedPreds t = rank_table(lo + p0, hi + p0, k);
       const uint64_t wgtiles = (n + kMultiTileRows * (kBlock / kWave) - 1) / (kMultiTileRows * (kBlock / kWave));
@@ -826,11 +845,11 @@ hipError_t scan_ranges(const CODE *col, uint64_t n, const CODE *lo, const CODE *
       grid = (grid + kScanXcds - 1) / kScanXcds * kScanXcds;
       const uint32_t run = large ? 16 : 1;
       if (k <= 32)
-        launch_ranked<1>(col, n, t, k, o, stride, run, partials, dim3(grid), s);
+        launch_ranked<1>(col, n, t, k, o, stride, run, sink, dim3(grid), s);
       else if (grid < cus * 2)  // the halves in workgroups of their own, so that a short column fills the device
-        launch_ranked<1>(col, n, t, k, o, stride, run, partials, dim3(grid, 2), s);
+        launch_ranked<1>(col, n, t, k, o, stride, run, sink, dim3(grid, 2), s);
       else
-        launch_ranked<2>(col, n, t, k, o, stride, run, partials, dim3(grid), s);
+        launch_ranked<2>(col, n, t, k, o, stride, run, sink, dim3(grid), s);
     } else {
       const uint64_t ntiles = aligned16(col) ? n / kMultiTileRows : 0;
       const uint64_t waves = std::max<uint64_t>(ntiles, (n - ntiles * kMultiTileRows + 63) / 64);
@@ -851,16 +870,12 @@ hipError_t scan_ranges(const CODE *col, uint64_t n, const CODE *lo, const CODE *
       const dim3 g2(grid, (unsigned)((k + pper - 1) / pper));
       if (counts)
         hipLaunchKernelGGL(k_scan_multi<true>, g2, dim3(kBlock), 0, s, col, n, ntiles, mp, k, pper, o, stride,
-                           partials);
+                           sink);
       else
         hipLaunchKernelGGL(k_scan_multi<false>, g2, dim3(kBlock), 0, s, col, n, ntiles, mp, k, pper, o, stride,
-                           nullptr);
+                           sink);
     }
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && counts) {
-      hipLaunchKernelGGL(k_multi_counts, dim3(k), dim3(kBlock), 0, s, partials, grid, counts + p0);
-      e = hipGetLastError();
-    }
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

@@ -66,7 +66,7 @@ def _check(eng, x, preds, offset=0, counted=True, pad=0):
         assert (got[:, words:] == 0xA5A5A5A5).all()
 
 
-@pytest.mark.parametrize("n", [(1 << 18) - 1, 1 << 18, (1 << 18) + 2047, (1 << 20) + 1])
+@pytest.mark.parametrize("n", [(1 << 18) - 1, (3 << 17) - 1, 3 << 17, (3 << 17) + 2047, (1 << 20) + 1])
 @pytest.mark.parametrize("npred", [17, 40, 41, 63, 64, 107])
 def test_many_ranges_sizes(eng, n, npred):
     x = _column(n, n)
@@ -83,7 +83,7 @@ def test_ranges_of_a_long_column(eng, npred):
 @pytest.mark.parametrize("offset", [1, 2, 3])
 @pytest.mark.parametrize("counted", [False, True])
 def test_many_ranges_of_an_unaligned_column(eng, offset, counted):
-    x = _column((1 << 18) + 77, offset)
+    x = _column((3 << 17) + 77, offset)
     _check(eng, x, _ranges(x, 64, offset), offset=offset, counted=counted)
 
 
@@ -129,3 +129,23 @@ def test_bitmaps_of_many_bytes_off_cache_lines(eng, n, npred, pad):
             assert np.array_equal(got[p, :words], pack_rows(interval_mask(x, lo, hi))), p
     if pad:
         assert (got[:, words:] == 0xA5A5A5A5).all()
+
+
+@pytest.mark.parametrize("npred", [1, 33, 64, 130])
+def test_counts_again_and_again_on_streams(eng, npred):
+    """Counts of launches of one to a few thousand workgroups, after each other on one stream and
+    in turn with another's: each finds the accumulators that the one before left."""
+    streams = [None, eng.Stream()]
+    for rep, n in enumerate([1, 700, 4097, 100_003, 1 << 20, 100_003, 9_000_001, 5, 1 << 20]):
+        x = _column(n, n % 1009)
+        preds = _ranges(x, npred, rep)
+        col = eng.DeviceBuffer.from_numpy(x)
+        words = (n + 31) // 32
+        out = eng.DeviceBuffer(4 * npred * words)
+        counts = [eng.DeviceBuffer(8 * npred).fill(0xFF) for _ in range(4)]
+        for i, c in enumerate(counts):
+            eng.scan_ranges(col, n, [p[0] for p in preds], [p[1] for p in preds], out, words, c, streams[i % 2])
+            streams[1].synchronize() if i % 2 else eng.synchronize()
+        want = [int(((x >= lo) & (x <= hi)).sum()) for lo, hi in preds]
+        for c in counts:
+            assert c.to_numpy(np.uint64, npred).tolist() == want, n

@@ -281,21 +281,22 @@ __global__ __launch_bounds__(kBlock) void k_build_fvs(const CODE *col, int64_t n
 // with their rows and gathering the values afterwards, a random 4-byte read a row, took 2.7
 // ms at 1e8 rows and 128 bins; this takes 0.5.)
 
-// counts[k * (ntiles + 1) + t] = rows of tile t with key k (k < bins), and 0 for t = ntiles.
-// One workgroup per tile, and one for the zeros; LDS adds, a count copy per wave.
+// counts[k * (ntiles + 1) + t] = rows of tile t of tile_rows rows with key k (k < bins), and 0
+// for t = ntiles.  One workgroup per tile, and one for the zeros; LDS adds, a count copy per
+// wave.
 __global__ __launch_bounds__(kBlock) void k_list_counts(const uint16_t *keys, int64_t n, int bins, int64_t ntiles,
-                                                        uint32_t *counts) {
+                                                        int tile_rows, uint32_t *counts) {
   extern __shared__ uint32_t cnt[];  // kBlock / kWave copies of bins + 1
   const int64_t t = blockIdx.x;
   const int copies = kBlock / kWave, per = bins + 1;
   for (int i = threadIdx.x; i < copies * per; i += kBlock) cnt[i] = 0;
   __syncthreads();
   uint32_t *mine = cnt + threadIdx.x / kWave * per;
-  const int64_t r0 = t * kTileRows, r1 = std::min<int64_t>(n, r0 + kTileRows);
-  if (r0 + kTileRows <= n) {
+  const int64_t r0 = t * tile_rows, r1 = std::min<int64_t>(n, r0 + tile_rows);
+  if (r0 + tile_rows <= n) {
     const uint4 *src = reinterpret_cast<const uint4 *>(keys + r0);  // 8 keys each
 #pragma unroll 4
-    for (int i = threadIdx.x; i < kTileRows / 8; i += kBlock) {
+    for (int i = threadIdx.x; i < tile_rows / 8; i += kBlock) {
       const uint4 v = src[i];
       for (const uint32_t w : {v.x, v.y, v.z, v.w}) {
         if ((int)(w & 0xFFFF) < bins) atomicAdd(&mine[w & 0xFFFF], 1u);
@@ -314,19 +315,18 @@ __global__ __launch_bounds__(kBlock) void k_list_counts(const uint16_t *keys, in
   }
 }
 
-// The entries (row, value) of `parts`-th parts of the directory tiles: workgroup -> part j of
-// tile t, in chunks of kPartRows rows.  In a chunk each wave takes kPartRows / waves rows, 64
+// The entries (row, value) of tiles of tile_rows rows with the directory `dir`, a workgroup a
+// tile, in chunks of kPartRows rows.  In a chunk each wave takes kPartRows / waves rows, 64
 // a step: a row's place among its wave's rows of the same key is the count so far (LDS, one
 // counter per key and wave) plus the lanes before it with the same key (NB ballots, one per
 // key bit).  The chunk is then laid out by key in LDS and written out in that order, so that
 // a bin's entries go to memory as one run (kPartRows / bins entries of 8 bytes) and in row
-// order.  parts > 1 (short columns, to fill the device) count the keys of the tile's rows
-// before theirs first.
+// order.
 constexpr int kPartRows = 4096;
 constexpr int kPartRowBits = 12;
 template <int NB>
 __global__ __launch_bounds__(kBlock) void k_list_entries(const CODE *col, const uint16_t *keys, int64_t n, int bins,
-                                                         int64_t ntiles, const uint32_t *bdir, int parts, uint2 *bent) {
+                                                         int64_t ntiles, int tile_rows, const uint32_t *dir, uint2 *bent) {
   constexpr int kWaves = kBlock / kWave, kSteps = kPartRows / kBlock, kPer = (1 << (NB - 1)) / kBlock + 1;
   extern __shared__ uint2 part_lds[];
   uint2 *const stage = part_lds;                                           // kPartRows entries
@@ -335,16 +335,9 @@ __global__ __launch_bounds__(kBlock) void k_list_entries(const CODE *col, const 
   uint32_t *const delta = next + bins;                                     // bins: entry - slot of the chunk
   __shared__ uint32_t wsum[kWaves];
   const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
-  const int64_t t = blockIdx.x / parts;
-  const int j = blockIdx.x % parts;
-  for (int k = threadIdx.x; k < bins; k += kBlock) next[k] = bdir[k * (ntiles + 1) + t];
-  const int64_t tile0 = t * kTileRows, part = kTileRows / parts;
-  const int64_t p0 = tile0 + j * part, p1 = std::min<int64_t>(n, p0 + part);
-  __syncthreads();
-  for (int64_t r = tile0 + threadIdx.x; r < std::min<int64_t>(p0, n); r += kBlock) {
-    const uint32_t k = keys[r];
-    if ((int)k < bins) atomicAdd(&next[k], 1u);
-  }
+  const int64_t t = blockIdx.x;
+  for (int k = threadIdx.x; k < bins; k += kBlock) next[k] = dir[k * (ntiles + 1) + t];
+  const int64_t p0 = t * tile_rows, p1 = std::min<int64_t>(n, p0 + tile_rows);
   for (int64_t c0 = p0; c0 < p1; c0 += kPartRows) {
     uint32_t key[kSteps], place[kSteps];
     CODE x[kSteps];
@@ -357,7 +350,7 @@ __global__ __launch_bounds__(kBlock) void k_list_entries(const CODE *col, const 
       x[i] = r < left ? col[c0 + r] : 0;
     }
     for (int i = threadIdx.x; i < kWaves * (bins + 1); i += kBlock) wcnt[i] = 0;
-    __syncthreads();  // also: the chunk before has been written out, the counts above are done
+    __syncthreads();  // also: the chunk before has been written out
     uint32_t *const mine = wcnt + wv * (bins + 1);
 #pragma unroll
     for (int i = 0; i < kSteps; i++) {
@@ -419,6 +412,14 @@ __global__ __launch_bounds__(kBlock) void k_list_entries(const CODE *col, const 
       bent[delta[v.x >> kPartRowBits] + e] = make_uint2((uint32_t)c0 + (v.x & (kPartRows - 1)), v.y);
     }
   }
+}
+
+// bdir[k * (ntiles + 1) + t] = the same of a directory of `parts` times the tiles.
+__global__ void k_thin_directory(const uint32_t *fine, int bins, int64_t ntiles, int parts, uint32_t *bdir) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= bins * (ntiles + 1)) return;
+  const int64_t k = i / (ntiles + 1), t = i % (ntiles + 1);
+  bdir[i] = fine[k * (ntiles * parts + 1) + t * parts];
 }
 
 // boff[k] = boff2[k] = the directory's first entry of bin k, for k in [0, bins] (its rows end at the next bin's).
@@ -676,8 +677,8 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   // few: copied with the head and moved on the host
   const bool tail_host = samples + 2 * max_blocks <= kStagedTail;
   int64_t nblocks = 0;
-  uint32_t nb = 0;
-  int bins = 0;
+  uint32_t nb = 0, *fine = nullptr;
+  int bins = 0, parts = 1;
   std::vector<int64_t> rk;
 
   if (!bx || !col || n < kAreas || n > 0x7FFFFFFFll || (sub != 1 && sub != 2 && sub != 4 && sub != 8))
@@ -727,17 +728,28 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   }
   RTS_TRY(hipGetLastError());
 
-  // 4. tile directory and B lists
+  // 4. tile directory and B lists.  A short column's tiles are cut into up to 8 parts, to fill the
+  //    device, with a directory of their own (1e6 rows, 256 bins: counts 19 -> 4 us, entries
+  //    40 -> 10, where the parts counted the rows of their tile before them themselves)
+  while (parts < kTileRows / kPartRows && n > (int64_t)kPartRows * parts && d->ntiles * parts < 4 * (int64_t)device_cu_count())
+    parts *= 2;
   {
-    const int64_t items = (int64_t)bins * (d->ntiles + 1);
-    RTS_TRY(pool_alloc(&d->bdir, items * sizeof(uint32_t)));
+    const int64_t tiles = d->ntiles * parts, items = (int64_t)bins * (tiles + 1);
+    RTS_TRY(pool_alloc(&d->bdir, (int64_t)bins * (d->ntiles + 1) * sizeof(uint32_t)));
+    if (parts > 1) RTS_TRY(pool_alloc(&fine, items * sizeof(uint32_t)));
+    uint32_t *const dir = parts > 1 ? fine : d->bdir;
     RTS_TRY(pool_alloc(&counts, items * sizeof(uint32_t)));
-    RTS_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, need, counts, d->bdir, items, s));
+    RTS_TRY(hipcub::DeviceScan::ExclusiveSum(nullptr, need, counts, dir, items, s));
     RTS_TRY(pool_alloc(&tmp, need));
-    hipLaunchKernelGGL(k_list_counts, dim3((unsigned)(d->ntiles + 1)), dim3(kBlock),
-                       kBlock / kWave * (bins + 1) * sizeof(uint32_t), s, keys, n, bins, d->ntiles, counts);
+    hipLaunchKernelGGL(k_list_counts, dim3((unsigned)(tiles + 1)), dim3(kBlock),
+                       kBlock / kWave * (bins + 1) * sizeof(uint32_t), s, keys, n, bins, tiles, kTileRows / parts, counts);
     RTS_TRY(hipGetLastError());
-    RTS_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, need, counts, d->bdir, items, s));
+    RTS_TRY(hipcub::DeviceScan::ExclusiveSum(tmp, need, counts, dir, items, s));
+    if (parts > 1) {
+      hipLaunchKernelGGL(k_thin_directory, dim3((unsigned)((bins * (d->ntiles + 1) + kBlock - 1) / kBlock)), dim3(kBlock),
+                         0, s, fine, bins, d->ntiles, parts, d->bdir);
+      RTS_TRY(hipGetLastError());
+    }
     RTS_TRY(pool_alloc(&d->boff, (bins + 1) * sizeof(uint32_t)));
     hipLaunchKernelGGL(k_bin_offsets, dim3((bins + 1 + kBlock - 1) / kBlock), dim3(kBlock), 0, s, d->bdir, d->ntiles,
                        bins, d->boff, head_d->boff);
@@ -759,14 +771,12 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
   mark_complete_bins(d, rk);
   RTS_TRY(pool_alloc(&d->bent, std::max<uint32_t>(nb, 1) * sizeof(uint2)));
   if (nb) {
-    // a workgroup a tile when that fills the device, else the tiles in up to 8 parts
-    int parts = 1;
-    while (parts < kTileRows / kPartRows && d->ntiles * parts < 4 * (int64_t)device_cu_count()) parts *= 2;
-    const dim3 grid((unsigned)(d->ntiles * parts));
+    const int64_t tiles = d->ntiles * parts;
+    const dim3 grid((unsigned)tiles);
     const size_t lds = kPartRows * sizeof(uint2) + (kBlock / kWave * (bins + 1) + 2 * bins) * sizeof(uint32_t);
 #define RTS_LIST_ENTRIES(NB)                                                                             \
-  hipLaunchKernelGGL(k_list_entries<NB>, grid, dim3(kBlock), lds, s, col, keys, n, bins, d->ntiles, d->bdir, \
-                     parts, d->bent)
+  hipLaunchKernelGGL(k_list_entries<NB>, grid, dim3(kBlock), lds, s, col, keys, n, bins, tiles, kTileRows / parts, \
+                     parts > 1 ? fine : d->bdir, d->bent)
     if (bins <= 128) RTS_LIST_ENTRIES(8);
     else if (bins <= 256) RTS_LIST_ENTRIES(9);
     else if (bins <= 512) RTS_LIST_ENTRIES(10);
@@ -803,7 +813,7 @@ hipError_t bindex_build(BinDex *bx, const CODE *col, int64_t n, CODE *owned, int
 fail:
   {
     const bool idle = hipStreamSynchronize(s) == hipSuccess;  // before other calls get the workspaces
-    for (void *p : {sort_tmp, (void *)counts, (void *)keys, tmp, (void *)head_d, (void *)tail_d})
+    for (void *p : {sort_tmp, (void *)counts, (void *)keys, tmp, (void *)fine, (void *)head_d, (void *)tail_d})
       pool_free(p, idle);
   }
   if (d) {

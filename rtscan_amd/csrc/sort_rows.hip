@@ -7,7 +7,7 @@
 // go through the same LDS one after the other, half the LDS of laying out pairs.  The first
 // pass reads no rows (a row's number is its place).  1e8 rows: 1.97 ms for uniform values,
 // 1.63 for one value (the library sort that this replaced: 3.0 ms); a pass moves its 1.6 GB
-// in 0.33 ms, at the rate of a copy, and counts in 0.11.  1e6 rows: 0.11 ms, by the launches.
+// in 0.33 ms, at the rate of a copy, and counts in 0.11.  1e6 rows: 0.08 ms, by the launches.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -20,29 +20,33 @@ namespace rts {
 namespace {
 
 constexpr int kDigits = 256, kDigitBits = 8;
-constexpr int kThreads = 512, kSteps = 16;  // of k_sort_move: rows per thread
-constexpr int kTile = kThreads * kSteps;
+constexpr int kThreads = 512;  // of k_sort_move
+constexpr int kSteps = 16;     // its rows per thread
+constexpr int tile_rows(int steps) { return kThreads * steps; }
 constexpr int kCountThreads = 256;
 constexpr int kCopies = 4;  // one / eight copies: 2.57 / 1.60 ms for 1e8 equal values, 1.91 / 2.04 for uniform ones
-constexpr unsigned kRun = 32;
+constexpr unsigned kRun = 32, kShortRun = 1;
 
 // Tile of a workgroup: workgroup b runs on XCD b % 8, and an XCD takes runs of kRun
 // neighbouring tiles, whose counts share lines and whose digits' runs join, so that these
 // lines are completed in one L2 (1e8 uniform rows 2.83 ms with neighbouring tiles on
 // different XCDs, 2.17 with runs of 8, 1.97 with runs of 32).
 constexpr unsigned kSortXcds = 8;
-__device__ __forceinline__ int64_t tile_of_block() {
+__device__ __forceinline__ int64_t tile_of_block(unsigned run) {
   const unsigned j = blockIdx.x / kSortXcds;
-  return (int64_t)(j / kRun) * (kSortXcds * kRun) + blockIdx.x % kSortXcds * kRun + j % kRun;
+  return (int64_t)(j / run) * (kSortXcds * run) + blockIdx.x % kSortXcds * run + j % run;
 }
 
-// counts[d * ntiles + t] = rows of tile t with digit d.  kCopies count arrays a wave, so that
-// the lanes of a skewed column do not all add to one address.
+// counts[d * ntiles + t], SHORT: counts[t * kDigits + d], = rows of tile t with digit d.
+// kCopies count arrays a wave, so that the lanes of a skewed column do not all add to one
+// address.
+template <int STEPS, bool SHORT>
 __global__ __launch_bounds__(kCountThreads) void k_sort_counts(const CODE *val, int64_t n, int shift, int64_t ntiles,
                                                                uint32_t *counts) {
-  constexpr int kArrays = kCountThreads / kWave * kCopies, kPad = kDigits + 1, kVec = kTile / 4 / kCountThreads;
+  constexpr int kArrays = kCountThreads / kWave * kCopies, kPad = kDigits + 1;
+  constexpr int kTile = tile_rows(STEPS), kVec = kTile / 4 / kCountThreads;
   __shared__ uint32_t cnt[kArrays * kPad];
-  const int64_t t = tile_of_block();
+  const int64_t t = tile_of_block(SHORT ? kShortRun : kRun);
   if (t >= ntiles) return;
   for (int i = threadIdx.x; i < kArrays * kPad; i += kCountThreads) cnt[i] = 0;
   __syncthreads();
@@ -66,7 +70,7 @@ __global__ __launch_bounds__(kCountThreads) void k_sort_counts(const CODE *val, 
     uint32_t c = 0;
 #pragma unroll
     for (int a = 0; a < kArrays; a++) c += cnt[a * kPad + d];
-    counts[d * ntiles + t] = c;
+    counts[SHORT ? t * kDigits + d : d * ntiles + t] = c;
   }
 }
 
@@ -79,8 +83,9 @@ struct RankLds {
 // place[i] = slot of the thread's row i (row w0 + i * kWave of the tile, below `left`) when
 // the tile's rows are laid out by digit.  Returns, for threads d below kDigits, the digit's
 // first slot.
-__device__ __forceinline__ uint32_t rank_tile(RankLds &l, CODE (&x)[kSteps], int shift, uint32_t w0, uint32_t left,
-                                              uint32_t (&place)[kSteps]) {
+template <int STEPS>
+__device__ __forceinline__ uint32_t rank_tile(RankLds &l, CODE (&x)[STEPS], int shift, uint32_t w0, uint32_t left,
+                                              uint32_t (&place)[STEPS]) {
   constexpr int kWaves = kThreads / kWave;
   const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
   const int d = threadIdx.x;  // the digit of threads below kDigits
@@ -90,7 +95,7 @@ __device__ __forceinline__ uint32_t rank_tile(RankLds &l, CODE (&x)[kSteps], int
   // it with the digit (one ballot a bit)
   uint32_t *const mine = l.wcnt[wv];
 #pragma unroll
-  for (int i = 0; i < kSteps; i++) {
+  for (int i = 0; i < STEPS; i++) {
     const uint32_t digit = (x[i] >> shift) & (kDigits - 1);
     const bool row = w0 + i * kWave < left;
     const uint64_t rows = __ballot(row);
@@ -135,45 +140,78 @@ __device__ __forceinline__ uint32_t rank_tile(RankLds &l, CODE (&x)[kSteps], int
   }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < kSteps; i++) place[i] += mine[(x[i] >> shift) & (kDigits - 1)];
+  for (int i = 0; i < STEPS; i++) place[i] += mine[(x[i] >> shift) & (kDigits - 1)];
   return first;
 }
 
+// For threads d below kDigits, the first place of digit d of tile t from all tiles' counts
+// (tile after tile): the rows of lower digits and, of the digit, of the tiles before.  Two
+// threads a digit; `lds`: 4 * kDigits + kDigits / kWave words.
+__device__ __forceinline__ uint32_t first_places(uint32_t *lds, const uint32_t *counts, int64_t ntiles, int64_t t) {
+  static_assert(kThreads == 2 * kDigits, "two threads a digit");
+  const int d = threadIdx.x % kDigits, h = threadIdx.x / kDigits, lane = threadIdx.x & (kWave - 1);
+  uint32_t before = 0, all = 0;
+#pragma unroll 8
+  for (int64_t u = h; u < ntiles; u += 2) {
+    const uint32_t c = counts[u * kDigits + d];
+    all += c;
+    before += u < t ? c : 0;
+  }
+  uint32_t *const part = lds + 2 * kDigits;
+  if (h) lds[d] = before, lds[kDigits + d] = all;
+  __syncthreads();
+  uint32_t upto = 0;
+  if (!h) {
+    before += lds[d];
+    all += lds[kDigits + d];
+    upto = all;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const uint32_t u = __shfl_up(upto, o, kWave);
+      if (lane >= o) upto += u;
+    }
+    if (lane == kWave - 1) part[d / kWave] = upto;
+  }
+  __syncthreads();
+  for (int w = 0; w < d / kWave; w++) before += part[w];
+  return before + upto - all;
+}
+
 // The rows of a tile to their places of this pass; places: the scanned counts, the first place
-// of each (digit, tile).
-template <bool FIRST>
+// of each (digit, tile), or, SHORT, the counts, from which the workgroup makes its own tile's.
+template <int STEPS, bool SHORT, bool FIRST>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_sort_move(
     const CODE *val, const uint32_t *pos, int64_t n, int shift, int64_t ntiles, const uint32_t *places, CODE *out_val,
     uint32_t *out_pos) {
-  constexpr int kWaves = kThreads / kWave;
+  constexpr int kWaves = kThreads / kWave, kTile = tile_rows(STEPS);
   __shared__ uint32_t stage[kTile];
   __shared__ RankLds rank;
   __shared__ uint32_t delta[kDigits];  // place - slot in the tile
   const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
   const int d = threadIdx.x;  // the digit of threads below kDigits
-  const int64_t t = tile_of_block();
+  const int64_t t = tile_of_block(SHORT ? kShortRun : kRun);
   if (t >= ntiles) return;
   const int64_t c0 = t * kTile;
   const uint32_t left = (uint32_t)min((int64_t)kTile, n - c0);
   const uint32_t w0 = wv * (kTile / kWaves) + lane;
-  CODE x[kSteps];
-  uint32_t p[kSteps], place[kSteps];
+  CODE x[STEPS];
+  uint32_t p[STEPS], place[STEPS];
 #pragma unroll
-  for (int i = 0; i < kSteps; i++) x[i] = w0 + i * kWave < left ? val[c0 + w0 + i * kWave] : 0;
-  const uint32_t first = d < kDigits ? places[d * ntiles + t] : 0;
+  for (int i = 0; i < STEPS; i++) x[i] = w0 + i * kWave < left ? val[c0 + w0 + i * kWave] : 0;
+  const uint32_t first = SHORT ? first_places(stage, places, ntiles, t) : d < kDigits ? places[d * ntiles + t] : 0;
   const uint32_t slot = rank_tile(rank, x, shift, w0, left, place);
   if (d < kDigits) delta[d] = first - slot;
 #pragma unroll
-  for (int i = 0; i < kSteps; i++)
+  for (int i = 0; i < STEPS; i++)
     if (w0 + i * kWave < left) stage[place[i]] = x[i];
   if (!FIRST) {
 #pragma unroll
-    for (int i = 0; i < kSteps; i++) p[i] = w0 + i * kWave < left ? pos[c0 + w0 + i * kWave] : 0;
+    for (int i = 0; i < STEPS; i++) p[i] = w0 + i * kWave < left ? pos[c0 + w0 + i * kWave] : 0;
   }
   __syncthreads();
-  uint32_t dest[kSteps];
+  uint32_t dest[STEPS];
 #pragma unroll
-  for (int i = 0; i < kSteps; i++) {
+  for (int i = 0; i < STEPS; i++) {
     const uint32_t e = threadIdx.x + i * kThreads;
     if (e < left) {
       const CODE v = stage[e];
@@ -183,26 +221,50 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(5))) v
   }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < kSteps; i++)
+  for (int i = 0; i < STEPS; i++)
     if (w0 + i * kWave < left) stage[place[i]] = FIRST ? (uint32_t)c0 + w0 + i * kWave : p[i];
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < kSteps; i++) {
+  for (int i = 0; i < STEPS; i++) {
     const uint32_t e = threadIdx.x + i * kThreads;
     if (e < left) out_pos[dest[i]] = stage[e];
   }
 }
 
-// Shorter columns are sorted by the library, which takes fewer launches for them (an encode of
-// 8193 rows 105 us against 128, of 1e5 rows 137 against 122, of 1e6 241 against 182).
-constexpr int64_t kLibraryRows = (int64_t)1 << 17;
+// Shorter columns are sorted by the library, which takes fewer launches for them (3e4 rows 39 us
+// against 44, 65536 41 against 37).
+constexpr int64_t kLibraryRows = (int64_t)1 << 16;
+// Up to this many rows a pass does without a scan, every workgroup adds up the counts of all
+// tiles instead, and the fewer the rows, the smaller are the tiles, so that they fill the
+// device.  Sorts of 200 thousand, 500 thousand, 1, 1.5, 2.1 and 3 million rows, us: tiles of
+// 2048 rows 49, 68, 102, 182, 261, 466; of 4096 60, 66, 81, 108, 120, 200; of 8192 78, 78, 93,
+// 99, 103, 140; with a scan 94, 103, 113, 114, 120, 134.
+constexpr int64_t kShortRows = (int64_t)1 << 21;
+int steps_of(int64_t n) { return n <= 1 << 18 ? 4 : n <= 5 << 18 ? 8 : kSteps; }
 
 __global__ void k_iota(uint32_t *p, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = i;
 }
 
-int64_t tiles_of(int64_t n) { return (n + kTile - 1) / kTile; }
+int64_t tiles_of(int64_t n) {
+  const int64_t rows = tile_rows(steps_of(n));
+  return (n + rows - 1) / rows;
+}
+
+// One pass without a scan.
+template <int STEPS>
+hipError_t short_pass(const CODE *v, const uint32_t *p, int64_t n, int shift, int64_t tiles, uint32_t *counts, CODE *ov,
+                      uint32_t *op, dim3 grid, hipStream_t s) {
+  hipLaunchKernelGGL((k_sort_counts<STEPS, true>), grid, dim3(kCountThreads), 0, s, v, n, shift, tiles, counts);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  if (p)
+    hipLaunchKernelGGL((k_sort_move<STEPS, true, false>), grid, dim3(kThreads), 0, s, v, p, n, shift, tiles, counts, ov, op);
+  else
+    hipLaunchKernelGGL((k_sort_move<STEPS, true, true>), grid, dim3(kThreads), 0, s, v, p, n, shift, tiles, counts, ov, op);
+  return hipGetLastError();
+}
 
 size_t up16(size_t b) { return (b + 15) & ~(size_t)15; }
 
@@ -238,7 +300,8 @@ hipError_t sort_rows(const CODE *col, int64_t n, CODE *val, uint32_t *pos, void 
     return hipcub::DeviceRadixSort::SortPairs(static_cast<char *>(work) + up16(n * sizeof(uint32_t)), need, col, val,
                                               iota, pos, (int)n, 0, 32, s);
   }
-  const dim3 grid((unsigned)((tiles + kSortXcds * kRun - 1) / (kSortXcds * kRun) * (kSortXcds * kRun)));
+  const unsigned round = kSortXcds * (n <= kShortRows ? kShortRun : kRun);
+  const dim3 grid((unsigned)((tiles + round - 1) / round * round));
   char *w = static_cast<char *>(work);
   auto take = [&w](size_t bytes) {
     char *p = w;
@@ -256,16 +319,25 @@ hipError_t sort_rows(const CODE *col, int64_t n, CODE *val, uint32_t *pos, void 
     const int shift = pass * kDigitBits;
     CODE *const ov = pass & 1 ? val : wval;
     uint32_t *const op = pass & 1 ? pos : wpos;
-    hipLaunchKernelGGL(k_sort_counts, grid, dim3(kCountThreads), 0, s, v, n, shift, tiles, counts);
-    hipError_t e = hipGetLastError();
-    size_t need = scan;
-    if (e == hipSuccess) e = hipcub::DeviceScan::ExclusiveSum(w, need, counts, places, tiles * kDigits, s);
-    if (e != hipSuccess) return e;
-    if (pass == 0)
-      hipLaunchKernelGGL(k_sort_move<true>, grid, dim3(kThreads), 0, s, v, p, n, shift, tiles, places, ov, op);
-    else
-      hipLaunchKernelGGL(k_sort_move<false>, grid, dim3(kThreads), 0, s, v, p, n, shift, tiles, places, ov, op);
-    e = hipGetLastError();
+    hipError_t e;
+    if (n <= kShortRows) {
+      e = steps_of(n) == 4   ? short_pass<4>(v, p, n, shift, tiles, counts, ov, op, grid, s)
+          : steps_of(n) == 8 ? short_pass<8>(v, p, n, shift, tiles, counts, ov, op, grid, s)
+                             : short_pass<kSteps>(v, p, n, shift, tiles, counts, ov, op, grid, s);
+    } else {
+      hipLaunchKernelGGL((k_sort_counts<kSteps, false>), grid, dim3(kCountThreads), 0, s, v, n, shift, tiles, counts);
+      e = hipGetLastError();
+      size_t need = scan;
+      if (e == hipSuccess) e = hipcub::DeviceScan::ExclusiveSum(w, need, counts, places, tiles * kDigits, s);
+      if (e != hipSuccess) return e;
+      if (p)
+        hipLaunchKernelGGL((k_sort_move<kSteps, false, false>), grid, dim3(kThreads), 0, s, v, p, n, shift, tiles, places,
+                           ov, op);
+      else
+        hipLaunchKernelGGL((k_sort_move<kSteps, false, true>), grid, dim3(kThreads), 0, s, v, p, n, shift, tiles, places,
+                           ov, op);
+      e = hipGetLastError();
+    }
     if (e != hipSuccess) return e;
     v = ov;
     p = op;

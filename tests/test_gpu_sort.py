@@ -1,5 +1,5 @@
 """The value sort behind index builds and encoders against numpy's stable argsort, at the edges
-of its tiles and of the runs of tiles an XCD takes."""
+of its tiles, of the ranges that take tiles of one size, and of the runs of tiles an XCD takes."""
 import numpy as np
 import pytest
 
@@ -14,7 +14,8 @@ def _columns(n):
     yield "one", np.full(n, 0xFFFFFFFF, np.uint32)
 
 
-@pytest.mark.parametrize("n", [128, (1 << 17) - 1, 1 << 17, (1 << 17) + 1, 32 * 8192 - 1, 32 * 8192 + 1, 256 * 8192 + 5, 3_000_001])
+@pytest.mark.parametrize("n", [128, (1 << 16) - 1, 1 << 16, (1 << 16) + 1, (1 << 17) + 1, (1 << 18) - 1, 1 << 18,
+                               (1 << 18) + 1, 5 << 18, (5 << 18) + 1, 1 << 21, (1 << 21) + 1, 256 * 8192 + 5, 3_000_001])
 @pytest.mark.parametrize("offset", [0, 3])
 def test_sorted_values_and_rows(eng, n, offset):
     for name, x in _columns(n):

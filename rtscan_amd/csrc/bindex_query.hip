@@ -41,10 +41,12 @@ struct QueryArgs {
   BoundDev hi[C];  // L(b + 1)
 };
 
+template <bool STREAM>
 __device__ __forceinline__ uint4 base_words(const BoundDev &b, int64_t w, int64_t words) {
   if (b.base == kBaseZero) return make_uint4(0, 0, 0, 0);
   if (b.base == kBaseOnes) return make_uint4(~0u, ~0u, ~0u, ~0u);
-  if (w + 3 < words) return *reinterpret_cast<const uint4 *>(b.fv + w);
+  const uint4 *whole = reinterpret_cast<const uint4 *>(b.fv + w);
+  if (w + 3 < words) return STREAM ? load_stream(whole) : *whole;
   uint4 v = make_uint4(0, 0, 0, 0);
   v.x = b.fv[w];
   if (w + 1 < words) v.y = b.fv[w + 1];
@@ -114,8 +116,9 @@ constexpr int kListU = 2;  // list entries per thread per list per round
 // A workgroup owns M directory tiles: TQ = M * kTileWords output words, kPer = TQ / kBlock
 // words per thread (4 or 8, one or two uint4 per filter vector).
 // With rank.sorted set, workgroup 0 writes the count by rank_count (one wave) and the
-// others take the tiles; COUNT (popcount of the stored words) is then false.
-template <int C, int MODE, bool COUNT, int M>
+// others take the tiles; COUNT (popcount of the stored words) is then false.  STREAM: filter
+// vectors and result non-temporal (kStreamBytes).
+template <int C, int MODE, bool COUNT, int M, bool STREAM>
 __global__ __launch_bounds__(kBlock) void k_bindex_query(QueryArgs<C> q, int64_t n, int64_t words,
                                                          int64_t ndir, BITS *out, bool out_vec,
                                                          CountSink sink, RankArgs rank) {
@@ -154,8 +157,8 @@ __global__ __launch_bounds__(kBlock) void k_bindex_query(QueryArgs<C> q, int64_t
       for (int k = 0; k < kVec; k++) {
         const int64_t w = t * TQ + k * kTileWords + lw;
         if (w < words) {
-          lo_w[c][k] = base_words(q.lo[c], w, words);
-          hi_w[c][k] = base_words(q.hi[c], w, words);
+          lo_w[c][k] = base_words<STREAM>(q.lo[c], w, words);
+          hi_w[c][k] = base_words<STREAM>(q.hi[c], w, words);
         }
       }
       lo_e[c][0] = lo_e[c][1] = hi_e[c][0] = hi_e[c][1] = 0;
@@ -230,7 +233,11 @@ __global__ __launch_bounds__(kBlock) void k_bindex_query(QueryArgs<C> q, int64_t
           if (w + j < words) v[j] &= out[w + j];
       }
       if (out_vec && w + 3 < words) {
-        *reinterpret_cast<uint4 *>(out + w) = make_uint4(v[0], v[1], v[2], v[3]);
+        const u32x4 y = {v[0], v[1], v[2], v[3]};
+        if (STREAM)
+          __builtin_nontemporal_store(y, reinterpret_cast<u32x4 *>(out + w));
+        else
+          *reinterpret_cast<u32x4 *>(out + w) = y;
       } else {
 #pragma unroll
         for (int j = 0; j < 4; j++)
@@ -271,7 +278,15 @@ static BoundDev make_bound(const rts_bindex_dev *d, const BoundSpec &s) {
 // 512).
 constexpr int64_t kWideQueryRows = (int64_t)1 << 24;
 
-template <int C, int MODE, int M>
+// Bytes of filter vectors and result from which on they pass the caches by: a query then finds
+// little there of the ones before, and the lists' entries and directories stay.  Distinct
+// queries, us, cached / streamed: 1e8 rows, 1 column, 128 bins 12.4 / 10.9, 512 bins 11.0 / 8.3,
+// 4 columns 29.2 / 26.9; 2e7 x 3 (17 MB) 8.8 / 8.2; 1.7e7 x 2 (10 MB) 6.8 / 6.4; 1.2e7 x 2 (7.5 MB)
+// 6.0 / 6.1; 6e6 x 2 (3.8 MB) 5.4 / 5.7.  The same query again and again: 1e8 x 1 10.0 / 7.6, x 3
+// 19.8 / 20.2.
+constexpr int64_t kStreamBytes = 9 << 20;
+
+template <int C, int MODE, int M, bool STREAM>
 static hipError_t launch_query_m(const QueryArgs<C> &q, const rts_bindex_dev *d, BITS *out,
                                  unsigned long long *count, const RankArgs &rank, hipStream_t s) {
   const bool vec = ((uintptr_t)out & 15) == 0;
@@ -279,18 +294,18 @@ static hipError_t launch_query_m(const QueryArgs<C> &q, const rts_bindex_dev *d,
   const unsigned grid = (unsigned)std::min<int64_t>(ntiles, (int64_t)device_cu_count() * 32);
   const CountSink none{nullptr, nullptr, nullptr};
   if (rank.sorted) {  // one more workgroup, for the count
-    hipLaunchKernelGGL((k_bindex_query<C, MODE, false, M>), dim3(grid + 1), dim3(kBlock), 0, s, q, d->n,
+    hipLaunchKernelGGL((k_bindex_query<C, MODE, false, M, STREAM>), dim3(grid + 1), dim3(kBlock), 0, s, q, d->n,
                        d->words, d->ntiles, out, vec, none, rank);
   } else if (count) {
     const CountSink sink = stream_count_sink(count, s);
     if (!sink.acc) return hipErrorOutOfMemory;
-    hipLaunchKernelGGL((k_bindex_query<C, MODE, true, M>), dim3(grid), dim3(kBlock), 0, s, q, d->n,
+    hipLaunchKernelGGL((k_bindex_query<C, MODE, true, M, STREAM>), dim3(grid), dim3(kBlock), 0, s, q, d->n,
                        d->words, d->ntiles, out, vec, sink, rank);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     return launch_count_finalize(sink, grid, s);
   } else {
-    hipLaunchKernelGGL((k_bindex_query<C, MODE, false, M>), dim3(grid), dim3(kBlock), 0, s, q, d->n,
+    hipLaunchKernelGGL((k_bindex_query<C, MODE, false, M, STREAM>), dim3(grid), dim3(kBlock), 0, s, q, d->n,
                        d->words, d->ntiles, out, vec, none, rank);
   }
   return hipGetLastError();
@@ -299,8 +314,12 @@ static hipError_t launch_query_m(const QueryArgs<C> &q, const rts_bindex_dev *d,
 template <int C, int MODE>
 static hipError_t launch_query(const QueryArgs<C> &q, const rts_bindex_dev *d, BITS *out,
                                unsigned long long *count, const RankArgs &rank, hipStream_t s) {
-  if (C <= 2 && d->n >= kWideQueryRows) return launch_query_m<C, MODE, 2>(q, d, out, count, rank, s);
-  return launch_query_m<C, MODE, 1>(q, d, out, count, rank, s);
+  const bool stream = d->words * (int64_t)sizeof(BITS) * (2 * C + 1) >= kStreamBytes;
+  if (C <= 2 && d->n >= kWideQueryRows)
+    return stream ? launch_query_m<C, MODE, 2, true>(q, d, out, count, rank, s)
+                  : launch_query_m<C, MODE, 2, false>(q, d, out, count, rank, s);
+  return stream ? launch_query_m<C, MODE, 1, true>(q, d, out, count, rank, s)
+                : launch_query_m<C, MODE, 1, false>(q, d, out, count, rank, s);
 }
 
 template <int C>

@@ -433,7 +433,7 @@ def bench_scan(args, R):
             "bindex_device_bytes": ix.device_bytes(),
             "ranges_in_passes": {
                 "call": "rts_scan_ranges: the 1000 predicates in 16 calls of up to 64, the "
-                        "column read once per call (k_scan_multi), no counts in the timed region",
+                        "column read once per call (k_scan_ranked), no counts in the timed region",
                 "ms_all_predicates": ms_multi / 2, "us_per_predicate": ms_multi / 2 / len(preds) * 1e3,
                 "row_predicates_per_s": n * len(preds) / (ms_multi / 2 / 1e3),
                 "roofline": {"bound": "hbm", "alg_bytes": multi_alg,
@@ -674,7 +674,7 @@ def bench_config1(R, n=1 << 20, reps=20):
                          "frac": alg / (us * 1e-6) / 1e9 / HBM_PEAK_GBS},
             "cpu_baseline": {"port": {"rows_per_s": done * n / secs, "cores": threads, "kind": "port"},
                              "reference_raw_scan": ref},
-            "one_pass": {"call": "rts_scan_ranges, all 64 ranges in one call (k_scan_multi + counts)",
+            "one_pass": {"call": "rts_scan_ranges, all 64 ranges in one call (k_scan_ranked, counted)",
                          "us_per_call": us_one, "us_per_query": us_one / len(preds),
                          "rows_per_s": n * len(preds) / (us_one * 1e-6),
                          "roofline": {"bound": "hbm", "alg_bytes": alg_one,

@@ -34,7 +34,7 @@ extern "C" {
  *   map_values / map_starts   device, room for n entries; the first *map_size receive the
  *                 distinct values and their start codes (encodeMap[column])
  *   map_size      host; written after the distinct values are counted (the call
- *                 synchronises the stream once for it; the last kernel stays queued).
+ *                 returns after the work has finished).
  * n must be in [1, 2^31 - 1]. */
 hipError_t rts_encode_column(const CODE *data, int64_t n, CODE encode_min, CODE encode_max, CODE *codes,
                              POSTYPE *sorted_pos, CODE *sorted_codes, CODE *map_values,

@@ -15,7 +15,7 @@
 // memory moves the columns and the bitmaps alone.  Launches, k_batch against this, us: 1e8
 // rows x 4, 1024 queries 7180 / 5250; 2^26 x 2, 64 queries 374 / 226 (its memory traffic
 // alone 210); 2e7 x 3, 333 queries 530 / 327; queries that no index serves, 1e8 x 4, 256:
-// 15500 / 1400.  plan_rank_groups says where the lines lie.
+// 15500 / 1400.  A batch takes the faster of the two by its estimates (plan_us, batch_us).
 #include <string.h>
 
 #include <algorithm>

@@ -4,8 +4,8 @@
 // The reference sorts on the host with an unstable parallel sort, builds the 127 filter
 // vectors with 127 host passes, then issues one cudaMalloc + cudaMemcpy per 3276-row block
 // (~30k per column at 1e8 rows).  Here everything stays on the device: one stable radix
-// sort of (value, row), a K-thread kernel for the area starts and one for the bin starts
-// (each area cut into `sub` equal-count bins), one pass over the column for all bins-1
+// sort of (value, row), one kernel for the area starts, the bin starts (each area cut into
+// `sub` equal-count bins) and their ranks, one pass over the column for all bins-1
 // filter vectors and the bin keys, and one stable partition of the rows by bin key for the
 // row-ordered B lists and their tile directory.
 #include <hipcub/hipcub.hpp>

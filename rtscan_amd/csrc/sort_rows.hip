@@ -5,9 +5,9 @@
 // memory, so the rows of a tile are laid out by digit in LDS first and each digit's go out
 // as one run (32 rows, 128 bytes, of a tile of 8192 with all digits in use).  Values and rows
 // go through the same LDS one after the other, half the LDS of laying out pairs.  The first
-// pass reads no rows (a row's number is its place).  1e8 rows: 1.97 ms for uniform values,
-// 1.63 for one value (the library sort that this replaced: 3.0 ms); a pass moves its 1.6 GB
-// in 0.33 ms, at the rate of a copy, and counts in 0.11.  1e6 rows: 0.08 ms, by the launches.
+// pass reads no rows (a row's number is its place).  1e8 rows: 1.85 ms for uniform values,
+// 1.58 for one value (the library sort that this replaced: 3.0 ms); a pass moves its 1.6 GB
+// in 0.33 ms, at the rate of a copy, and counts in 0.11.  1e6 rows: 0.07 ms, by the launches.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -20,17 +20,20 @@ namespace rts {
 namespace {
 
 constexpr int kDigits = 256, kDigitBits = 8;
-constexpr int kThreads = 512;  // of k_sort_move
-constexpr int kSteps = 16;     // its rows per thread
-constexpr int tile_rows(int steps) { return kThreads * steps; }
+// Workgroups of k_sort_move, and their rows a thread.  Twice the waves at half the rows of
+// 512 x 16, with as many rows in flight and shorter chains of ranking: 1e8 uniform rows 2.01 ->
+// 1.85 ms, 2e7 0.41 -> 0.40 (1024 x 10, x 12 and x 16: 1.87, 1.79, 2.25 and 0.39, 0.42, 0.52).
+constexpr int kThreads = 1024, kSteps = 8;
+constexpr int kShortThreads = 512;
 constexpr int kCountThreads = 256;
 constexpr int kCopies = 4;  // one / eight copies: 2.57 / 1.60 ms for 1e8 equal values, 1.91 / 2.04 for uniform ones
 constexpr unsigned kRun = 32, kShortRun = 1;
 
 // Tile of a workgroup: workgroup b runs on XCD b % 8, and an XCD takes runs of kRun
 // neighbouring tiles, whose counts share lines and whose digits' runs join, so that these
-// lines are completed in one L2 (1e8 uniform rows 2.83 ms with neighbouring tiles on
-// different XCDs, 2.17 with runs of 8, 1.97 with runs of 32).
+// lines are completed in one L2 (workgroups of 512, 1e8 uniform rows: 2.83 ms with neighbouring
+// tiles on different XCDs; of 1024: 1.99 with runs of 8, 1.85 with 32, 1.77 with 64, which make
+// 6e6 rows take 186 us against 166).
 constexpr unsigned kSortXcds = 8;
 __device__ __forceinline__ int64_t tile_of_block(unsigned run) {
   const unsigned j = blockIdx.x / kSortXcds;
@@ -40,11 +43,11 @@ __device__ __forceinline__ int64_t tile_of_block(unsigned run) {
 // counts[d * ntiles + t], SHORT: counts[t * kDigits + d], = rows of tile t with digit d.
 // kCopies count arrays a wave, so that the lanes of a skewed column do not all add to one
 // address.
-template <int STEPS, bool SHORT>
+template <int TILE, bool SHORT>
 __global__ __launch_bounds__(kCountThreads) void k_sort_counts(const CODE *val, int64_t n, int shift, int64_t ntiles,
                                                                uint32_t *counts) {
   constexpr int kArrays = kCountThreads / kWave * kCopies, kPad = kDigits + 1;
-  constexpr int kTile = tile_rows(STEPS), kVec = kTile / 4 / kCountThreads;
+  constexpr int kVec = TILE / 4 / kCountThreads;
   __shared__ uint32_t cnt[kArrays * kPad];
   const int64_t t = tile_of_block(SHORT ? kShortRun : kRun);
   if (t >= ntiles) return;
@@ -52,8 +55,8 @@ __global__ __launch_bounds__(kCountThreads) void k_sort_counts(const CODE *val, 
   __syncthreads();
   uint32_t *mine = cnt + (threadIdx.x / kWave * kCopies + threadIdx.x % kCopies) * kPad;
   auto add = [&](CODE v) { atomicAdd(&mine[(v >> shift) & (kDigits - 1)], 1u); };
-  const int64_t r0 = t * kTile;
-  if (r0 + kTile <= n && ((uintptr_t)val & 15) == 0) {
+  const int64_t r0 = t * TILE;
+  if (r0 + TILE <= n && ((uintptr_t)val & 15) == 0) {
     const uint4 *src = reinterpret_cast<const uint4 *>(val + r0) + threadIdx.x;
     uint4 v[kVec];
 #pragma unroll
@@ -61,7 +64,7 @@ __global__ __launch_bounds__(kCountThreads) void k_sort_counts(const CODE *val, 
 #pragma unroll
     for (int i = 0; i < kVec; i++) add(v[i].x), add(v[i].y), add(v[i].z), add(v[i].w);
   } else {
-    const int64_t r1 = min(n, r0 + kTile);
+    const int64_t r1 = min(n, r0 + TILE);
 #pragma unroll 8
     for (int64_t r = r0 + threadIdx.x; r < r1; r += kCountThreads) add(val[r]);
   }
@@ -75,21 +78,22 @@ __global__ __launch_bounds__(kCountThreads) void k_sort_counts(const CODE *val, 
 }
 
 // LDS of the ranking of a tile's rows by digit.
+template <int THREADS>
 struct RankLds {
-  uint32_t wcnt[kThreads / kWave][kDigits];
+  alignas(16) uint32_t wcnt[THREADS / kWave][kDigits];
   uint32_t part[kDigits / kWave];
 };
 
 // place[i] = slot of the thread's row i (row w0 + i * kWave of the tile, below `left`) when
 // the tile's rows are laid out by digit.  Returns, for threads d below kDigits, the digit's
 // first slot.
-template <int STEPS>
-__device__ __forceinline__ uint32_t rank_tile(RankLds &l, CODE (&x)[STEPS], int shift, uint32_t w0, uint32_t left,
+template <int THREADS, int STEPS>
+__device__ __forceinline__ uint32_t rank_tile(RankLds<THREADS> &l, CODE (&x)[STEPS], int shift, uint32_t w0, uint32_t left,
                                               uint32_t (&place)[STEPS]) {
-  constexpr int kWaves = kThreads / kWave;
+  constexpr int kWaves = THREADS / kWave;
   const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
   const int d = threadIdx.x;  // the digit of threads below kDigits
-  for (int i = threadIdx.x; i < kWaves * kDigits; i += kThreads) (&l.wcnt[0][0])[i] = 0;
+  for (int i = threadIdx.x; i < kWaves * kDigits; i += THREADS) (&l.wcnt[0][0])[i] = 0;
   __syncthreads();
   // a row's place among its wave's rows of the digit: the count so far plus the lanes before
   // it with the digit (one ballot a bit)
@@ -145,47 +149,63 @@ __device__ __forceinline__ uint32_t rank_tile(RankLds &l, CODE (&x)[STEPS], int 
 }
 
 // For threads d below kDigits, the first place of digit d of tile t from all tiles' counts
-// (tile after tile): the rows of lower digits and, of the digit, of the tiles before.  Two
-// threads a digit; `lds`: 4 * kDigits + kDigits / kWave words.
-__device__ __forceinline__ uint32_t first_places(uint32_t *lds, const uint32_t *counts, int64_t ntiles, int64_t t) {
-  static_assert(kThreads == 2 * kDigits, "two threads a digit");
-  const int d = threadIdx.x % kDigits, h = threadIdx.x / kDigits, lane = threadIdx.x & (kWave - 1);
-  uint32_t before = 0, all = 0;
-#pragma unroll 8
-  for (int64_t u = h; u < ntiles; u += 2) {
-    const uint32_t c = counts[u * kDigits + d];
-    all += c;
-    before += u < t ? c : 0;
+// (tile after tile): the rows of lower digits and, of the digit, of the tiles before.  A wave
+// adds up every kWaves-th tile, four digits a lane, with kPlaceTiles tiles' loads in flight:
+// their latency is what a pass over a short column waits for.
+template <int THREADS>
+__device__ __forceinline__ uint32_t first_places(uint32_t *lds, RankLds<THREADS> &l, const uint32_t *counts,
+                                                 int64_t ntiles, int64_t t) {
+  constexpr int kWaves = THREADS / kWave, kPlaceTiles = 16;
+  static_assert(kDigits == 4 * kWave, "four digits a lane");
+  const int d = threadIdx.x, lane = threadIdx.x & (kWave - 1), wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int tiles = (int)ntiles, own = (int)t;
+  uint4 before = make_uint4(0, 0, 0, 0), all = before;
+  const uint4 *src = reinterpret_cast<const uint4 *>(counts) + lane;
+  for (int u0 = wv; u0 < tiles; u0 += kWaves * kPlaceTiles) {
+    uint4 c[kPlaceTiles];
+#pragma unroll
+    for (int k = 0; k < kPlaceTiles; k++) {
+      const int u = u0 + k * kWaves;
+      c[k] = u < tiles ? src[(int64_t)u * kWave] : make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int k = 0; k < kPlaceTiles; k++) {
+      const uint32_t m = u0 + k * kWaves < own ? 0xFFFFFFFFu : 0;
+      all.x += c[k].x, all.y += c[k].y, all.z += c[k].z, all.w += c[k].w;
+      before.x += c[k].x & m, before.y += c[k].y & m, before.z += c[k].z & m, before.w += c[k].w & m;
+    }
   }
-  uint32_t *const part = lds + 2 * kDigits;
-  if (h) lds[d] = before, lds[kDigits + d] = all;
+  reinterpret_cast<uint4 *>(lds + wv * kDigits)[lane] = before;
+  reinterpret_cast<uint4 *>(l.wcnt[wv])[lane] = all;
   __syncthreads();
-  uint32_t upto = 0;
-  if (!h) {
-    before += lds[d];
-    all += lds[kDigits + d];
-    upto = all;
+  uint32_t first = 0, total = 0, upto = 0;
+  if (d < kDigits) {
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) first += lds[w * kDigits + d], total += l.wcnt[w][d];
+    upto = total;
 #pragma unroll
     for (int o = 1; o < kWave; o <<= 1) {
       const uint32_t u = __shfl_up(upto, o, kWave);
       if (lane >= o) upto += u;
     }
-    if (lane == kWave - 1) part[d / kWave] = upto;
+    if (lane == kWave - 1) l.part[d / kWave] = upto;
   }
   __syncthreads();
-  for (int w = 0; w < d / kWave; w++) before += part[w];
-  return before + upto - all;
+  if (d < kDigits)
+    for (int w = 0; w < d / kWave; w++) first += l.part[w];
+  return first + upto - total;
 }
 
 // The rows of a tile to their places of this pass; places: the scanned counts, the first place
 // of each (digit, tile), or, SHORT, the counts, from which the workgroup makes its own tile's.
-template <int STEPS, bool SHORT, bool FIRST>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(5))) void k_sort_move(
+template <int THREADS, int STEPS, bool SHORT, bool FIRST>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(5))) void k_sort_move(
     const CODE *val, const uint32_t *pos, int64_t n, int shift, int64_t ntiles, const uint32_t *places, CODE *out_val,
     uint32_t *out_pos) {
-  constexpr int kWaves = kThreads / kWave, kTile = tile_rows(STEPS);
-  __shared__ uint32_t stage[kTile];
-  __shared__ RankLds rank;
+  constexpr int kWaves = THREADS / kWave, kTile = THREADS * STEPS;
+  static_assert(!SHORT || kTile >= kWaves * kDigits, "first_places");
+  alignas(16) __shared__ uint32_t stage[kTile];
+  __shared__ RankLds<THREADS> rank;
   __shared__ uint32_t delta[kDigits];  // place - slot in the tile
   const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
   const int d = threadIdx.x;  // the digit of threads below kDigits
@@ -198,7 +218,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(5))) v
   uint32_t p[STEPS], place[STEPS];
 #pragma unroll
   for (int i = 0; i < STEPS; i++) x[i] = w0 + i * kWave < left ? val[c0 + w0 + i * kWave] : 0;
-  const uint32_t first = SHORT ? first_places(stage, places, ntiles, t) : d < kDigits ? places[d * ntiles + t] : 0;
+  const uint32_t first = SHORT ? first_places(stage, rank, places, ntiles, t) : d < kDigits ? places[d * ntiles + t] : 0;
   const uint32_t slot = rank_tile(rank, x, shift, w0, left, place);
   if (d < kDigits) delta[d] = first - slot;
 #pragma unroll
@@ -212,7 +232,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(5))) v
   uint32_t dest[STEPS];
 #pragma unroll
   for (int i = 0; i < STEPS; i++) {
-    const uint32_t e = threadIdx.x + i * kThreads;
+    const uint32_t e = threadIdx.x + i * THREADS;
     if (e < left) {
       const CODE v = stage[e];
       dest[i] = delta[(v >> shift) & (kDigits - 1)] + e;
@@ -226,7 +246,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(5))) v
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < STEPS; i++) {
-    const uint32_t e = threadIdx.x + i * kThreads;
+    const uint32_t e = threadIdx.x + i * THREADS;
     if (e < left) out_pos[dest[i]] = stage[e];
   }
 }
@@ -236,11 +256,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(5))) v
 constexpr int64_t kLibraryRows = (int64_t)1 << 16;
 // Up to this many rows a pass does without a scan, every workgroup adds up the counts of all
 // tiles instead, and the fewer the rows, the smaller are the tiles, so that they fill the
-// device.  Sorts of 200 thousand, 500 thousand, 1, 1.5, 2.1 and 3 million rows, us: tiles of
-// 2048 rows 49, 68, 102, 182, 261, 466; of 4096 60, 66, 81, 108, 120, 200; of 8192 78, 78, 93,
-// 99, 103, 140; with a scan 94, 103, 113, 114, 120, 134.
-constexpr int64_t kShortRows = (int64_t)1 << 21;
-int steps_of(int64_t n) { return n <= 1 << 18 ? 4 : n <= 5 << 18 ? 8 : kSteps; }
+// device.  Sorts of 200, 300, 500 thousand, 1, 1.4, 2, 3 and 4 million rows, us: tiles of 2048
+// rows 47, 50, 58, 95, 142, 211, 385, 619; of 4096 58, 52, 57, 69, 96, 107, 168, 238; of 8192
+// 71, 78, 69, 81, 101, 90, 119, 135; with a scan 93, 102, 96, 106, 122, 108, 128, 129.
+constexpr int64_t kShortRows = (int64_t)7 << 19;
+int short_steps(int64_t n) { return n <= 3 << 17 ? 4 : n <= 3 << 19 ? 8 : 16; }
 
 __global__ void k_iota(uint32_t *p, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -248,7 +268,7 @@ __global__ void k_iota(uint32_t *p, uint32_t n) {
 }
 
 int64_t tiles_of(int64_t n) {
-  const int64_t rows = tile_rows(steps_of(n));
+  const int64_t rows = n <= kShortRows ? kShortThreads * short_steps(n) : kThreads * kSteps;
   return (n + rows - 1) / rows;
 }
 
@@ -256,13 +276,15 @@ int64_t tiles_of(int64_t n) {
 template <int STEPS>
 hipError_t short_pass(const CODE *v, const uint32_t *p, int64_t n, int shift, int64_t tiles, uint32_t *counts, CODE *ov,
                       uint32_t *op, dim3 grid, hipStream_t s) {
-  hipLaunchKernelGGL((k_sort_counts<STEPS, true>), grid, dim3(kCountThreads), 0, s, v, n, shift, tiles, counts);
+  hipLaunchKernelGGL((k_sort_counts<kShortThreads * STEPS, true>), grid, dim3(kCountThreads), 0, s, v, n, shift, tiles, counts);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (p)
-    hipLaunchKernelGGL((k_sort_move<STEPS, true, false>), grid, dim3(kThreads), 0, s, v, p, n, shift, tiles, counts, ov, op);
+    hipLaunchKernelGGL((k_sort_move<kShortThreads, STEPS, true, false>), grid, dim3(kShortThreads), 0, s, v, p, n,
+                       shift, tiles, counts, ov, op);
   else
-    hipLaunchKernelGGL((k_sort_move<STEPS, true, true>), grid, dim3(kThreads), 0, s, v, p, n, shift, tiles, counts, ov, op);
+    hipLaunchKernelGGL((k_sort_move<kShortThreads, STEPS, true, true>), grid, dim3(kShortThreads), 0, s, v, p, n,
+                       shift, tiles, counts, ov, op);
   return hipGetLastError();
 }
 
@@ -321,21 +343,23 @@ hipError_t sort_rows(const CODE *col, int64_t n, CODE *val, uint32_t *pos, void 
     uint32_t *const op = pass & 1 ? pos : wpos;
     hipError_t e;
     if (n <= kShortRows) {
-      e = steps_of(n) == 4   ? short_pass<4>(v, p, n, shift, tiles, counts, ov, op, grid, s)
-          : steps_of(n) == 8 ? short_pass<8>(v, p, n, shift, tiles, counts, ov, op, grid, s)
-                             : short_pass<kSteps>(v, p, n, shift, tiles, counts, ov, op, grid, s);
+      const int steps = short_steps(n);
+      e = steps == 4   ? short_pass<4>(v, p, n, shift, tiles, counts, ov, op, grid, s)
+          : steps == 8 ? short_pass<8>(v, p, n, shift, tiles, counts, ov, op, grid, s)
+                       : short_pass<16>(v, p, n, shift, tiles, counts, ov, op, grid, s);
     } else {
-      hipLaunchKernelGGL((k_sort_counts<kSteps, false>), grid, dim3(kCountThreads), 0, s, v, n, shift, tiles, counts);
+      hipLaunchKernelGGL((k_sort_counts<kThreads * kSteps, false>), grid, dim3(kCountThreads), 0, s, v, n, shift, tiles,
+                         counts);
       e = hipGetLastError();
       size_t need = scan;
       if (e == hipSuccess) e = hipcub::DeviceScan::ExclusiveSum(w, need, counts, places, tiles * kDigits, s);
       if (e != hipSuccess) return e;
       if (p)
-        hipLaunchKernelGGL((k_sort_move<kSteps, false, false>), grid, dim3(kThreads), 0, s, v, p, n, shift, tiles, places,
-                           ov, op);
+        hipLaunchKernelGGL((k_sort_move<kThreads, kSteps, false, false>), grid, dim3(kThreads), 0, s, v, p, n, shift,
+                           tiles, places, ov, op);
       else
-        hipLaunchKernelGGL((k_sort_move<kSteps, false, true>), grid, dim3(kThreads), 0, s, v, p, n, shift, tiles, places,
-                           ov, op);
+        hipLaunchKernelGGL((k_sort_move<kThreads, kSteps, false, true>), grid, dim3(kThreads), 0, s, v, p, n, shift,
+                           tiles, places, ov, op);
       e = hipGetLastError();
     }
     if (e != hipSuccess) return e;

@@ -15,7 +15,8 @@ def _columns(n):
 
 
 @pytest.mark.parametrize("n", [128, (1 << 16) - 1, 1 << 16, (1 << 16) + 1, (1 << 17) + 1, (1 << 18) - 1, 1 << 18,
-                               (1 << 18) + 1, 5 << 18, (5 << 18) + 1, 1 << 21, (1 << 21) + 1, 256 * 8192 + 5, 3_000_001])
+                               (1 << 18) + 1, 5 << 18, (5 << 18) + 1, 1 << 21, (1 << 21) + 1, 256 * 8192 + 5, 3_000_001,
+                               3 << 17, (3 << 17) + 1, 3 << 19, (3 << 19) + 1, 7 << 19, (7 << 19) + 1])
 @pytest.mark.parametrize("offset", [0, 3])
 def test_sorted_values_and_rows(eng, n, offset):
     for name, x in _columns(n):

@@ -222,12 +222,13 @@ constexpr int kMultiLaneRows = 32;                      // rows per lane: one bi
 constexpr int kMultiTileRows = kWave * kMultiLaneRows;  // 2048 rows per wave tile
 constexpr unsigned kMultiMaxGrid = 4096;
 
-constexpr int kStaged = 8;               // predicates whose words pass through LDS at once
+constexpr int kStagedBlock = 512;         // threads of a workgroup whose words pass through LDS
+constexpr int kStaged = 8;                // predicates whose words do so at once
 // Bitmaps that do not start on cache lines: bytes of them from which on that pays.  In less
 // the parts of a line meet in the caches before they are written, and the barriers show (33
 // bitmaps of 5e7 rows, 206 MB, counted: 93 us without, 98 with); more is bound by the rate at
-// which partial lines are written: 64 bitmaps of 1e8 rows, 800 MB, 322 -> 286 us (259 when
-// they start on lines), 32, 400 MB, 197 -> 181; 64 of 2e8 rows 607 -> 517.
+// which partial lines are written: 64 bitmaps of 1e8 rows, 800 MB, 322 -> 268 us (250 when
+// they start on lines), 32, 400 MB, 197 -> 166; 64 of 2e8 rows 607 -> 500.
 constexpr uint64_t kStagedBytes = 320u << 20;
 constexpr uint32_t kHistEntries = 1024;  // row counts of a workgroup: all copies
 constexpr unsigned kScanXcds = 8;
@@ -360,7 +361,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_multi(const uint32_t *col, uint
 // predicates) in a register; the wave stores 64 consecutive words of each bitmap.  COUNT:
 // rows per range by LDS adds, which make each predicate's rows at the end (popcounts of the
 // words cost 180 us more at 64 predicates).  1e8 rows, 64 predicates, counted: 732 us by
-// testing each predicate, 288 this way, 176 of it when nothing is stored.
+// testing each predicate, 268 this way, 176 of it when nothing is stored.
 struct RankedPreds {
   uint32_t tree[128];             // [1, 2^levels): bounds but the smallest, breadth-first, padded with 2^32 - 1
   uint32_t mask[2][kRankEntries];  // predicates matching range r, 32 per half; the last entry is 0
@@ -401,13 +402,15 @@ __device__ __forceinline__ void store_ranked(uint32_t (&rank4)[8], const uint32_
 }
 
 // As store_ranked for a workgroup of whole tiles, in step: the waves' words pass through LDS,
-// so that one wave stores the workgroup's 1 KB of a predicate at once, and fewer cache lines
+// so that one wave stores the workgroup's 2 KB of a predicate at once, and fewer cache lines
 // are filled by several stores (256 bytes a store: 2.7 TB/s where the bitmaps do not start on
-// lines, 1 KB: 3.9).  Bitmaps at 16-byte offsets take non-temporal 16-byte stores (64 of 1e8
-// rows: 303 -> 286 us); 4-byte ones are slower non-temporal (322 -> 336).  w0: of wave 0.
+// lines, 1 KB: 3.9, 4 KB: 4.7).  64 / 32 predicates, workgroups of 256 (1 KB) and of 512: 1e8 rows
+// 280 / 173 and 268 / 166 us, 1e8 + 1 297 and 275, 2e8 511 and 500; 40 of 99,999,900 203 and 207.
+// Bitmaps at 16-byte offsets take non-temporal 16-byte stores (64 of 1e8 rows: 303 -> 286 us);
+// 4-byte ones are slower non-temporal (322 -> 336).  w0: of wave 0.
 template <int HALVES, bool FULL>
 __device__ __forceinline__ void store_ranked_staged(uint32_t (&rank4)[8], const uint32_t (&mask)[HALVES][kRankEntries],
-                                                    uint32_t (&words)[2][kStaged][kBlock], int half0, int np, BITS *out,
+                                                    uint32_t (&words)[2][kStaged][kStagedBlock], int half0, int np, BITS *out,
                                                     uint64_t stride, uint64_t w0, int wv, int lane) {
 #pragma unroll 1
   for (int h = 0; h < HALVES; h++) {
@@ -423,22 +426,25 @@ __device__ __forceinline__ void store_ranked_staged(uint32_t (&rank4)[8], const 
     int left = np - p0;
 #pragma unroll
     for (int k = 0; k < 32; k += kStaged) {
-      uint32_t(&buf)[kStaged][kBlock] = words[k / kStaged % 2];
+      uint32_t(&buf)[kStaged][kStagedBlock] = words[k / kStaged % 2];
 #pragma unroll
       for (int q = 0; q < kStaged; q++) buf[q][kWave * wv + lane] = a[31 - k - q];
       __syncthreads();
 #pragma unroll
-      for (int q = 0; q < kStaged; q += kBlock / kWave) {
+      for (int q = 0; q < kStaged; q += kStagedBlock / kWave) {
         if (FULL || left > 0) {
           if (vec) {
-            __builtin_nontemporal_store(reinterpret_cast<const u32x4 *>(buf[q + wv])[lane], reinterpret_cast<u32x4 *>(o) + lane);
+#pragma unroll
+            for (int j = 0; j < kStagedBlock / kWave / 4; j++)
+              __builtin_nontemporal_store(reinterpret_cast<const u32x4 *>(buf[q + wv])[kWave * j + lane],
+                                          reinterpret_cast<u32x4 *>(o) + kWave * j + lane);
           } else {
 #pragma unroll
-            for (int j = 0; j < kBlock / kWave; j++) o[kWave * j + lane] = buf[q + wv][kWave * j + lane];
+            for (int j = 0; j < kStagedBlock / kWave; j++) o[kWave * j + lane] = buf[q + wv][kWave * j + lane];
           }
         }
-        o += stride * (kBlock / kWave);
-        left -= kBlock / kWave;
+        o += stride * (kStagedBlock / kWave);
+        left -= kStagedBlock / kWave;
         asm volatile("" : "+s"(left));
       }
     }
@@ -446,13 +452,14 @@ __device__ __forceinline__ void store_ranked_staged(uint32_t (&rank4)[8], const 
 }
 
 template <int HALVES, bool COUNT, bool FULL, bool STAGED>
-__global__ __launch_bounds__(kBlock) void k_scan_ranked(const uint32_t *col, uint64_t n, uint64_t whole,
+__global__ __launch_bounds__(STAGED ? kStagedBlock : kBlock) void k_scan_ranked(const uint32_t *col, uint64_t n, uint64_t whole,
                                                         RankedPreds rp, int np, BITS *out, uint64_t stride,
                                                         uint32_t run, MultiSink sink) {
+  constexpr int B = STAGED ? kStagedBlock : kBlock;
   __shared__ uint32_t tree[128];
   __shared__ uint32_t mask[HALVES][kRankEntries];
-  __shared__ alignas(16) uint32_t xch[kBlock / kWave][kMultiTileRows / 4];
-  __shared__ alignas(16) uint32_t staged[2][kStaged][kBlock];
+  __shared__ alignas(16) uint32_t xch[B / kWave][kMultiTileRows / 4];
+  __shared__ alignas(16) uint32_t staged[2][kStaged][kStagedBlock];
   // rows per range (COUNT), in as many copies as fit (four for 64 predicates, one a lane for
   // four): a wave's rows of one range would otherwise add to one address one after another
   // (3 predicates over 2^25 rows, counted: 48 us with four copies)
@@ -462,10 +469,10 @@ __global__ __launch_bounds__(kBlock) void k_scan_ranked(const uint32_t *col, uin
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int half0 = HALVES == 1 ? blockIdx.y : 0;  // one half a workgroup: which one
   if (threadIdx.x < 128) tree[threadIdx.x] = rp.tree[threadIdx.x];
-  for (int i = threadIdx.x; i < HALVES * kRankEntries; i += kBlock)
+  for (int i = threadIdx.x; i < HALVES * kRankEntries; i += B)
     mask[i / kRankEntries][i % kRankEntries] = rp.mask[half0 + i / kRankEntries][i % kRankEntries];
   if (COUNT)
-    for (uint32_t i = threadIdx.x; i < kHistEntries; i += kBlock) hist[i] = 0;
+    for (uint32_t i = threadIdx.x; i < kHistEntries; i += B) hist[i] = 0;
   __syncthreads();
   const uint64_t words = words_for_rows(n), ntiles = (n + kMultiTileRows - 1) / kMultiTileRows;
   const uint32_t first = rp.first, root = rp.tree[1];
@@ -489,7 +496,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_ranked(const uint32_t *col, uin
   // in one L2
   const uint64_t xcd = blockIdx.x % kScanXcds, step0 = blockIdx.x / kScanXcds, steps = gridDim.x / kScanXcds;
   auto tile_of = [&](uint64_t i) {
-    return (i / run * run * kScanXcds + xcd * run + i % run) * (kBlock / kWave) + wv;
+    return (i / run * run * kScanXcds + xcd * run + i % run) * (B / kWave) + wv;
   };
   uint4 v[8];
   auto load = [&](uint64_t t) {
@@ -567,7 +574,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_ranked(const uint32_t *col, uin
   if (COUNT) {
     __syncthreads();
     // rows of each range over the copies, then rows below each range, then each predicate's
-    for (uint32_t r = threadIdx.x; r < kRankEntries; r += kBlock) {
+    for (uint32_t r = threadIdx.x; r < kRankEntries; r += B) {
       uint32_t a = 0;
       if (r <= top)
         for (uint32_t c = 0; c < rp.copies; c++) a += hist[c * rp.stride + r];
@@ -777,10 +784,14 @@ static void launch_ranked(const uint32_t *col, uint64_t n, const RankedPreds &t,
   const bool staged = ((uintptr_t)out % 128 || stride * sizeof(BITS) % 128) &&
                       (uint64_t)np * words_for_rows(n) * sizeof(BITS) >= kStagedBytes;
   // staged, a workgroup's waves go in step: whole tiles for all of them
-  const uint64_t tiles = aligned16(col) ? n / kMultiTileRows : 0, whole = staged ? tiles / (kBlock / kWave) * (kBlock / kWave) : tiles;
+  const uint64_t tiles = aligned16(col) ? n / kMultiTileRows : 0, whole = staged ? tiles / (kStagedBlock / kWave) * (kStagedBlock / kWave) : tiles;
+  if (staged) {
+    grid.x = (grid.x * kBlock / kStagedBlock + kScanXcds - 1) / kScanXcds * kScanXcds;
+    run = std::max<uint32_t>(1, run * kBlock / kStagedBlock);
+  }
   auto go = [&](auto count, auto full, auto staged) {
     k_scan_ranked<HALVES, decltype(count)::value, decltype(full)::value, decltype(staged)::value>
-        <<<grid, kBlock, 0, s>>>(col, n, whole, t, np, out, stride, run, sink);
+        <<<grid, decltype(staged)::value ? kStagedBlock : kBlock, 0, s>>>(col, n, whole, t, np, out, stride, run, sink);
   };
   auto pick = [&](auto count) {
     constexpr std::true_type yes{};
@@ -800,7 +811,7 @@ static void launch_ranked(const uint32_t *col, uint64_t n, const RankedPreds &t,
 // counted, tests against search: 2^18 rows, 64 predicates 7.2 / 8.6 us; 2^19 rows, 33: 7.7 /
 // 8.9, 40: 9.2 / 9.0, 64: 9.4 / 8.8; 2^20 rows, 16: 7.1 / 8.2, 24: 9.3 / 8.8, 64: 13.7 / 9.6;
 // 4.2e6 rows, 8: 10.9 / 11.3, 10: 11.4 / 12.2, 12: 12.8 / 12.3, 16: 15.8 / 12.5; 1e8 rows, 5:
-// 95 / 99, 8: 110 / 100, 16: 194 / 117, 32: 374 / 172, 64: 730 / 281 (252 when every bitmap
+// 95 / 99, 8: 110 / 100, 16: 194 / 117, 32: 374 / 166, 64: 730 / 268 (250 when every bitmap
 // starts on a 128-byte line: what is left is the writes' rate).
 static int direct_preds(uint64_t n) {
   return n < 3u << 17 ? kMultiPreds : n < 1u << 20 ? 40 : n < 1u << 22 ? 16 : 8;

@@ -27,6 +27,8 @@
 
 namespace rts {
 
+// Two workgroups of 256 a compute unit, one searching while the other stores (one of 512, with 2
+// KB a store: 1024 queries on 1e8 rows x 4 6280 us against 5270).
 constexpr int kRankThreads = 256, kRankWaves = kRankThreads / kWave, kRankPerCu = 2;  // workgroups
 constexpr int kRankTileRows = 2048;  // of a wave: lane l makes word l
 constexpr int kRankStepRows = kRankWaves * kRankTileRows, kRankStepWords = kRankStepRows / 32;

@@ -25,7 +25,9 @@
  * Launches of one plan must not overlap (use one stream per plan, or order them): they share
  * the plan's counters and partials.  rts_batch_plan_graph_launch captures them in a hipGraph
  * and replays it; queries set with rts_batch_plan_set_queries live in device memory at a fixed
- * address, so a replay, of a graph of the caller's own too, evaluates the current set.
+ * address, so a replay, of a graph of the caller's own too, evaluates the current set: every
+ * bitmap, and the counts of as many of its queries as there were at the capture (with fewer
+ * queries now, the other counts are left as they are).
  */
 #ifndef RTS_BATCH_H_
 #define RTS_BATCH_H_

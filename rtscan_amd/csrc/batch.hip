@@ -588,22 +588,28 @@ __global__ __launch_bounds__(kBlock) void k_batch_counts(const uint32_t *partial
 }
 
 // The same where queries may be evaluated together (`ranked`, per query): those have their sum
-// in rank_counts, which is left at zero for the next launch.
+// in rank_counts, which is left at zero for the next launch.  The queries that are set now need
+// not be those of a captured launch: it runs a workgroup for every query that the plan has room
+// for, so that all sums are cleared, and writes the counts of its first `out_nq` queries, as far
+// as they are set.
 __global__ __launch_bounds__(kBlock) void k_batch_counts_mixed(const uint32_t *partials, int64_t ntiles,
-                                                               const uint8_t *ranked,
-                                                               unsigned long long *rank_counts,
+                                                               const RankHeader *header,
+                                                               unsigned long long *rank_counts, unsigned out_nq,
                                                                unsigned long long *counts) {
   __shared__ unsigned long long part[kBlock / kWave];
+  const uint8_t *ranked = reinterpret_cast<const uint8_t *>(header + 1);
+  if (blockIdx.x >= (unsigned)header->nq) return;  // no launch adds to its sum
   unsigned long long s = 0;
   if (ranked[blockIdx.x]) {
     if (threadIdx.x == 0) {
       s = rank_counts[blockIdx.x];
       rank_counts[blockIdx.x] = 0;
     }
-  } else {
+  } else if (blockIdx.x < out_nq) {
     const uint32_t *p = partials + (int64_t)blockIdx.x * ntiles;
     for (int64_t i = threadIdx.x; i < ntiles; i += kBlock) s += p[i];
   }
+  if (blockIdx.x >= out_nq) return;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, kWave);
   if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x / kWave] = s;
@@ -691,10 +697,11 @@ struct rts_batch_plan {
   BatchGroup *d_groups = nullptr;  // max_queries records
   // One block of device memory, uploaded in one copy as far as a set of queries fills it:
   // the header, per query a byte that says whether it is evaluated together with others
-  // (k_batch_ranked), the groups of those; then their counts (zero between launches).
+  // (k_batch_ranked), the sums of those (zero between launches, and uploaded as zeros with
+  // queries that use them), their groups.
   uint8_t *d_plan = nullptr;
   std::vector<uint8_t> h_plan;
-  size_t rank_groups_at = 0, rank_counts_at = 0;
+  size_t rank_counts_at = 0, rank_groups_at = 0;
   int max_rank_groups = 0;
   bool has_ranked = false, has_bindex = false;  // the forms that the current queries need
   uint32_t *d_zero_dir = nullptr;  // ntiles + 1 zeros: the directory of an unused list
@@ -817,14 +824,15 @@ static int forms_needed(const rts_batch_plan *p) {
   return (p->has_bindex ? kFormBindex : 0) | (p->has_ranked ? kFormRanked : 0);
 }
 
+// captured: by the caller, who may set other queries, and more or fewer, before a replay.
 static hipError_t launch_batch(rts_batch_plan *p, BITS *out, int64_t out_stride, unsigned long long *counts, int forms,
-                               hipStream_t s) {
+                               bool captured, hipStream_t s) {
+  const auto *const header = reinterpret_cast<const RankHeader *>(p->d_plan);
   auto *const rank_counts = reinterpret_cast<unsigned long long *>(p->d_plan + p->rank_counts_at);
   hipError_t e = hipSuccess;
   if (forms & kFormRanked)
-    e = launch_rank_groups(reinterpret_cast<const RankGroup *>(p->d_plan + p->rank_groups_at),
-                           reinterpret_cast<const RankHeader *>(p->d_plan), p->n, out, out_stride,
-                           counts ? rank_counts : nullptr, s);
+    e = launch_rank_groups(reinterpret_cast<const RankGroup *>(p->d_plan + p->rank_groups_at), header, p->n, out,
+                           out_stride, counts ? rank_counts : nullptr, s);
   if (e == hipSuccess && (forms & kFormBindex)) {
     const bool small = p->cfg.threads == 256;
     switch (p->cfg.tile_words) {
@@ -839,14 +847,15 @@ static hipError_t launch_batch(rts_batch_plan *p, BITS *out, int64_t out_stride,
     }
     e = hipGetLastError();
   }
-  if (e != hipSuccess || !counts) return e;
-  if (forms & kFormRanked)
-    hipLaunchKernelGGL(k_batch_counts_mixed, dim3((unsigned)p->nq), dim3(kBlock), 0, s, p->d_partials, p->ntiles,
-                       p->d_plan + sizeof(RankHeader), rank_counts, counts);
-  else
+  if (!counts) return e;
+  if (forms & kFormRanked)  // also after an error, so that no sum is left for the next launch
+    hipLaunchKernelGGL(k_batch_counts_mixed, dim3((unsigned)(captured ? p->max_queries : p->nq)), dim3(kBlock), 0, s,
+                       p->d_partials, p->ntiles, header, rank_counts, (unsigned)p->nq, counts);
+  else if (e == hipSuccess)
     hipLaunchKernelGGL(k_batch_counts, dim3((unsigned)p->nq), dim3(kBlock), 0, s, p->d_partials, p->ntiles,
                        counts);
-  return hipGetLastError();
+  const hipError_t ce = hipGetLastError();
+  return e != hipSuccess ? e : ce;
 }
 
 // Query-columns a work item has toggle arrays for.
@@ -969,11 +978,10 @@ hipError_t rts_batch_plan_create(rts_batch_plan **out, const CODE *const *column
   p->index = p->index_sets[p->active_set].data();
   hipError_t e = device_malloc((void **)&p->d_groups, (size_t)max_queries * sizeof(BatchGroup));
   p->max_rank_groups = max_rank_groups(max_queries);
-  p->rank_groups_at = (sizeof(RankHeader) + (size_t)max_queries + 15) / 16 * 16;
-  p->rank_counts_at = p->rank_groups_at + (size_t)p->max_rank_groups * sizeof(RankGroup);
-  const size_t rank_counts = p->max_rank_groups ? (size_t)max_queries * sizeof(unsigned long long) : 0;
-  if (e == hipSuccess) e = device_malloc((void **)&p->d_plan, p->rank_counts_at + rank_counts);
-  if (e == hipSuccess && rank_counts) e = hipMemsetAsync(p->d_plan + p->rank_counts_at, 0, rank_counts, stream);
+  p->rank_counts_at = (sizeof(RankHeader) + (size_t)max_queries + 15) / 16 * 16;
+  p->rank_groups_at = (p->rank_counts_at + (size_t)max_queries * sizeof(unsigned long long) + 15) / 16 * 16;
+  if (e == hipSuccess)
+    e = device_malloc((void **)&p->d_plan, p->rank_groups_at + (size_t)p->max_rank_groups * sizeof(RankGroup));
   if (e == hipSuccess) e = device_malloc((void **)&p->d_sched, kSchedWords * sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMemsetAsync(p->d_sched, 0, kSchedWords * sizeof(unsigned long long), stream);
   if (e == hipSuccess) e = build_dirs(p, stream);
@@ -1267,10 +1275,13 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
   p->has_ranked = !rank_groups.empty();
   if (nq == 0) return hipSuccess;
   header.bindex_groups = p->ngroups;
-  p->h_plan.resize(p->rank_groups_at + rank_groups.size() * sizeof(RankGroup));
+  header.nq = nq;
+  p->h_plan.assign(p->has_ranked ? p->rank_groups_at + rank_groups.size() * sizeof(RankGroup)
+                                 : sizeof(header) + ranked.size(), 0);
   memcpy(p->h_plan.data(), &header, sizeof(header));
   memcpy(p->h_plan.data() + sizeof(header), ranked.data(), ranked.size());
-  memcpy(p->h_plan.data() + p->rank_groups_at, rank_groups.data(), rank_groups.size() * sizeof(RankGroup));
+  if (p->has_ranked)
+    memcpy(p->h_plan.data() + p->rank_groups_at, rank_groups.data(), rank_groups.size() * sizeof(RankGroup));
   hipError_t e = hipMemcpyAsync(p->d_plan, p->h_plan.data(), p->h_plan.size(), hipMemcpyHostToDevice, stream);
   if (e == hipSuccess && p->has_bindex)
     e = hipMemcpyAsync(p->d_groups, p->h_groups.data(), (size_t)p->ngroups * sizeof(BatchGroup),
@@ -1290,14 +1301,16 @@ hipError_t rts_batch_plan_launch(rts_batch_plan *p, BITS *out, int64_t out_strid
     return set_error(hipErrorInvalidValue, "rts_batch_plan_launch: output must be 16-byte aligned, stride a multiple of 4 words");
   if (p->nq == 0) return hipSuccess;
   int forms = forms_needed(p);
+  bool captured = false;
   if (p->max_rank_groups && stream) {
     // a launch captured by the caller runs both forms: either may have the queries set later
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     const hipError_t e = hipStreamIsCapturing(stream, &capture);
     if (e != hipSuccess) return set_error(e, "rts_batch_plan_launch");
-    if (capture != hipStreamCaptureStatusNone) forms = kFormBindex | kFormRanked;
+    captured = capture != hipStreamCaptureStatusNone;
+    if (captured) forms = kFormBindex | kFormRanked;
   }
-  return set_error(launch_batch(p, out, out_stride_words, counts, forms, stream), "rts_batch_plan_launch");
+  return set_error(launch_batch(p, out, out_stride_words, counts, forms, captured, stream), "rts_batch_plan_launch");
 }
 
 hipError_t rts_batch_plan_graph_launch(rts_batch_plan *p, BITS *out, int64_t out_stride_words,
@@ -1314,7 +1327,7 @@ hipError_t rts_batch_plan_graph_launch(rts_batch_plan *p, BITS *out, int64_t out
     p->graph = nullptr;
     e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return set_error(e, "rts_batch_plan_graph_launch: capture");
-    hipError_t le = launch_batch(p, out, out_stride_words, counts, forms_needed(p), stream);
+    hipError_t le = launch_batch(p, out, out_stride_words, counts, forms_needed(p), false, stream);
     e = hipStreamEndCapture(stream, &p->graph);
     if (le != hipSuccess) e = le;
     if (e == hipSuccess) e = hipGraphInstantiate(&p->exec, p->graph, nullptr, nullptr, 0);

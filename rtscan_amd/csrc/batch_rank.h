@@ -36,6 +36,8 @@ struct RankHeader {
   int steps;          // of kRankStepRows rows, that a workgroup takes of a group at a time
   int own_outs;       // the queries have their own bitmaps
   int bindex_groups;  // groups of k_batch
+  int nq;             // queries that are set
+  int pad[3];
 };
 
 // A query as the planner sees it: distinct columns (by address), no empty range unless `empty`.

@@ -570,7 +570,7 @@ static void free_dev(rts_bindex_dev *d) {
   int dev = 0;
   const bool here = hipGetDevice(&dev) == hipSuccess;
   const bool away = here && d->device != dev && hipSetDevice(d->device) == hipSuccess;
-  const bool idle = here && (away || d->device == dev) && hipDeviceSynchronize() == hipSuccess;
+  const bool idle = here && (away || d->device == dev) && device_wait();
   for (void *p : {(void *)d->sorted_val, (void *)d->sorted_pos, (void *)d->fvs, (void *)d->bent, (void *)d->boff,
                   (void *)d->bdir})
     pool_free(p, idle);

@@ -18,6 +18,11 @@ inline hipError_t pool_alloc(T **ptr, size_t bytes) {
   return pool_alloc(reinterpret_cast<void **>(ptr), bytes);
 }
 
+// Waits for all work of the current device, as a hipFree of the memory would; false where that
+// is refused (a capture in progress that forbids hipFree, no memory).  hipDeviceSynchronize will
+// not do: it ends the stream captures of all threads, in the relaxed mode too.
+bool device_wait();
+
 // hipMalloc, tried again with the pool's kept blocks given back when the device is out of
 // memory.
 hipError_t device_malloc(void **ptr, size_t bytes);

@@ -121,8 +121,13 @@ hipError_t rts_event_elapsed_ms(float *ms, hipEvent_t start, hipEvent_t stop);
 /* Device count, name and compute-unit count of the current device. */
 int rts_device_count(void);
 hipError_t rts_device_info(char *name, size_t name_len, int *cu_count, size_t *total_mem);
-/* Free and total device memory of the current device (hipMemGetInfo). */
+/* Free and total device memory of the current device: hipMemGetInfo's, with the memory that
+ * the library keeps of freed index arrays and of build and encode workspaces (at most 8 GB)
+ * counted as free.  The library's own allocations (rts_malloc among them) get that memory
+ * when the device has no other left; rts_device_mem_trim gives it back to the device, for
+ * other allocators of the process (it waits for the device's work, like hipFree). */
 hipError_t rts_device_mem_info(size_t *free_bytes, size_t *total_bytes);
+hipError_t rts_device_mem_trim(void);
 /* Message of the last error recorded by this library on the calling thread. */
 const char *rts_last_error(void);
 /* Scratch buffers (count partials, checker parts) the calling thread holds: one per

@@ -65,6 +65,7 @@ SIGNATURES = {
     "rts_thread_scratch_buffers": (_int, []),
     "rts_probe_read": (_err, [_vp, ctypes.c_size_t, _int, _int, _vp, _vp]),
     "rts_device_mem_info": (_err, [ctypes.POINTER(ctypes.c_size_t), ctypes.POINTER(ctypes.c_size_t)]),
+    "rts_device_mem_trim": (_err, []),
     # scans
     "rts_predicate_interval": (_int, [_int, _u32, _u32, ctypes.POINTER(_u32),
                                       ctypes.POINTER(_u32)]),
@@ -304,6 +305,11 @@ def device_free_bytes():
     f, t = ctypes.c_size_t(), ctypes.c_size_t()
     check(lib().rts_device_mem_info(ctypes.byref(f), ctypes.byref(t)), "mem_info")
     return f.value
+
+
+def device_mem_trim():
+    """Gives the device memory that the library keeps for later calls back to the device."""
+    check(lib().rts_device_mem_trim(), "mem_trim")
 
 
 def _sh(stream):

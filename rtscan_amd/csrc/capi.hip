@@ -3,6 +3,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <map>
 #include <mutex>
@@ -487,11 +488,19 @@ int rts_thread_scratch_buffers(void) { return (int)thread_scratch_entries(); }
 hipError_t rts_device_mem_info(size_t *free_bytes, size_t *total_bytes) {
   size_t f = 0, t = 0;
   int dev = 0;
-  if (hipGetDevice(&dev) == hipSuccess) pool_trim(dev);  // what the library keeps counts as free
-  hipError_t e = hipMemGetInfo(&f, &t);
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess) e = hipMemGetInfo(&f, &t);
   if (e != hipSuccess) return set_error(e, "rts_device_mem_info");
-  if (free_bytes) *free_bytes = f;
+  if (free_bytes) *free_bytes = std::min(t, f + pool_kept(dev));
   if (total_bytes) *total_bytes = t;
+  return hipSuccess;
+}
+
+hipError_t rts_device_mem_trim(void) {
+  int dev = 0;
+  const hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return set_error(e, "rts_device_mem_trim");
+  pool_trim(dev);
   return hipSuccess;
 }
 

@@ -10,7 +10,7 @@
 //     can be handed out at once;
 //   - at most kPoolBytes are kept on each device, the oldest going back first;
 //   - all of a device's kept blocks go back when an allocation of the library fails there
-//     (which is then tried again) and when a caller asks how much memory is free.
+//     (which is then tried again) and when a caller asks for it (rts_device_mem_trim).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -50,6 +50,12 @@ Pool &pool() {
   return *p;
 }
 
+size_t kept_bytes(const Pool &p, int dev) {
+  size_t total = 0;
+  for (const Block &k : p.kept) total += k.dev == dev ? k.bytes : 0;
+  return total;
+}
+
 // hipFree of blocks taken off the pool's lists, outside its lock (hipFree waits for the device).
 void give_back(const std::list<Block> &blocks) {
   for (const Block &b : blocks) (void)hipFree(b.ptr);
@@ -69,6 +75,12 @@ void pool_trim(int dev) {
     }
   }
   give_back(out);
+}
+
+size_t pool_kept(int dev) {
+  Pool &p = pool();
+  std::lock_guard<std::mutex> lock(p.mu);
+  return kept_bytes(p, dev);
 }
 
 bool device_wait() {
@@ -133,8 +145,7 @@ void pool_free(void *ptr, bool idle) {
       out.push_back(b);
     } else {
       p.kept.push_back(b);
-      size_t total = 0;
-      for (const Block &k : p.kept) total += k.dev == b.dev ? k.bytes : 0;
+      size_t total = kept_bytes(p, b.dev);
       for (auto k = p.kept.begin(); k != p.kept.end() && total > kPoolBytes;) {
         auto next = std::next(k);
         if (k->dev == b.dev) {

@@ -58,3 +58,13 @@ def test_an_index_freed(eng, mode, other_thread):
     d = eng.DeviceBuffer.from_numpy(rng.integers(0, 2 ** 32, N, dtype=np.uint64).astype(np.uint32))
     index = eng.BinDexIndex(d, N)
     captured_beside(eng, mode, other_thread, index.free)
+
+
+@pytest.mark.parametrize("mode", [GLOBAL, THREAD_LOCAL, RELAXED])
+@pytest.mark.parametrize("other_thread", [False, True])
+def test_free_memory_asked_for(eng, mode, other_thread):
+    """While the library keeps memory of a freed index."""
+    rng = np.random.default_rng(5)
+    d = eng.DeviceBuffer.from_numpy(rng.integers(0, 2 ** 32, N, dtype=np.uint64).astype(np.uint32))
+    eng.BinDexIndex(d, N).free()
+    captured_beside(eng, mode, other_thread, eng.device_free_bytes)

@@ -108,6 +108,10 @@ hipError_t rts_batch_plan_launch(rts_batch_plan *plan, BITS *out, int64_t out_st
  * stream must not be the null stream. */
 hipError_t rts_batch_plan_graph_launch(rts_batch_plan *plan, BITS *out, int64_t out_stride_words,
                                        unsigned long long *counts, hipStream_t stream);
+/* Queries of the current set that are evaluated together from the columns' values; the others
+ * are evaluated by their columns' forms (-1 for a NULL plan).  The statistics and the group
+ * count below describe all queries as if they were evaluated by their columns' forms. */
+int rts_batch_plan_together(const rts_batch_plan *plan);
 /* Planner statistics of the current queries: query-columns on the BinDex path, on the direct
  * path, BinDex columns whose range lies inside one bin (no filter vector read); row tiles. */
 void rts_batch_plan_stats(const rts_batch_plan *plan, int *bindex_cols, int *direct_cols,
@@ -125,7 +129,7 @@ int rts_batch_plan_list_cols(const rts_batch_plan *plan);
  * of the column's 128 areas), in sixteenths.  Batches drawn from one distribution get the
  * same digest; the autotuner's cache is keyed by it. */
 unsigned long long rts_batch_plan_mix_digest(const rts_batch_plan *plan);
-/* Work-item groups the current queries were planned into, and (cfg non-NULL) the launch
+/* Work-item groups the current queries are planned into by their columns' forms, and (cfg non-NULL) the launch
  * shape they were planned for; -1 for a NULL plan. */
 int rts_batch_plan_groups(const rts_batch_plan *plan, rts_batch_config *cfg);
 /* Rows, table columns and current query count of a plan. */

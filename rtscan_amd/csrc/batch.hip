@@ -719,7 +719,7 @@ struct rts_batch_plan {
   int64_t graph_stride = 0;
   int graph_forms = 0;
   int stats_bindex_cols = 0, stats_direct_cols = 0, stats_narrow_cols = 0, stats_auto_direct = 0;
-  int stats_list_cols = 0;
+  int stats_list_cols = 0, stats_together = 0;
   std::vector<rts_query_spec> specs;  // the current queries, re-planned on a new tiling
   std::vector<BITS *> outs;           // their per-query outputs, if given
   bool has_outs = false;
@@ -1267,6 +1267,7 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
   p->stats_narrow_cols = st_narrow;
   p->stats_list_cols = st_list;
   p->stats_auto_direct = st_auto;
+  p->stats_together = nq - (int)order.size();
   p->nq = nq;
   p->specs.assign(queries, queries + nq);
   p->h_groups.swap(groups);
@@ -1351,6 +1352,8 @@ void rts_batch_plan_stats(const rts_batch_plan *p, int *bindex_cols, int *direct
 }
 
 int rts_batch_plan_auto_direct(const rts_batch_plan *p) { return p ? p->stats_auto_direct : -1; }
+
+int rts_batch_plan_together(const rts_batch_plan *p) { return p ? p->stats_together : -1; }
 
 int rts_batch_plan_list_cols(const rts_batch_plan *p) { return p ? p->stats_list_cols : -1; }
 

@@ -884,19 +884,21 @@ static int pack_groups(const std::vector<int> &need, int slot_cap, int per_group
   return (int)free_slots.size();
 }
 
-// Time of k_batch in microseconds for nq queries whose columns take the forms pc: latency that
+// Time of k_batch in microseconds for `queries`, whose columns take the forms pc: latency that
 // grows with the items up to a chain of them, the bitmaps, and of each query-column its share
 // of reads, where filter vectors that other queries have read cost less.  Measured (mixed
 // queries unless noted): 1e8 rows, 4 columns, 256 bins: 8 queries 145, 32 370, 64 650, 256
 // 2110, 1024 7170; one column and bin each: 64 373, 256 1175; 2e7 rows, 2 columns: 8 73, 32
-// 107, 64 144; 4.2e6 rows, 4 columns: 8 40, 32 78, 256 140; 1e6 rows: 8 30, 64 44.
-static double batch_us(const rts_batch_plan *p, const std::vector<RankQuery> &queries, const std::vector<int> &ncols,
-                       const std::vector<PlannedCol> &pc) {
+// 107, 64 144; 4.2e6 rows, 4 columns: 8 40, 32 78, 256 140; 1e6 rows: 8 30, 64 44.  High for many
+// queries and for tables in the caches (1e6 rows, 4 columns, 1024 queries 200 for 135), where a
+// whole batch has time to spare either way; to compare one with its parts takes the closer form.
+static double batch_us(const rts_batch_plan *p, const std::vector<int> &queries, const std::vector<int> &ncols,
+                       const std::vector<int> &empty, const std::vector<PlannedCol> &pc, bool parts) {
   std::vector<int> wide((size_t)p->ncols, 0);  // query-columns that read filter vectors
   auto reads = [&](const PlannedCol &P) { return !P.direct && !P.narrow && P.list_b0 < 0; };
   auto each = [&](auto f) {
-    for (const RankQuery &q : queries)
-      for (int c = 0; !q.empty && c < ncols[q.id]; c++) f(pc[(size_t)q.id * kBatchMaxCols + c]);
+    for (const int q : queries)
+      for (int c = 0; !empty[q] && c < ncols[q]; c++) f(pc[(size_t)q * kBatchMaxCols + c]);
   };
   each([&](const PlannedCol &P) { wide[P.col] += reads(P); });
   const double n = (double)p->n, nq = (double)queries.size();
@@ -907,7 +909,9 @@ static double batch_us(const rts_batch_plan *p, const std::vector<RankQuery> &qu
                      : 1.1;
   });
   const double chain = std::max(std::min(40.0, n / 1e5), n / 1e6);
-  return 28 + chain * std::min(1.0, nq / 64 * std::max(1.0, n / 4e6)) + 0.08 * nq + us * n / 1e8;
+  const double few = std::min(nq, 256.0);
+  return 28 + chain * std::min(1.0, nq / 64 * std::max(1.0, n / 4e6)) +
+         (parts ? 0.1 * few + 0.04 * (nq - few) : 0.08 * nq) + us * n / 1e8 * (parts && n < 4e6 ? 0.65 : 1);
 }
 
 // The query as plan_rank_groups takes it, its columns read where its forms would read or have
@@ -1148,8 +1152,15 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
       R.own = outs ? outs[q] : nullptr;
       together.push_back(R);
     }
-    if (plan_rank_groups(together, p->n, p->max_rank_groups, batch_us(p, together, qcols, pc), rank_groups, &header))
-      for (const RankQuery &R : together) ranked[R.id] = 1;
+    std::vector<int> all(nq), rest;
+    for (int q = 0; q < nq; q++) all[q] = q;
+    for (const RankQuery &R : together) ranked[R.id] = 1;
+    for (int q = 0; q < nq; q++)
+      if (!ranked[q]) rest.push_back(q);
+    const double all_us = batch_us(p, all, qcols, qempty, pc, !rest.empty());
+    const double rest_us = rest.empty() ? 0 : batch_us(p, rest, qcols, qempty, pc, true);
+    if (!plan_rank_groups(together, p->n, p->max_rank_groups, all_us, rest_us, rank_groups, &header))
+      std::fill(ranked.begin(), ranked.end(), 0);
   }
   // 3. the order the others are grouped in: the caller's, or sorted by the (column, lower and
   //    upper filter vector) of their BinDex columns taken in column order, so that the

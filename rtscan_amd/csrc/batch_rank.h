@@ -52,9 +52,10 @@ struct RankQuery {
 // Groups a plan of max_queries queries has room for; 0: it never has any.
 int max_rank_groups(int max_queries);
 
-// All queries of `in` in groups, at most max_groups, if that is faster than the bindex_us
-// microseconds that their columns' forms take (else false, and none).
-bool plan_rank_groups(const std::vector<RankQuery> &in, int64_t n, int max_groups, double bindex_us,
+// All queries of `in` in groups, at most max_groups, if that is faster than the columns' forms
+// (else false, and none): by those the whole batch takes bindex_us microseconds, and its queries
+// that are not in `in` rest_us (0: none), which a second kernel then takes beside the groups.
+bool plan_rank_groups(const std::vector<RankQuery> &in, int64_t n, int max_groups, double bindex_us, double rest_us,
                       std::vector<RankGroup> &groups, RankHeader *header);
 
 // counts (zero between launches): the queries' rows are added.  nullptr: not counted.

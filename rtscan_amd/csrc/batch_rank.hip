@@ -331,8 +331,16 @@ __global__ __launch_bounds__(kRankThreads) __attribute__((amdgpu_waves_per_eu(kR
 
 // ------------------------------------------------------------------------------ planner
 
-// The models are off by a few per cent.
-static bool rank_cheaper(double rank_us, double bindex_us) { return rank_us < 0.9 * bindex_us; }
+// The models are off by a few per cent.  Where other queries of the batch keep to their columns'
+// forms (rest_us), their kernel is one more, and it costs more for each query the fewer there are.
+// Of 99 such batches (2e4 to 6.7e7 rows, 2 and 4 columns, 16 to 1024 queries, 1, 4 and 7 of 8 kept
+// apart) those taken here save 3 to 23 per cent; with the whole of bindex_us charged to the
+// queries in question, 1e5 rows x 4 with 8 of 16 took 49 us for 29, 4.2e6 x 4 with 128 of 256 186 for
+// 139, 2e7 x 4 with 32 of 64 249 for 192.
+constexpr double kBesideUs = 8;
+static bool rank_cheaper(double rank_us, double rest_us, double bindex_us) {
+  return rest_us > 0 ? rank_us + rest_us + kBesideUs < bindex_us : rank_us < 0.9 * bindex_us;
+}
 
 namespace {
 
@@ -509,14 +517,14 @@ double plan_us(const Plan &p, const std::vector<Predicates> &q, int64_t n) {
 
 int max_rank_groups(int max_queries) { return std::min(max_queries / kRankMinQueries, kRankMaxGroups); }
 
-bool plan_rank_groups(const std::vector<RankQuery> &in, int64_t n, int max_groups, double bindex_us,
+bool plan_rank_groups(const std::vector<RankQuery> &in, int64_t n, int max_groups, double bindex_us, double rest_us,
                       std::vector<RankGroup> &groups, RankHeader *header) {
   groups.clear();
   header->ngroups = 0;
   header->steps = 1;
   if (in.size() < (size_t)kRankMinQueries || in.size() > (size_t)max_groups * kRankQueries) return false;
   // at least the bitmaps are written
-  if (2.9 * in.size() * n / 1e8 >= bindex_us) return false;
+  if (2.9 * in.size() * n / 1e8 + rest_us >= bindex_us) return false;
   std::vector<Column> columns;
   std::vector<std::vector<std::pair<uint32_t, int *>>> bounds;  // (bound less one, where its number goes)
   std::vector<Predicates> q(in.size());
@@ -561,7 +569,7 @@ bool plan_rank_groups(const std::vector<RankQuery> &in, int64_t n, int max_group
       us = dealt_us;
     }
   }
-  if ((int)plan.size() > max_groups || !rank_cheaper(us, bindex_us)) return false;
+  if ((int)plan.size() > max_groups || !rank_cheaper(us, rest_us, bindex_us)) return false;
   groups.resize(plan.size());
   for (size_t g = 0; g < plan.size(); g++) fill_group(groups[g], plan[g], in, q, columns);
   header->ngroups = (int)groups.size();

@@ -27,7 +27,9 @@
  * and replays it; queries set with rts_batch_plan_set_queries live in device memory at a fixed
  * address, so a replay, of a graph of the caller's own too, evaluates the current set: every
  * bitmap, and the counts of as many of its queries as there were at the capture (with fewer
- * queries now, the other counts are left as they are).
+ * queries now, the other counts mean nothing).  A graph of the caller's own that is captured while
+ * none of the queries are evaluated together evaluates every later set by its columns' forms;
+ * one captured while some are evaluates each set as a launch does.
  */
 #ifndef RTS_BATCH_H_
 #define RTS_BATCH_H_

@@ -338,6 +338,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   // the group count is read from device memory, so a captured launch stays valid when the
   // queries are planned again
   const int ngroups = *ngroups_ptr;
+  if (ngroups == 0) return;  // all queries are evaluated together: the counters keep their zeros
   const int xcd = blockIdx.x % kXcds, nblk_x = gridDim.x / kXcds, j = blockIdx.x / kXcds;
   const int64_t tiles_x = ntiles > xcd ? (ntiles - 1 - xcd) / kXcds + 1 : 0;
   const int64_t items_x = tiles_x * ngroups;
@@ -589,27 +590,27 @@ __global__ __launch_bounds__(kBlock) void k_batch_counts(const uint32_t *partial
 
 // The same where queries may be evaluated together (`ranked`, per query): those have their sum
 // in rank_counts, which is left at zero for the next launch.  The queries that are set now need
-// not be those of a captured launch: it runs a workgroup for every query that the plan has room
-// for, so that all sums are cleared, and writes the counts of its first `out_nq` queries, as far
-// as they are set.
+// not be those of a captured launch: it clears the sums of those past its own, and leaves the
+// counts of its own that are no longer set as they are.
 __global__ __launch_bounds__(kBlock) void k_batch_counts_mixed(const uint32_t *partials, int64_t ntiles,
                                                                const RankHeader *header,
-                                                               unsigned long long *rank_counts, unsigned out_nq,
+                                                               unsigned long long *rank_counts,
                                                                unsigned long long *counts) {
   __shared__ unsigned long long part[kBlock / kWave];
   const uint8_t *ranked = reinterpret_cast<const uint8_t *>(header + 1);
-  if (blockIdx.x >= (unsigned)header->nq) return;  // no launch adds to its sum
+  const unsigned nq = (unsigned)header->nq;
+  for (unsigned q = gridDim.x + blockIdx.x * kBlock + threadIdx.x; q < nq; q += gridDim.x * kBlock) rank_counts[q] = 0;
+  if (blockIdx.x >= nq) return;
   unsigned long long s = 0;
   if (ranked[blockIdx.x]) {
     if (threadIdx.x == 0) {
       s = rank_counts[blockIdx.x];
       rank_counts[blockIdx.x] = 0;
     }
-  } else if (blockIdx.x < out_nq) {
+  } else {
     const uint32_t *p = partials + (int64_t)blockIdx.x * ntiles;
     for (int64_t i = threadIdx.x; i < ntiles; i += kBlock) s += p[i];
   }
-  if (blockIdx.x >= out_nq) return;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, kWave);
   if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x / kWave] = s;
@@ -704,6 +705,7 @@ struct rts_batch_plan {
   size_t rank_counts_at = 0, rank_groups_at = 0;
   int max_rank_groups = 0;
   bool has_ranked = false, has_bindex = false;  // the forms that the current queries need
+  bool captured_apart = false;  // the caller captured a launch that has k_batch alone
   uint32_t *d_zero_dir = nullptr;  // ntiles + 1 zeros: the directory of an unused list
   int ngroups = 0;  // of k_batch
   uint32_t *d_partials = nullptr;
@@ -806,51 +808,51 @@ static int batch_resident_per_cu() {
 }
 
 template <int TW, int NT>
-static void launch_k_batch(rts_batch_plan *p, BITS *out, int64_t out_stride, hipStream_t s) {
+static void launch_k_batch(rts_batch_plan *p, const int *ngroups, BITS *out, int64_t out_stride, hipStream_t s) {
   const int cus = std::max(1, device_cu_count());
   // a persistent grid larger than what is resident would leave its statically assigned
   // work items to a second round: clamp to the occupancy limit
   unsigned grid = (unsigned)(cus * std::min(p->cfg.blocks_per_cu, batch_resident_per_cu<TW, NT>()));
   grid = std::max<unsigned>(kXcds, grid / kXcds * kXcds);
-  hipLaunchKernelGGL((k_batch<TW, NT>), dim3(grid), dim3(NT), 0, s, p->d_groups,
-                     &reinterpret_cast<const RankHeader *>(p->d_plan)->bindex_groups, p->n,
+  hipLaunchKernelGGL((k_batch<TW, NT>), dim3(grid), dim3(NT), 0, s, p->d_groups, ngroups, p->n,
                      p->words, p->ntiles, out, out_stride, p->d_partials, p->d_sched);
 }
 
-// The forms of evaluation a launch runs.
-enum : int { kFormBindex = 1, kFormRanked = 2 };
+// The forms of evaluation a launch runs: k_batch for the queries that are not evaluated together,
+// k_batch_ranked for those that are, k_batch for all.
+enum : int { kFormBindex = 1, kFormRanked = 2, kFormApart = 4 };
 
 static int forms_needed(const rts_batch_plan *p) {
   return (p->has_bindex ? kFormBindex : 0) | (p->has_ranked ? kFormRanked : 0);
 }
 
-// captured: by the caller, who may set other queries, and more or fewer, before a replay.
 static hipError_t launch_batch(rts_batch_plan *p, BITS *out, int64_t out_stride, unsigned long long *counts, int forms,
-                               bool captured, hipStream_t s) {
+                               hipStream_t s) {
   const auto *const header = reinterpret_cast<const RankHeader *>(p->d_plan);
   auto *const rank_counts = reinterpret_cast<unsigned long long *>(p->d_plan + p->rank_counts_at);
   hipError_t e = hipSuccess;
   if (forms & kFormRanked)
     e = launch_rank_groups(reinterpret_cast<const RankGroup *>(p->d_plan + p->rank_groups_at), header, p->n, out,
                            out_stride, counts ? rank_counts : nullptr, s);
-  if (e == hipSuccess && (forms & kFormBindex)) {
+  if (e == hipSuccess && (forms & (kFormBindex | kFormApart))) {
+    const int *const ng = forms & kFormApart ? &header->apart_groups : &header->bindex_groups;
     const bool small = p->cfg.threads == 256;
     switch (p->cfg.tile_words) {
       case 2048:
-        small ? launch_k_batch<2048, 256>(p, out, out_stride, s) : launch_k_batch<2048, 512>(p, out, out_stride, s);
+        small ? launch_k_batch<2048, 256>(p, ng, out, out_stride, s) : launch_k_batch<2048, 512>(p, ng, out, out_stride, s);
         break;
       case 1024:
-        small ? launch_k_batch<1024, 256>(p, out, out_stride, s) : launch_k_batch<1024, 512>(p, out, out_stride, s);
+        small ? launch_k_batch<1024, 256>(p, ng, out, out_stride, s) : launch_k_batch<1024, 512>(p, ng, out, out_stride, s);
         break;
       default:
-        small ? launch_k_batch<512, 256>(p, out, out_stride, s) : launch_k_batch<512, 512>(p, out, out_stride, s);
+        small ? launch_k_batch<512, 256>(p, ng, out, out_stride, s) : launch_k_batch<512, 512>(p, ng, out, out_stride, s);
     }
     e = hipGetLastError();
   }
   if (!counts) return e;
   if (forms & kFormRanked)  // also after an error, so that no sum is left for the next launch
-    hipLaunchKernelGGL(k_batch_counts_mixed, dim3((unsigned)(captured ? p->max_queries : p->nq)), dim3(kBlock), 0, s,
-                       p->d_partials, p->ntiles, header, rank_counts, (unsigned)p->nq, counts);
+    hipLaunchKernelGGL(k_batch_counts_mixed, dim3((unsigned)p->nq), dim3(kBlock), 0, s, p->d_partials, p->ntiles,
+                       header, rank_counts, counts);
   else if (e == hipSuccess)
     hipLaunchKernelGGL(k_batch_counts, dim3((unsigned)p->nq), dim3(kBlock), 0, s, p->d_partials, p->ntiles,
                        counts);
@@ -1159,15 +1161,18 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
       if (!ranked[q]) rest.push_back(q);
     const double all_us = batch_us(p, all, qcols, qempty, pc, !rest.empty());
     const double rest_us = rest.empty() ? 0 : batch_us(p, rest, qcols, qempty, pc, true);
-    if (!plan_rank_groups(together, p->n, p->max_rank_groups, all_us, rest_us, rank_groups, &header))
+    // k_batch has one set of groups: for the rest, or for all where a captured launch needs them
+    if ((p->captured_apart && !rest.empty()) ||
+        !plan_rank_groups(together, p->n, p->max_rank_groups, all_us, rest_us, rank_groups, &header))
       std::fill(ranked.begin(), ranked.end(), 0);
   }
+  const int nranked = (int)std::count(ranked.begin(), ranked.end(), 1);
   // 3. the order the others are grouped in: the caller's, or sorted by the (column, lower and
   //    upper filter vector) of their BinDex columns taken in column order, so that the
   //    groups a tile's workgroups run together read few distinct filter vectors
   std::vector<int> order;
   for (int q = 0; q < nq; q++)
-    if (!ranked[q]) order.push_back(q);
+    if (!ranked[q] || p->captured_apart) order.push_back(q);
   if (p->cfg.order == 1) {
     std::vector<std::vector<int>> key(nq);
     for (const int q : order) {
@@ -1278,15 +1283,16 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
   p->stats_narrow_cols = st_narrow;
   p->stats_list_cols = st_list;
   p->stats_auto_direct = st_auto;
-  p->stats_together = nq - (int)order.size();
+  p->stats_together = nranked;
   p->nq = nq;
   p->specs.assign(queries, queries + nq);
   p->h_groups.swap(groups);
   p->ngroups = (int)p->h_groups.size();
-  p->has_bindex = p->ngroups > 0;
+  p->has_bindex = nranked < nq;
   p->has_ranked = !rank_groups.empty();
   if (nq == 0) return hipSuccess;
-  header.bindex_groups = p->ngroups;
+  header.bindex_groups = p->has_bindex ? p->ngroups : 0;
+  header.apart_groups = p->ngroups;
   header.nq = nq;
   p->h_plan.assign(p->has_ranked ? p->rank_groups_at + rank_groups.size() * sizeof(RankGroup)
                                  : sizeof(header) + ranked.size(), 0);
@@ -1295,7 +1301,7 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
   if (p->has_ranked)
     memcpy(p->h_plan.data() + p->rank_groups_at, rank_groups.data(), rank_groups.size() * sizeof(RankGroup));
   hipError_t e = hipMemcpyAsync(p->d_plan, p->h_plan.data(), p->h_plan.size(), hipMemcpyHostToDevice, stream);
-  if (e == hipSuccess && p->has_bindex)
+  if (e == hipSuccess && p->ngroups)
     e = hipMemcpyAsync(p->d_groups, p->h_groups.data(), (size_t)p->ngroups * sizeof(BatchGroup),
                        hipMemcpyHostToDevice, stream);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);  // the host vectors change on the next call
@@ -1313,16 +1319,20 @@ hipError_t rts_batch_plan_launch(rts_batch_plan *p, BITS *out, int64_t out_strid
     return set_error(hipErrorInvalidValue, "rts_batch_plan_launch: output must be 16-byte aligned, stride a multiple of 4 words");
   if (p->nq == 0) return hipSuccess;
   int forms = forms_needed(p);
-  bool captured = false;
   if (p->max_rank_groups && stream) {
-    // a launch captured by the caller runs both forms: either may have the queries set later
+    // A launch captured by the caller runs both forms, as either may have the queries set later;
+    // but if none of the present ones are evaluated together, k_batch alone, for all queries of
+    // the sets to come too.  (A kernel that finds no groups adds 4.5 us: 8 queries on 1e5 rows x 2
+    // 34 to 39 us, 64 on 4.2e6 x 4 93 to 98.)
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     const hipError_t e = hipStreamIsCapturing(stream, &capture);
     if (e != hipSuccess) return set_error(e, "rts_batch_plan_launch");
-    captured = capture != hipStreamCaptureStatusNone;
-    if (captured) forms = kFormBindex | kFormRanked;
+    if (capture != hipStreamCaptureStatusNone) {
+      forms = p->has_ranked ? kFormBindex | kFormRanked : kFormApart;
+      p->captured_apart = p->captured_apart || forms == kFormApart;
+    }
   }
-  return set_error(launch_batch(p, out, out_stride_words, counts, forms, captured, stream), "rts_batch_plan_launch");
+  return set_error(launch_batch(p, out, out_stride_words, counts, forms, stream), "rts_batch_plan_launch");
 }
 
 hipError_t rts_batch_plan_graph_launch(rts_batch_plan *p, BITS *out, int64_t out_stride_words,
@@ -1339,7 +1349,7 @@ hipError_t rts_batch_plan_graph_launch(rts_batch_plan *p, BITS *out, int64_t out
     p->graph = nullptr;
     e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return set_error(e, "rts_batch_plan_graph_launch: capture");
-    hipError_t le = launch_batch(p, out, out_stride_words, counts, forms_needed(p), false, stream);
+    hipError_t le = launch_batch(p, out, out_stride_words, counts, forms_needed(p), stream);
     e = hipStreamEndCapture(stream, &p->graph);
     if (le != hipSuccess) e = le;
     if (e == hipSuccess) e = hipGraphInstantiate(&p->exec, p->graph, nullptr, nullptr, 0);

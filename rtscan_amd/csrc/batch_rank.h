@@ -35,9 +35,10 @@ struct RankHeader {
   int ngroups;
   int steps;          // of kRankStepRows rows, that a workgroup takes of a group at a time
   int own_outs;       // the queries have their own bitmaps
-  int bindex_groups;  // groups of k_batch
+  int bindex_groups;  // groups of k_batch for the queries that are not evaluated together
+  int apart_groups;   // and for all, where a captured launch may need them
   int nq;             // queries that are set
-  int pad[3];
+  int pad[2];
 };
 
 // A query as the planner sees it: distinct columns (by address), no empty range unless `empty`.

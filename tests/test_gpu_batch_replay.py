@@ -13,9 +13,11 @@ pytestmark = pytest.mark.gpu
 POISON = 0x5A5A5A5A5A5A5A5A
 
 
+# captured with queries that are evaluated together, and with queries that keep to their indexes
+@pytest.mark.parametrize("first", [AUTO, BINDEX])
 @pytest.mark.parametrize("modes", [(AUTO,), (AUTO, BINDEX)])
 @pytest.mark.parametrize("captured", [16, 100])
-def test_replays_with_more_and_fewer_queries(eng, captured, modes):
+def test_replays_with_more_and_fewer_queries(eng, captured, modes, first):
     n, most = 100003, 300
     cols = make_columns(n, 3, 8)
     plan = make_plan(eng, cols, most)
@@ -28,7 +30,8 @@ def test_replays_with_more_and_fewer_queries(eng, captured, modes):
     hip = ctypes.CDLL("libamdhip64.so.7")
     graph, instance = ctypes.c_void_p(), ctypes.c_void_p()
     s = ctypes.c_void_p(stream.handle)
-    plan.set_queries(sets[captured], stream)
+    plan.set_queries(make_queries(cols, captured, captured, (first,), most=2), stream)
+    assert plan.stats()["together"] == (captured if first == AUTO else 0)
     plan.launch(out, stride, counts, stream)
     stream.synchronize()
     assert hip.hipStreamBeginCapture(s, 1) == 0
@@ -38,6 +41,8 @@ def test_replays_with_more_and_fewer_queries(eng, captured, modes):
     for nq in (captured, 300, 64, 9, 300, 100, 16, 300):
         queries = sets[nq]
         plan.set_queries(queries, stream)
+        # a graph that has the indexes' kernel alone takes nothing from the launches beside it
+        assert plan.stats()["together"] == sum(all(m == AUTO for *_, m in q) for q in queries) or nq > 64 and BINDEX in modes
         for launch in ("replay", "replay", "launch", "graph_launch", "replay", "launch"):
             out.fill(0x5A)
             counts.fill(0x5A)
@@ -50,7 +55,8 @@ def test_replays_with_more_and_fewer_queries(eng, captured, modes):
             got = out.to_numpy(np.uint32, stride * most).reshape(most, stride)
             cnt = counts.to_numpy(np.uint64, most)
             written = min(nq, captured) if launch == "replay" else nq
-            assert (cnt[written:] == POISON).all(), (nq, launch)
+            first_unwritten = captured if launch == "replay" and first == BINDEX else written
+            assert (cnt[first_unwritten:] == POISON).all(), (nq, launch)
             assert (got[nq:] == POISON & 0xFFFFFFFF).all(), (nq, launch)
             verify(cols, queries[:written], got[:written, :words], cnt[:written])
             verify(cols, queries, got[:nq, :words], None)

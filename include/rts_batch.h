@@ -138,12 +138,13 @@ int rts_batch_plan_groups(const rts_batch_plan *plan, rts_batch_config *cfg);
 void rts_batch_plan_info(const rts_batch_plan *plan, long long *n, int *ncols, int *nq);
 void rts_batch_plan_free(rts_batch_plan *plan);
 
-/* Autotuner: time every candidate launch shape on the plan's current queries (median of
- * `reps` launches each) and keep the fastest in the plan.  Candidates span tile size, group
+/* Autotuner: time every candidate launch shape on the plan's current queries, all evaluated by
+ * their columns' forms (median of `reps` launches each), and keep the fastest in the plan.  Candidates span tile size, group
  * size, workgroups per CU, order, workgroup size, bin count (the plan's index sets) and the
  * planner's direct weight.  With cache_path non-NULL the result is read from / appended to
  * that file, keyed by device, n, column count, query count and the query-mix digest, so
- * later runs skip the search.  best_ms (may be NULL) receives the winner's time. */
+ * later runs skip the search.  best_ms (may be NULL) receives the winner's time, by the
+ * columns' forms too. */
 hipError_t rts_batch_autotune(rts_batch_plan *plan, BITS *out, int64_t out_stride_words,
                               const rts_batch_config *candidates, int ncandidates, int reps,
                               const char *cache_path, rts_batch_config *chosen, float *best_ms,

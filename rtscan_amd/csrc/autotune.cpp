@@ -1,6 +1,7 @@
 // autotune.cpp -- the batched launch's autotuner: times candidate launch shapes (tile and
 // group sizes, workgroups, order, bin count, the planner's direct weight) on the plan's
-// current queries and keeps the fastest; results cached in a text file keyed by the
+// current queries, all evaluated by their columns' forms (the launch shape means nothing to
+// queries that are evaluated together), and keeps the fastest; results cached in a text file keyed by the
 // device, the table, the query count and the query-mix digest.
 #include <hip/hip_runtime_api.h>
 #include <stdio.h>
@@ -12,7 +13,7 @@
 #include <string>
 #include <vector>
 
-#include "rts_batch.h"
+#include "batch_forms.h"
 
 namespace {
 
@@ -95,6 +96,7 @@ extern "C" hipError_t rts_batch_autotune(rts_batch_plan *plan, BITS *out, int64_
     return e;
   }
   bool have = false;
+  rts::batch_plan_all_apart(plan, true);
   for (int i = 0; i < ncandidates && e == hipSuccess; i++) {
     e = rts_batch_plan_set_config(plan, &candidates[i], stream);
     if (e != hipSuccess) break;
@@ -120,7 +122,12 @@ extern "C" hipError_t rts_batch_autotune(rts_batch_plan *plan, BITS *out, int64_
   }
   (void)hipEventDestroy(a);
   (void)hipEventDestroy(b);
-  if (e != hipSuccess) return e;
+  rts::batch_plan_all_apart(plan, false);
+  if (e != hipSuccess) {  // the shape that the plan has now, its queries evaluated as it sees fit again
+    rts_batch_plan_groups(plan, &best);
+    (void)rts_batch_plan_set_config(plan, &best, stream);
+    return e;
+  }
   e = rts_batch_plan_set_config(plan, &best, stream);
   if (e != hipSuccess) return e;
   if (cache_path) cache_store(cache_path, key, best, best_t);

@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "batch.h"
+#include "batch_forms.h"
 #include "batch_rank.h"
 #include "bindex_dev.h"
 #include "device_ptr.h"
@@ -705,6 +706,8 @@ struct rts_batch_plan {
   size_t rank_counts_at = 0, rank_groups_at = 0;
   int max_rank_groups = 0;
   bool has_ranked = false, has_bindex = false;  // the forms that the current queries need
+  bool all_apart = false;       // batch_plan_all_apart
+  bool planned_apart = false;   // of the current queries
   bool captured_apart = false;  // the caller captured a launch that has k_batch alone
   uint32_t *d_zero_dir = nullptr;  // ntiles + 1 zeros: the directory of an unused list
   int ngroups = 0;  // of k_batch
@@ -860,6 +863,8 @@ static hipError_t launch_batch(rts_batch_plan *p, BITS *out, int64_t out_stride,
   return e != hipSuccess ? e : ce;
 }
 
+void batch_plan_all_apart(rts_batch_plan *p, bool apart) { p->all_apart = apart; }
+
 // Query-columns a work item has toggle arrays for.
 static int batch_slots(const rts_batch_config &c) { return kBatchLdsWords / 512 * c.threads / c.tile_words; }
 
@@ -1010,10 +1015,11 @@ hipError_t rts_batch_plan_set_config(rts_batch_plan *p, const rts_batch_config *
   // a new tiling or index set needs new list directories
   const bool retile = cfg->tile_words != p->cfg.tile_words || set != p->active_set;
   // the grouping depends on the order, the slots a workgroup's LDS holds, the group size
-  // and which query-columns the cost model sends to the direct form
+  // and which query-columns the cost model sends to the direct form; the autotuner changes
+  // whether queries are evaluated together
   const bool reorder = cfg->order != p->cfg.order || cfg->threads != p->cfg.threads ||
                        cfg->queries_per_group != p->cfg.queries_per_group ||
-                       cfg->direct_weight != p->cfg.direct_weight;
+                       cfg->direct_weight != p->cfg.direct_weight || p->planned_apart != p->all_apart;
   p->cfg = *cfg;
   p->active_set = set;
   p->index = p->index_sets[set].data();
@@ -1144,7 +1150,7 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
   header.own_outs = outs != nullptr;
   std::vector<RankGroup> rank_groups;
   std::vector<uint8_t> ranked((size_t)nq, 0);
-  if (p->max_rank_groups) {
+  if (p->max_rank_groups && !p->all_apart) {
     std::vector<RankQuery> together;
     together.reserve((size_t)nq);
     for (int q = 0; q < nq; q++) {
@@ -1284,6 +1290,7 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
   p->stats_list_cols = st_list;
   p->stats_auto_direct = st_auto;
   p->stats_together = nranked;
+  p->planned_apart = p->all_apart;
   p->nq = nq;
   p->specs.assign(queries, queries + nq);
   p->h_groups.swap(groups);

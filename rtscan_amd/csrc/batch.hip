@@ -1150,7 +1150,7 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
   header.own_outs = outs != nullptr;
   std::vector<RankGroup> rank_groups;
   std::vector<uint8_t> ranked((size_t)nq, 0);
-  if (p->max_rank_groups && !p->all_apart) {
+  if (p->max_rank_groups && !p->all_apart && nq >= kRankMinQueries) {
     std::vector<RankQuery> together;
     together.reserve((size_t)nq);
     for (int q = 0; q < nq; q++) {
@@ -1160,17 +1160,18 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
       R.own = outs ? outs[q] : nullptr;
       together.push_back(R);
     }
-    std::vector<int> all(nq), rest;
-    for (int q = 0; q < nq; q++) all[q] = q;
-    for (const RankQuery &R : together) ranked[R.id] = 1;
-    for (int q = 0; q < nq; q++)
-      if (!ranked[q]) rest.push_back(q);
-    const double all_us = batch_us(p, all, qcols, qempty, pc, !rest.empty());
-    const double rest_us = rest.empty() ? 0 : batch_us(p, rest, qcols, qempty, pc, true);
     // k_batch has one set of groups: for the rest, or for all where a captured launch needs them
-    if ((p->captured_apart && !rest.empty()) ||
-        !plan_rank_groups(together, p->n, p->max_rank_groups, all_us, rest_us, rank_groups, &header))
-      std::fill(ranked.begin(), ranked.end(), 0);
+    if (together.size() >= (size_t)kRankMinQueries && (!p->captured_apart || together.size() == (size_t)nq)) {
+      std::vector<int> all(nq), rest;
+      for (int q = 0; q < nq; q++) all[q] = q;
+      for (const RankQuery &R : together) ranked[R.id] = 1;
+      for (int q = 0; q < nq; q++)
+        if (!ranked[q]) rest.push_back(q);
+      const double all_us = batch_us(p, all, qcols, qempty, pc, !rest.empty());
+      const double rest_us = rest.empty() ? 0 : batch_us(p, rest, qcols, qempty, pc, true);
+      if (!plan_rank_groups(together, p->n, p->max_rank_groups, all_us, rest_us, rank_groups, &header))
+        std::fill(ranked.begin(), ranked.end(), 0);
+    }
   }
   const int nranked = (int)std::count(ranked.begin(), ranked.end(), 1);
   // 3. the order the others are grouped in: the caller's, or sorted by the (column, lower and
@@ -1307,10 +1308,13 @@ hipError_t rts_batch_plan_set_queries_out(rts_batch_plan *p, const rts_query_spe
   memcpy(p->h_plan.data() + sizeof(header), ranked.data(), ranked.size());
   if (p->has_ranked)
     memcpy(p->h_plan.data() + p->rank_groups_at, rank_groups.data(), rank_groups.size() * sizeof(RankGroup));
-  hipError_t e = hipMemcpyAsync(p->d_plan, p->h_plan.data(), p->h_plan.size(), hipMemcpyHostToDevice, stream);
-  if (e == hipSuccess && p->ngroups)
+  // the longer copy first: behind another it takes 2 us more (16 queries apart 25.7 us in all, 23.3)
+  hipError_t e = hipSuccess;
+  if (p->ngroups)
     e = hipMemcpyAsync(p->d_groups, p->h_groups.data(), (size_t)p->ngroups * sizeof(BatchGroup),
                        hipMemcpyHostToDevice, stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(p->d_plan, p->h_plan.data(), p->h_plan.size(), hipMemcpyHostToDevice, stream);
   if (e == hipSuccess) e = hipStreamSynchronize(stream);  // the host vectors change on the next call
   return set_error(e, "rts_batch_plan_set_queries");
 }

@@ -513,6 +513,18 @@ double plan_us(const Plan &p, const std::vector<Predicates> &q, int64_t n) {
   return (rounds > 1 ? 25 : 15) + worst * round * (2 * steps * p.size() <= grid ? 0.7 : rounds);
 }
 
+// plan_us is no less than this, which takes no planning: the bitmaps are written and, in more
+// than a round, the columns read.
+double least_us(const std::vector<RankQuery> &in, int64_t n) {
+  if (n <= (int64_t)rank_grid() * kRankStepRows) return 0.7 * 2.9 * in.size() * n / 1e8;
+  const CODE *seen[kRankCols];
+  int ncols = 0;
+  for (const RankQuery &q : in)
+    for (int c = 0; c < q.ncols && ncols < kRankCols; c++)
+      if (std::find(seen, seen + ncols, q.col[c]) == seen + ncols) seen[ncols++] = q.col[c];
+  return 25 + (2.9 * in.size() + 82.0 * ncols) * n / 1e8;
+}
+
 }  // namespace
 
 int max_rank_groups(int max_queries) { return std::min(max_queries / kRankMinQueries, kRankMaxGroups); }
@@ -523,8 +535,7 @@ bool plan_rank_groups(const std::vector<RankQuery> &in, int64_t n, int max_group
   header->ngroups = 0;
   header->steps = 1;
   if (in.size() < (size_t)kRankMinQueries || in.size() > (size_t)max_groups * kRankQueries) return false;
-  // at least the bitmaps are written
-  if (2.9 * in.size() * n / 1e8 + rest_us >= bindex_us) return false;
+  if (!rank_cheaper(least_us(in, n), rest_us, bindex_us)) return false;
   std::vector<Column> columns;
   std::vector<std::vector<std::pair<uint32_t, int *>>> bounds;  // (bound less one, where its number goes)
   std::vector<Predicates> q(in.size());

@@ -807,14 +807,16 @@ static void launch_ranked(const uint32_t *col, uint64_t n, const RankedPreds &t,
 // Predicates up to which a pass tests each one (k_scan_multi) instead of searching
 // (k_scan_ranked).  The search costs a row the same for any number of predicates up to 32 and
 // half as much again up to 64, a test three instructions a row and predicate; on a short
-// column the search's chain of dependent steps (one tile a wave) is what shows.  Measured,
-// counted, tests against search: 2^18 rows, 64 predicates 7.2 / 8.6 us; 2^19 rows, 33: 7.7 /
-// 8.9, 40: 9.2 / 9.0, 64: 9.4 / 8.8; 2^20 rows, 16: 7.1 / 8.2, 24: 9.3 / 8.8, 64: 13.7 / 9.6;
-// 4.2e6 rows, 8: 10.9 / 11.3, 10: 11.4 / 12.2, 12: 12.8 / 12.3, 16: 15.8 / 12.5; 1e8 rows, 5:
-// 95 / 99, 8: 110 / 100, 16: 194 / 117, 32: 374 / 166, 64: 730 / 268 (250 when every bitmap
-// starts on a 128-byte line: what is left is the writes' rate).
+// column the search's chain of dependent steps (one tile a wave) is what shows.  Measured, tests
+// against search, counted / not: 2^18 rows, 64 predicates 7.5 : 9.1 / 6.5 : 7.4; 2^19 rows, 36:
+// 7.8 : 9.3 / 6.2 : 7.4, 48: 9.6 : 9.3 / 7.7 : 7.6; 2^20 rows, 20: 8.5 : 8.9 / 6.8 : 6.9, 24: 9.6 :
+// 9.0 / 7.7 : 7.0, 64: 14.1 : 10.1 / 12.1 : 8.0; 1.5e6 rows, 16: 9.7 : 9.2 / 7.7 : 6.8; 4.2e6 rows, 8:
+// 9.8 : 10.0 / 8.3 : 7.8, 10: 10.5 : 10.7 / 9.0 : 8.4, 12: 11.6 : 10.7 / 10.1 : 8.4; 6e6 rows, 8: 12.0 : 12.2 /
+// 10.1 : 9.6, 10: 14.4 : 13.2 / 12.6 : 10.7; counted, 1e8 rows, 5: 95 : 99, 8: 110 : 100, 16: 194 : 117, 32:
+// 374 : 166, 64: 730 : 268 (250 when every bitmap starts on a 128-byte line: what is left is the
+// writes' rate).
 static int direct_preds(uint64_t n) {
-  return n < 3u << 17 ? kMultiPreds : n < 1u << 20 ? 40 : n < 1u << 22 ? 16 : 8;
+  return n < 3u << 17 ? kMultiPreds : n < 1u << 20 ? 40 : n < 5u << 18 ? 20 : n < 1u << 22 ? 16 : n < 5u << 20 ? 9 : 8;
 }
 
 hipError_t scan_ranges(const CODE *col, uint64_t n, const CODE *lo, const CODE *hi, int np, BITS *out,

@@ -74,6 +74,7 @@ struct ScratchEntry {
   int kind, dev;
   uintptr_t stream;
   void *dptr, *hptr;
+  bool fresh;
 };
 
 const std::thread::id g_main_thread = std::this_thread::get_id();
@@ -98,21 +99,20 @@ thread_local ThreadScratch t_scratch;
 }  // namespace
 
 hipError_t thread_scratch(int kind, hipStream_t stream, size_t dev_bytes, size_t host_bytes, void **dptr,
-                          void **hptr, bool *created) {
+                          void **hptr, bool **fresh) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
-  if (created) *created = false;
   std::vector<ScratchEntry> &tab = t_scratch.entries;
-  for (const ScratchEntry &x : tab) {
+  for (ScratchEntry &x : tab) {
     if (x.kind == kind && x.dev == dev && x.stream == (uintptr_t)stream) {
       *dptr = x.dptr;
       if (hptr) *hptr = x.hptr;
+      if (fresh) *fresh = &x.fresh;
       return hipSuccess;
     }
   }
-  if (created) *created = true;
-  ScratchEntry x{kind, dev, (uintptr_t)stream, nullptr, nullptr};
+  ScratchEntry x{kind, dev, (uintptr_t)stream, nullptr, nullptr, true};
   if (dev_bytes) e = device_malloc(&x.dptr, dev_bytes);
   if (e == hipSuccess && host_bytes) e = hipHostMalloc(&x.hptr, host_bytes, 0);
   if (e != hipSuccess) {
@@ -126,6 +126,7 @@ hipError_t thread_scratch(int kind, hipStream_t stream, size_t dev_bytes, size_t
   tab.push_back(x);
   *dptr = x.dptr;
   if (hptr) *hptr = x.hptr;
+  if (fresh) *fresh = &tab.back().fresh;
   return hipSuccess;
 }
 
@@ -133,11 +134,12 @@ size_t thread_scratch_entries() { return t_scratch.entries.size(); }
 
 CountSink stream_count_sink(unsigned long long *out, hipStream_t stream) {
   void *p = nullptr;
-  bool created = false;
-  if (thread_scratch(kScratchCountAcc, stream, kCountAccBytes, 0, &p, nullptr, &created) != hipSuccess)
+  bool *fresh = nullptr;
+  if (thread_scratch(kScratchCountAcc, stream, kCountAccBytes, 0, &p, nullptr, &fresh) != hipSuccess)
     return CountSink{out, nullptr, nullptr};
   // the counting kernels leave the accumulators at zero; a new set starts there too
-  if (created && hipMemsetAsync(p, 0, kCountAccBytes, stream) != hipSuccess) return CountSink{out, nullptr, nullptr};
+  if (*fresh && hipMemsetAsync(p, 0, kCountAccBytes, stream) != hipSuccess) return CountSink{out, nullptr, nullptr};
+  *fresh = false;
   return CountSink{out, nullptr, static_cast<unsigned long long *>(p)};
 }
 

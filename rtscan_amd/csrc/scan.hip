@@ -832,14 +832,23 @@ hipError_t scan_ranges(const CODE *col, uint64_t n, const CODE *lo, const CODE *
   MultiSink sink{};
   if (counts) {
     void *acc = nullptr;
-    bool created = false;
-    hipError_t e = thread_scratch(kScratchMulti, s, kMultiAccBytes, 0, &acc, nullptr, &created);
-    if (e == hipSuccess && created) {  // the kernels leave the accumulators at zero; new ones start there too
-      hipLaunchKernelGGL(k_zero_multi, dim3(1), dim3(kBlock), 0, s, static_cast<unsigned long long *>(acc));
-      e = hipGetLastError();
-    }
+    bool *fresh = nullptr;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    hipError_t e = thread_scratch(kScratchMulti, s, 2 * kMultiAccBytes, 0, &acc, nullptr, &fresh);
+    if (e == hipSuccess && s) e = hipStreamIsCapturing(s, &capture);
     if (e != hipSuccess) return e;
     sink.acc = static_cast<unsigned long long *>(acc);
+    const bool captured = capture != hipStreamCaptureStatusNone;
+    if (captured) sink.acc += kMultiAccBytes / sizeof(*sink.acc);
+    // The kernels leave the accumulators at zero; new ones start there too.  A captured launch may be
+    // replayed on any stream, beside the ones that its own has queued by then: it has accumulators
+    // apart from theirs, and clears them, which two replays at once may leave in any state.
+    if (*fresh || captured) {
+      hipLaunchKernelGGL(k_zero_multi, dim3(1), dim3(kBlock), 0, s, sink.acc);
+      e = hipGetLastError();
+      if (e != hipSuccess) return e;
+      if (!captured) *fresh = false;
+    }
   }
   for (int p0 = 0; p0 < np; p0 += kMultiPreds) {  // one pass over the column per 64 predicates
     const int k = std::min(kMultiPreds, np - p0);

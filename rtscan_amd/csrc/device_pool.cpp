@@ -10,14 +10,18 @@
 //     can be handed out at once;
 //   - at most kPoolBytes are kept on each device, the oldest going back first;
 //   - all of a device's kept blocks go back when an allocation of the library fails there
-//     (which is then tried again) and when a caller asks for it (rts_device_mem_trim).
+//     (which is then tried again) and when a caller asks for it (rts_device_mem_trim);
+//   - a kept block that the device does not take back (hipFree is refused beside some stream
+//     captures) stays kept.
+// A block's list node is made before the block and moves from list to list with it, so nothing
+// here throws into the C entry points that call it.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <iterator>
 #include <list>
 #include <mutex>
-#include <unordered_map>
+#include <new>
 
 #include "device_mem.h"
 
@@ -40,8 +44,8 @@ struct Block {
 
 struct Pool {
   std::mutex mu;
-  std::list<Block> kept;                         // oldest first
-  std::unordered_map<void *, Block> in_use;
+  std::list<Block> kept;  // oldest first
+  std::list<Block> in_use;
 };
 
 // Never destroyed: blocks may be freed while the process ends, in any order.
@@ -56,9 +60,18 @@ size_t kept_bytes(const Pool &p, int dev) {
   return total;
 }
 
-// hipFree of blocks taken off the pool's lists, outside its lock (hipFree waits for the device).
-void give_back(const std::list<Block> &blocks) {
-  for (const Block &b : blocks) (void)hipFree(b.ptr);
+// hipFree of kept blocks taken off the list, outside the lock (hipFree waits for the device).
+void give_back(std::list<Block> &blocks) {
+  for (auto b = blocks.begin(); b != blocks.end();) {
+    auto next = std::next(b);
+    if (hipFree(b->ptr) == hipSuccess) blocks.erase(b);
+    b = next;
+  }
+  if (blocks.empty()) return;
+  (void)hipGetLastError();
+  Pool &p = pool();
+  std::lock_guard<std::mutex> lock(p.mu);
+  p.kept.splice(p.kept.begin(), blocks);
 }
 
 }  // namespace
@@ -116,18 +129,22 @@ hipError_t pool_alloc(void **ptr, size_t bytes) {
           (best == p.kept.end() || it->bytes < best->bytes))
         best = it;
     if (best != p.kept.end()) {
-      p.in_use.emplace(best->ptr, *best);
       *ptr = best->ptr;
-      p.kept.erase(best);
+      p.in_use.splice(p.in_use.end(), p.kept, best);
       return hipSuccess;
     }
   }
-  void *q = nullptr;
-  e = device_malloc(&q, bytes);
+  std::list<Block> block;
+  try {
+    block.push_back(Block{nullptr, bytes, dev});
+  } catch (const std::bad_alloc &) {
+    return hipErrorOutOfMemory;
+  }
+  e = device_malloc(&block.front().ptr, bytes);
   if (e != hipSuccess) return e;
+  *ptr = block.front().ptr;
   std::lock_guard<std::mutex> lock(p.mu);
-  p.in_use.emplace(q, Block{q, bytes, dev});
-  *ptr = q;
+  p.in_use.splice(p.in_use.end(), block);
   return hipSuccess;
 }
 
@@ -137,18 +154,17 @@ void pool_free(void *ptr, bool idle) {
   {
     Pool &p = pool();
     std::lock_guard<std::mutex> lock(p.mu);
-    auto it = p.in_use.find(ptr);
+    auto it = std::find_if(p.in_use.begin(), p.in_use.end(), [&](const Block &b) { return b.ptr == ptr; });
     if (it == p.in_use.end()) return;
-    const Block b = it->second;
-    p.in_use.erase(it);
-    if (!idle) {  // the device may still use it: hipFree waits
-      out.push_back(b);
+    if (!idle) {
+      out.splice(out.end(), p.in_use, it);
     } else {
-      p.kept.push_back(b);
-      size_t total = kept_bytes(p, b.dev);
+      const int dev = it->dev;
+      p.kept.splice(p.kept.end(), p.in_use, it);
+      size_t total = kept_bytes(p, dev);
       for (auto k = p.kept.begin(); k != p.kept.end() && total > kPoolBytes;) {
         auto next = std::next(k);
-        if (k->dev == b.dev) {
+        if (k->dev == dev) {
           total -= k->bytes;
           out.splice(out.end(), p.kept, k);
         }
@@ -156,7 +172,10 @@ void pool_free(void *ptr, bool idle) {
       }
     }
   }
-  give_back(out);
+  if (idle)
+    give_back(out);
+  else
+    (void)hipFree(out.front().ptr);  // the device may still use it: hipFree waits
 }
 
 }  // namespace rts

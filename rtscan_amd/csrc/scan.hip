@@ -10,7 +10,6 @@
 
 #include <algorithm>
 #include <type_traits>
-#include <vector>
 
 #include "common.h"
 #include "transpose.h"
@@ -741,38 +740,39 @@ hipError_t scan_conjunction(const CODE *const *cols, const CODE *lo, const CODE 
 // (range r = the values with r bounds at or below them), as k_scan_ranked searches them.
 static RankedPreds rank_table(const CODE *lo, const CODE *hi, int np) {
   RankedPreds t;
-  std::vector<uint32_t> b;
+  uint32_t b[2 * kMultiPreds];  // no host memory: a caller in C cannot take an exception
+  size_t nb = 0;
   for (int p = 0; p < np; p++) {
     if (lo[p] > hi[p]) continue;
-    b.push_back(lo[p]);
-    if (hi[p] != 0xFFFFFFFFu) b.push_back(hi[p] + 1);
+    b[nb++] = lo[p];
+    if (hi[p] != 0xFFFFFFFFu) b[nb++] = hi[p] + 1;
   }
-  std::sort(b.begin(), b.end());
-  b.erase(std::unique(b.begin(), b.end()), b.end());
+  std::sort(b, b + nb);
+  nb = std::unique(b, b + nb) - b;
   memset(t.mask, 0, sizeof(t.mask));
   memset(t.r0, 0, sizeof(t.r0));
   memset(t.r1, 0, sizeof(t.r1));
   for (int p = 0; p < np; p++) {
     if (lo[p] > hi[p]) continue;
-    const size_t r0 = std::lower_bound(b.begin(), b.end(), lo[p]) - b.begin() + 1;
+    const size_t r0 = std::lower_bound(b, b + nb, lo[p]) - b + 1;
     // a value of 2^32 - 1 also passes the padding bounds: the last range's mask fills up
-    const size_t r1 = hi[p] == 0xFFFFFFFFu ? kRankEntries - 1 : std::lower_bound(b.begin(), b.end(), hi[p] + 1) - b.begin() + 1;
+    const size_t r1 = hi[p] == 0xFFFFFFFFu ? kRankEntries - 1 : std::lower_bound(b, b + nb, hi[p] + 1) - b + 1;
     t.r0[p] = (uint8_t)r0;
     t.r1[p] = (uint8_t)r1;
     for (size_t r = r0; r < r1; r++) t.mask[p / 32][r] |= 1u << (p % 32);
   }
-  t.last = (uint32_t)b.size();
+  t.last = (uint32_t)nb;
   t.stride = (t.last + 1) | 1;  // odd: the copies start in different LDS banks
   t.copies = 64;
   while (t.copies * t.stride > kHistEntries) t.copies /= 2;
-  t.first = b.empty() ? 0xFFFFFFFFu : b[0];
+  t.first = nb == 0 ? 0xFFFFFFFFu : b[0];
   t.levels = 1;
-  while ((1u << t.levels) < b.size()) t.levels++;  // 2^levels - 1 nodes for the bounds but the first
+  while ((1u << t.levels) < nb) t.levels++;  // 2^levels - 1 nodes for the bounds but the first
   for (uint32_t &v : t.tree) v = 0xFFFFFFFFu;
   for (int l = 0; l < t.levels; l++)  // node i of level l: the bound in the middle of its span
     for (uint32_t i = 0; i < 1u << l; i++) {
       const size_t at = ((2 * (size_t)i + 1) << (t.levels - 1 - l));  // 1 .. 2^levels - 1
-      if (at < b.size()) t.tree[(1u << l) + i] = b[at];
+      if (at < nb) t.tree[(1u << l) + i] = b[at];
     }
   return t;
 }

@@ -43,7 +43,7 @@ __host__ __device__ __forceinline__ uint32_t rank_stride(uint32_t ngroups, uint3
 }
 
 // 2 i + (v > t), in two instructions.
-__device__ __forceinline__ uint32_t descend(uint32_t i, uint32_t v, uint32_t t) {
+static __device__ __forceinline__ uint32_t descend_above(uint32_t i, uint32_t v, uint32_t t) {
   asm("v_cmp_gt_u32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(i) : "v"(v), "v"(t) : "vcc");
   return i;
 }
@@ -210,11 +210,11 @@ __global__ __launch_bounds__(kRankThreads) __attribute__((amdgpu_waves_per_eu(kR
 #pragma unroll
           for (int j = 0; j < 32; j++) {
             const bool up = v[j] > root;
-            i[j] = descend(up ? 3 : 2, v[j], up ? node3 : node2);
+            i[j] = descend_above(up ? 3 : 2, v[j], up ? node3 : node2);
           }
           for (int l = 2; l < levels; l++) {
 #pragma unroll
-            for (int j = 0; j < 32; j++) i[j] = descend(i[j], v[j], tree[i[j]]);
+            for (int j = 0; j < 32; j++) i[j] = descend_above(i[j], v[j], tree[i[j]]);
           }
           // range = leaf less 2^levels: no byte of four borrows, and at 8 levels the low byte is it
           const uint32_t leaf0 = levels < 8 ? 0x01010101u << levels : 0u;

@@ -112,7 +112,7 @@ __global__ void k_rank_samples(const CODE *sorted, int64_t m, CODE *out) {
 }
 
 // 2 i + (v >= t), in two instructions.
-__device__ __forceinline__ uint32_t descend(uint32_t i, uint32_t v, uint32_t t) {
+static __device__ __forceinline__ uint32_t descend_from(uint32_t i, uint32_t v, uint32_t t) {
   asm("v_cmp_ge_u32 vcc, %1, %2\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc" : "+v"(i) : "v"(v), "v"(t) : "vcc");
   return i;
 }
@@ -191,11 +191,11 @@ __global__ __launch_bounds__(kBlock) void k_build_fvs(const CODE *col, int64_t n
 #pragma unroll
     for (int j = 0; j < 32; j++) {
       const bool up = x[j] >= root;
-      t[j] = descend(up ? 3 : 2, x[j], up ? node3 : node2);
+      t[j] = descend_from(up ? 3 : 2, x[j], up ? node3 : node2);
     }
     for (int l = 2; l < M; l++) {
 #pragma unroll
-      for (int j = 0; j < 32; j++) t[j] = descend(t[j], x[j], tree[t[j]]);
+      for (int j = 0; j < 32; j++) t[j] = descend_from(t[j], x[j], tree[t[j]]);
     }
 #pragma unroll
     for (int j = 0; j < 32; j += 4) {

@@ -10,7 +10,7 @@
 // k_batch reads two filter-vector words (8 bytes) and two list slices for every word of every
 // query-column, 16 KB a query-column and tile through the L2: that is its bound (1024 queries
 // on 4 columns of 1e8 rows: 7.2 ms, 11-13 TB/s from L2).  Here a row costs, per 256 queries,
-// a search of every column (24 VALU instructions, 8 LDS reads at 254 bounds) and per 32
+// a search of every column (24 VALU instructions, 6 LDS reads at 254 bounds) and per 32
 // queries 17 VALU instructions for four columns (8 lookups and ANDs, 8 the transpose), and
 // memory moves the columns and the bitmaps alone.  Launches, k_batch against this, us: 1e8
 // rows x 4, 1024 queries 7180 / 5250; 2^26 x 2, 64 queries 374 / 226 (its memory traffic

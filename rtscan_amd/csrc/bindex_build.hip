@@ -37,8 +37,9 @@ struct BuildHead {
 // bin a * sub + j starts at the value in slot idx[a] + j * len / sub, so bin a * sub is
 // the area's own start.  Ranks of the bin starts: searched between the neighbouring bins'
 // slots, unless a run reaches over one.  Bound by latency, chains of a dozen or two loads in
-// one workgroup.  Three kernels with the host between them, and the blocks' slots from the
-// host, made a build of 1e6 rows and 256 bins take 423 us; it is 308 (1e5: 353, 245).
+// one workgroup (15 us at 1e6 rows, 26 at 1e8).  Three kernels with the host between them, and the
+// blocks' slots from the host, in its place: a build of 1e6 rows and 256 bins 423 us against 308
+// (1e5: 353, 245); with what has changed elsewhere since, 240.
 constexpr int kStartThreads = 1024;
 __global__ __launch_bounds__(kStartThreads) void k_build_starts(const CODE *sorted, int64_t n, int sub, BuildHead *head) {
   __shared__ int64_t idx[kAreas + 1];

@@ -405,8 +405,9 @@ __device__ __forceinline__ void store_ranked(uint32_t (&rank4)[8], const uint32_
 // are filled by several stores (256 bytes a store: 2.7 TB/s where the bitmaps do not start on
 // lines, 1 KB: 3.9, 4 KB: 4.7).  64 / 32 predicates, workgroups of 256 (1 KB) and of 512: 1e8 rows
 // 280 / 173 and 268 / 166 us, 1e8 + 1 297 and 275, 2e8 511 and 500; 40 of 99,999,900 203 and 207.
-// Bitmaps at 16-byte offsets take non-temporal 16-byte stores (64 of 1e8 rows: 303 -> 286 us);
-// 4-byte ones are slower non-temporal (322 -> 336).  w0: of wave 0.
+// Bitmaps at 16-byte offsets take non-temporal 16-byte stores (64 / 32 of 1e8 rows, counted, 4-byte
+// stores 273 / 172 us, these 267 / 167; of 2e8 523 / 338, 492 / 313); 4-byte ones are slower
+// non-temporal (in workgroups of 256, 64 of 1e8 rows 322 -> 336).  w0: of wave 0.
 template <int HALVES, bool FULL>
 __device__ __forceinline__ void store_ranked_staged(uint32_t (&rank4)[8], const uint32_t (&mask)[HALVES][kRankEntries],
                                                     uint32_t (&words)[2][kStaged][kStagedBlock], int half0, int np, BITS *out,
